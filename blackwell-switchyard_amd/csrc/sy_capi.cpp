@@ -83,7 +83,7 @@ int bwd_grid(const sy_plan& p, int64_t n_tok, int dtype, bool stats, int variant
 // other caller.
 int bwd_plan(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, int aligned,
              bool stats, int variant, sy_plan* p) {
-  int rc = make_plan(SY_OP_BWD, n_src, 0, d, v_dtype, w_dtype, aligned, p, stats);
+  int rc = make_launch_plan(SY_OP_BWD, n_src, d, v_dtype, w_dtype, aligned, p, stats);
   if (rc != SY_OK) return rc;
   apply_tile_rules(SY_OP_BWD, n_src, n_tok, d, p);
   if (p->family != SY_FAMILY_GENERIC && p->rows_per_tile > 16 && (!stats || variant != 0))
@@ -192,10 +192,13 @@ int batched_workspace_rows(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d,
 }
 
 
-hipError_t fwd_vec(const sy_plan& p, const FwdArgs& a, hipStream_t s) {
-  if (a.v_dtype == SY_BF16) return launch_fwd_vec_bf16(p, a, s, nullptr);
-  if (a.v_dtype == SY_F16) return launch_fwd_vec_f16(p, a, s, nullptr);
-  return launch_fwd_vec_f32(p, a, s, nullptr);
+hipError_t fwd_vec(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info = nullptr) {
+  const bool wide = a.w_dtype != a.v_dtype;
+  if (a.v_dtype == SY_BF16)
+    return wide ? launch_fwd_wide_bf16(p, a, s, info) : launch_fwd_vec_bf16(p, a, s, info);
+  if (a.v_dtype == SY_F16)
+    return wide ? launch_fwd_wide_f16(p, a, s, info) : launch_fwd_vec_f16(p, a, s, info);
+  return launch_fwd_vec_f32(p, a, s, info);
 }
 hipError_t sol_vec(const sy_plan& p, const FwdArgs& a, hipStream_t s) {
   if (a.v_dtype == SY_BF16) return launch_sol_vec_bf16(p, a, s);
@@ -321,7 +324,7 @@ int fwd_impl(const RowTable& v, bool v_ok, const void* w, void* out, float* stat
              int w_dtype, float eps, hipStream_t s) {
   const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out);
   sy_plan p;
-  const int rc = make_plan(SY_OP_FWD, n_src, 0, d, v_dtype, w_dtype, aligned, &p);
+  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p);
   if (rc != SY_OK) return rc;
   apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
   if (n_tok == 0) return SY_OK;
@@ -431,7 +434,9 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
                        int w_dtype, int aligned, sy_plan* out) {
   if (out == nullptr) return SY_ERR_NULL;
   if (n_tok < 0) return SY_ERR_SHAPE;
-  const int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  if (rc == SY_OK && (op == SY_OP_FWD || op == SY_OP_BWD))
+    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out);
   if (rc != SY_OK) return rc;
   if (op == SY_OP_FWD || op == SY_OP_BWD) apply_tile_rules(op, n_src, n_tok, d, out);
   return SY_OK;
@@ -657,7 +662,7 @@ int sy_kernel_info(int op, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
   if (rc != SY_OK) return rc;
   if (op != SY_OP_FWD && op != SY_OP_BWD) return SY_ERR_OP;
   sy_plan p;
-  rc = make_plan(op, n_src, 0, d, v_dtype, w_dtype, 1, &p);
+  rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, 1, &p);
   if (rc != SY_OK) return rc;
   apply_tile_rules(op, n_src, n_tok, d, &p);
   out[0] = out[1] = out[2] = out[3] = 0;
@@ -667,9 +672,7 @@ int sy_kernel_info(int op, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
   if (op == SY_OP_FWD) {
     const FwdArgs a{RowTable{}, nullptr, nullptr, nullptr, nullptr, nullptr, 1, (int)n_src,
                     n_tok,      (int)d,  v_dtype, w_dtype, 0.0f};
-    e = v_dtype == SY_BF16 ? launch_fwd_vec_bf16(p, a, nullptr, &r)
-        : v_dtype == SY_F16 ? launch_fwd_vec_f16(p, a, nullptr, &r)
-                            : launch_fwd_vec_f32(p, a, nullptr, &r);
+    e = fwd_vec(p, a, nullptr, &r);
   } else {
     e = bwd_resources(p, v_dtype, true, 0, &r);
     if (e == hipSuccess) {

@@ -199,6 +199,87 @@ template <> __device__ __forceinline__ float dot<F32>(const i32x4_t& a, const i3
   return acc;
 }
 
+// The CE elements of chunk c of a query row of dtype wt (0 fp32, 1 fp16, 2 bf16,
+// uniform over the launch) as fp32. r covers the row, so elements past its end
+// read 0. A query may have another dtype than the sources (fp32 parameters with
+// 16-bit activations); the widening is exact.
+template <int CE>
+__device__ __forceinline__ void ld_query(__amdgpu_buffer_rsrc_t r, uint32_t c, int wt, float* f) {
+  if (wt == F32::code) {
+#pragma unroll
+    for (int q = 0; q < CE / 4; ++q) {
+      const i32x4_t x = ld16(r, (c * CE + 4 * q) * 4u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * q + e] = __int_as_float(x[e]);
+    }
+    return;
+  }
+  int x[CE / 2];
+  if constexpr (CE == 8) {
+    const i32x4_t t = ld16(r, c * 16u);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = t[k];
+  } else {
+    const auto t = __builtin_amdgcn_raw_buffer_load_b64(r, c * 8u, 0, 0);
+    x[0] = (int)t[0];
+    x[1] = (int)t[1];
+  }
+  const bool bf = wt == BF16::code;
+#pragma unroll
+  for (int k = 0; k < CE / 2; ++k) {
+    const f16x2_t h = __builtin_bit_cast(f16x2_t, x[k]);
+    f[2 * k] = bf ? bf_lo((uint32_t)x[k]) : (float)h.x;
+    f[2 * k + 1] = bf ? bf_hi((uint32_t)x[k]) : (float)h.y;
+  }
+}
+
+// acc + sum_e x[e] * f[e] with an fp32 query chunk.
+template <class T>
+__device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, float acc) {
+#pragma unroll
+  for (int e = 0; e < T::ce; ++e) acc = fmaf(elem<T>(x, e), f[e], acc);
+  return acc;
+}
+
+// A lane's query chunks: packed in the sources' dtype, or (WIDE) as fp32 values
+// when the query has another dtype. fp32 sources hold any query as fp32 chunks.
+template <class T, bool WIDE, int VPL>
+struct Query {
+  i32x4_t q[VPL];
+  __device__ __forceinline__ void load(const void* w, int wt, uint32_t d, uint32_t lane_off,
+                                       uint32_t step) {
+    if constexpr (T::code == F32::code) {
+      const auto r = make_rsrc(w, d * (wt == F32::code ? 4u : 2u));
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) {
+        float f[4];
+        ld_query<4>(r, (lane_off + j * step) / 16u, wt, f);
+        q[j] = pack<T>(f);
+      }
+    } else {
+      const auto r = make_rsrc(w, d * 2u);
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) q[j] = ld16(r, lane_off + j * step);
+    }
+  }
+  __device__ __forceinline__ float dot(const i32x4_t& x, int j, float acc) const {
+    return sy::dot<T>(x, q[j], acc);
+  }
+};
+template <class T, int VPL>
+struct Query<T, true, VPL> {
+  float f[VPL][T::ce];
+  __device__ __forceinline__ void load(const void* w, int wt, uint32_t d, uint32_t lane_off,
+                                       uint32_t step) {
+    const auto r = make_rsrc(w, d * (wt == F32::code ? 4u : 2u));
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) ld_query<T::ce>(r, (lane_off + j * step) / 16u, wt, f[j]);
+  }
+  __device__ __forceinline__ float dot(const i32x4_t& x, int j, float acc) const {
+    return dot_wide<T>(x, f[j], acc);
+  }
+};
+
 // Scalar element load/store for the generic (unaligned) path.
 __device__ __forceinline__ float load_elem(const void* p, int64_t i, int dtype) {
   if (dtype == 2) return __uint_as_float((uint32_t)((const uint16_t*)p)[i] << 16);

@@ -1,12 +1,15 @@
 // Instantiates the register-tiled kernels for one dtype and maps a plan onto
-// them. Built three times: -DSY_TAG=BF16 -DSY_NAME=bf16, F16/f16, F32/f32.
+// them. Built per dtype (-DSY_TAG=BF16 -DSY_NAME=bf16, F16/f16, F32/f32) and per
+// part, so that the parts compile side by side: -DSY_PART=0 the forward and the
+// speed-of-light kernels, 1 the backward, 2 the batched kernels, 3 (16-bit
+// dtypes) the forward with a query of another dtype.
 #include <algorithm>
 
 #include "sy_kernels.hpp"
 #include "sy_launch.hpp"
 
-#if !defined(SY_TAG) || !defined(SY_NAME)
-#error "build with -DSY_TAG=<BF16|F16|F32> -DSY_NAME=<bf16|f16|f32>"
+#if !defined(SY_TAG) || !defined(SY_NAME) || !defined(SY_PART)
+#error "build with -DSY_TAG=<BF16|F16|F32> -DSY_NAME=<bf16|f16|f32> -DSY_PART=<0..3>"
 #endif
 
 #define SY_CAT2(a, b) a##b
@@ -51,6 +54,7 @@ KernelRes resources_of(K* kernel, int block_threads) {
 }
 }  // namespace
 
+#if SY_PART == 0
 hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_t s,
                                  KernelRes* info) {
   const float inv_d = 1.0f / (float)a.d;
@@ -73,14 +77,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
           static const KernelRes km = resources_of(k_fwd_res<T, W_, V_, N_, true, true>, kB); \
           if (n_iter <= 2 && km.blocks_per_cu >= kr.blocks_per_cu) {                         \
             hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true, true>), dim3(grid), dim3(kB), \
-                               0, s, a.v, (const St*)a.w, (St*)a.out, a.stats, a.m_out,      \
+                               0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,      \
                                a.l_out, a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d,    \
                                n_iter, a.prior_m, a.prior_l);                                \
             return hipGetLastError();                                                        \
           }                                                                                  \
         }                                                                                    \
         hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true>), dim3(grid), dim3(kB), 0, s, a.v, \
-                           (const St*)a.w, (St*)a.out, a.stats, a.m_out, a.l_out,            \
+                           a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,            \
                            a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,         \
                            a.prior_m, a.prior_l);                                            \
         return hipGetLastError();                                                            \
@@ -90,14 +94,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
         static const KernelRes kf = resources_of(k_fwd_res<T, W_, V_, N_, false, true>, kB); \
         if (n_iter <= 2 && kf.blocks_per_cu >= kr.blocks_per_cu) {                           \
           hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, true>), dim3(grid), dim3(kB), 0, \
-                             s, a.v, (const St*)a.w, (St*)a.out, a.stats, a.m_out, a.l_out,  \
+                             s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,  \
                              a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,       \
                              nullptr, nullptr);                                              \
           return hipGetLastError();                                                          \
         }                                                                                    \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_>), dim3(grid), dim3(kB), 0, s, a.v,        \
-                         (const St*)a.w, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
+                         a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
                          a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter, nullptr, nullptr);     \
     } else {                                                                                 \
       if (a.prior_m != nullptr) return hipErrorInvalidConfiguration;                         \
@@ -108,7 +112,7 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
         return hipSuccess;                                                                   \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd<T, W_, V_, N_>), dim3((unsigned)grid), dim3(kB), 0, s, a.v,  \
-                         (const St*)a.w, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
+                         a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
                          a.n_src, a.n_tok, a.d, a.eps, inv_d);                               \
     }                                                                                        \
     return hipGetLastError();                                                                \
@@ -138,6 +142,9 @@ hipError_t SY_FN(launch_sol_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
   return hipErrorInvalidConfiguration;
 }
 
+#endif
+
+#if SY_PART == 2
 hipError_t SY_FN(launch_batched_vec_)(const sy_plan& p, const BatchedArgs& a, hipStream_t s) {
   const float inv_d = 1.0f / (float)a.d;
 #define X(W_, V_, N_)                                                                            \
@@ -153,6 +160,9 @@ hipError_t SY_FN(launch_batched_vec_)(const sy_plan& p, const BatchedArgs& a, hi
   return hipErrorInvalidConfiguration;
 }
 
+#endif
+
+#if SY_PART == 1
 // The backward's grid must be known before launch (it sizes the workspace),
 // so it is computed here from the instantiation's resources.
 // variant: a BwdVariant (kBwdStacked, kBwdListed, kBwdStatsGrad).
@@ -196,7 +206,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
   if (tile_is(p, W_, V_, N_)) {                                                              \
     if (a.stats == nullptr || a.listed || a.gm != nullptr) return hipErrorInvalidConfiguration; \
     hipLaunchKernelGGL((k_bwd_tall<T, W_, V_, N_>), dim3(grid), dim3(TallGeom<W_, V_, N_>::kBlock), 0, \
-                       s, a.v, (const St*)a.w, (const St*)a.g, a.stats, a.dv, a.partial,       \
+                       s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.dv, a.partial,       \
                        a.n_src, a.n_tok, a.d, inv_d, n_iter);                                 \
     return hipGetLastError();                                                                 \
   }
@@ -204,7 +214,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
 #undef X
 #define SY_BWD_LAUNCH(W_, V_, N_, ST_, LI_)                                                  \
   hipLaunchKernelGGL((k_bwd<T, W_, V_, N_, ST_, LI_>), dim3(grid), dim3(BwdGeom<W_, V_>::kBlock), 0, \
-                     s, a.v, (const St*)a.w, (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, \
+                     s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, \
                      a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter)
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
@@ -227,6 +237,9 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
   return hipErrorInvalidConfiguration;
 }
 
+#endif
+
+#if SY_PART == 2
 // Batched backward tiles: one chunk per lane, W waves per token, NR rows,
 // up to kBwdBatchedMaxQ queries.
 #define SY_BB_TILES(X) X(1, 4) X(1, 9) X(2, 4) X(2, 9) X(4, 4) X(4, 9) X(8, 4) X(8, 9)
@@ -264,5 +277,50 @@ hipError_t SY_FN(launch_bwd_batched_vec_)(const sy_plan& p, const BwdBatchedArgs
 #undef SY_BB_LAUNCH
   return hipErrorInvalidConfiguration;
 }
+#endif
+
+#if SY_PART == 3
+// The forward over 16-bit sources with a query of another dtype (fp32 parameters,
+// or the other 16-bit type): the same tiles with the query widened to fp32.
+hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream_t s,
+                                  KernelRes* info) {
+  const float inv_d = 1.0f / (float)a.d;
+  const bool res = p.family == SY_FAMILY_RESIDENT;
+  if (a.prior_m != nullptr) return hipErrorInvalidConfiguration;
+#define X(W_, V_, N_)                                                                        \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
+    if (res) {                                                                               \
+      static const KernelRes kr =                                                            \
+          resources_of(k_fwd_res<T, W_, V_, N_, false, false, true>, kB);                    \
+      const int grid = launch_grid(kr, a.n_tok, kT);                                         \
+      if (info) {                                                                            \
+        *info = kr;                                                                          \
+        info->grid = grid;                                                                   \
+        return hipSuccess;                                                                   \
+      }                                                                                      \
+      const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * kT);                             \
+      hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, true>), dim3(grid),         \
+                         dim3(kB), 0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,  \
+                         a.l_out, a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,  \
+                         nullptr, nullptr);                                                  \
+    } else {                                                                                 \
+      const int64_t grid = cdiv(a.n_tok, kT);                                                \
+      if (info) {                                                                            \
+        *info = resources_of(k_fwd<T, W_, V_, N_, true>, kB);                                \
+        info->grid = (int)grid;                                                              \
+        return hipSuccess;                                                                   \
+      }                                                                                      \
+      hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true>), dim3((unsigned)grid), dim3(kB), \
+                         0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,   \
+                         a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d);                  \
+    }                                                                                        \
+    return hipGetLastError();                                                                \
+  }
+  SY_TILES(X)
+#undef X
+  return hipErrorInvalidConfiguration;
+}
+#endif
 
 }  // namespace sy

@@ -33,6 +33,14 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
+// With a wide query (WIDE) the dots widen every element of the tile, and the
+// weighted sum widens it again: the opaque copy keeps the first widening from being
+// held for the second one, which would double the tile's registers (the chunked
+// (1,4,4) tile 310 VGPRs without it).
+template <bool WIDE>
+__device__ __forceinline__ void reconvert(i32x4_t& x) {
+  if constexpr (WIDE) asm volatile("" : "+v"(x));
+}
 
 // Forward-shaped kernels: 256-thread workgroups (or one token per workgroup
 // when a token needs more than four waves).
@@ -123,9 +131,12 @@ __device__ __forceinline__ void row_sums_transposed(const float (&tv)[P], float 
 // m_out[t] = max logit and l_out[t] = sum_n exp(logit_n - m) (both or neither).
 // normalize = 0 stores the unnormalised o = sum_n exp(logit_n - m) v_n instead
 // of o / l (reference src/switchyard/reference.py:194-215, attn_with_stats).
-template <class T, int W, int VPL, int NR>
+//
+// WIDE: 16-bit sources with a query of another dtype (in earnest: a module's fp32
+// parameters), held as fp32 values; its dots are FMAs on widened elements.
+template <class T, int W, int VPL, int NR, bool WIDE = false>
 __global__ void __launch_bounds__(FwdGeom<W>::kBlock)
-k_fwd(const RowTable v, const typename T::storage* __restrict__ w,
+k_fwd(const RowTable v, const void* __restrict__ w, int wt,
       typename T::storage* __restrict__ out, float* __restrict__ stats, float* __restrict__ m_out,
       float* __restrict__ l_out, int normalize, int n_src, int64_t n_tok, int d, float eps,
       float inv_d) {
@@ -149,12 +160,8 @@ k_fwd(const RowTable v, const typename T::storage* __restrict__ w,
   const uint32_t row_bytes = (uint32_t)d * sizeof(S);
   const uint32_t lane_off = (uint32_t)(seg * 64 + lane) * 16u;
 
-  i32x4_t wq[VPL];
-  {
-    const auto wr = make_rsrc(w, row_bytes);
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) wq[j] = ld16(wr, lane_off + j * kStep);
-  }
+  Query<T, WIDE, VPL> wq;
+  wq.load(w, wt, (uint32_t)d, lane_off, kStep);
 
   float m_run = -INFINITY, l_run = 0.0f;
   float acc[VPL][CE];
@@ -190,7 +197,8 @@ k_fwd(const RowTable v, const typename T::storage* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             ss = dot<T>(x[n][j], x[n][j], ss);
-            dt = dot<T>(x[n][j], wq[j], dt);
+            dt = wq.dot(x[n][j], j, dt);
+            reconvert<WIDE>(x[n][j]);
           }
           tv[n] = ss;
           tv[NR + n] = dt;
@@ -205,7 +213,8 @@ k_fwd(const RowTable v, const typename T::storage* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             ss = dot<T>(x[n][j], x[n][j], ss);
-            dt = dot<T>(x[n][j], wq[j], dt);
+            dt = wq.dot(x[n][j], j, dt);
+            reconvert<WIDE>(x[n][j]);
           }
           part[n] = wave_sum(ss);
           part[NR + n] = wave_sum(dt);
@@ -498,9 +507,11 @@ k_batched(const RowTable v, const typename T::storage* __restrict__ q,
 // slower (T = 8192: 56.1 vs 56.5; T = 16384: 111.9 vs 113.3). A final token's
 // weights carry a different rounding than the two-pass form's, so a token's
 // bits depend on whether it is its wave's last (both within one rounding).
-template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false>
-__global__ void __launch_bounds__(FwdGeom<W>::kBlock)
-k_fwd_res(const RowTable v, const typename T::storage* __restrict__ w,
+// WIDE as in k_fwd. Its 9-row four-chunk tiles would take 256-268 VGPRs; they are
+// held to 256, two waves a SIMD like the packed query's (239).
+template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false, bool WIDE = false>
+__global__ void __launch_bounds__(FwdGeom<W>::kBlock, WIDE && VPL == 4 && NR == 9 ? 2 : 1)
+k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
           typename T::storage* __restrict__ out, float* __restrict__ stats,
           float* __restrict__ m_out, float* __restrict__ l_out, int normalize, int n_src,
           int64_t n_tok, int d, float eps, float inv_d, int n_iter,
@@ -532,12 +543,8 @@ k_fwd_res(const RowTable v, const typename T::storage* __restrict__ w,
   // sits at the use).
   const float* pstat_src = (lane & 1) ? pl : pm;
 
-  i32x4_t wq[VPL];
-  {
-    const auto wr = make_rsrc(w, row_bytes);
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) wq[j] = ld16(wr, lane_off + j * kStep);
-  }
+  Query<T, WIDE, VPL> wq;
+  wq.load(w, wt, (uint32_t)d, lane_off, kStep);
   i32x4_t x[NR][VPL];
   float pstat = 0.0f;
   {
@@ -589,7 +596,9 @@ k_fwd_res(const RowTable v, const typename T::storage* __restrict__ w,
 #pragma unroll
               for (int j = 0; j < VPL; ++j) {
                 ss = dot<T>(x[n][j], x[n][j], ss);
-                dt = dot<T>(x[n][j], wq[j], dt);
+                dt = wq.dot(x[n][j], j, dt);
+                reconvert<WIDE>(x[n][j]);
+            reconvert<WIDE>(x[n][j]);
               }
               const float pv[2] = {ss, dt};
               const float s2 = tsum<2>(pv, lane);  // lanes 0..31: ss, 32..63: dt
@@ -660,7 +669,8 @@ k_fwd_res(const RowTable v, const typename T::storage* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             ss = dot<T>(x[n][j], x[n][j], ss);
-            dt = dot<T>(x[n][j], wq[j], dt);
+            dt = wq.dot(x[n][j], j, dt);
+            reconvert<WIDE>(x[n][j]);
           }
           tv[n] = ss;
           tv[NR + n] = dt;
@@ -675,7 +685,8 @@ k_fwd_res(const RowTable v, const typename T::storage* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             ss = dot<T>(x[n][j], x[n][j], ss);
-            dt = dot<T>(x[n][j], wq[j], dt);
+            dt = wq.dot(x[n][j], j, dt);
+            reconvert<WIDE>(x[n][j]);
           }
           part[n] = wave_sum(ss);
           part[NR + n] = wave_sum(dt);
@@ -852,7 +863,7 @@ enum BwdVariant { kBwdStacked = 0, kBwdListed = 1, kBwdStatsGrad = 2 };
 
 template <class T, int W, int VPL, int NR, bool STATS, int VAR>
 __global__ void __launch_bounds__((BwdGeom<W, VPL, NR>::kBlock))
-k_bwd(const RowTable v, const typename T::storage* __restrict__ w,
+k_bwd(const RowTable v, const void* __restrict__ w, int wt,
       const typename T::storage* __restrict__ g, const float* __restrict__ stats,
       const float* __restrict__ gm, const float* __restrict__ gl, const RowTable dv,
       float* __restrict__ partial, int n_src, int64_t n_tok, int d, float eps, float inv_d,
@@ -906,9 +917,15 @@ k_bwd(const RowTable v, const typename T::storage* __restrict__ w,
   // 223.2 -> 221.5), nt alone elsewhere (N=4 27.6 vs 28.8, N=16 97.4 vs 98.2,
   // fp32 N=9 111.8 vs 112.7, D=1024 B=4 (two chunks) 118.9 vs 119.5 with the bit).
   constexpr int kDvAux = CE == 8 && NR == 9 && W * VPL >= 4 ? SY_DV_STORE_AUX : SY_STREAM_STORE_AUX;
+  // Only the fp32 copies are used with stats, so there the query may have any
+  // dtype; the recompute variants and the lean tile need it packed like v.
   float wf[VPL][CE];
-  i32x4_t wq[VPL];
-  {
+  [[maybe_unused]] i32x4_t wq[VPL];
+  if constexpr (STATS && !kLean) {
+    const auto wr = make_rsrc(w, (uint32_t)d * (wt == F32::code ? 4u : 2u));
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) ld_query<CE>(wr, (lane_off + j * kStep) / 16u, wt, wf[j]);
+  } else {
     const auto wr = make_rsrc(w, row_bytes);
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
@@ -1205,7 +1222,7 @@ struct TallGeom {
 
 template <class T, int W, int VPL, int NR>
 __global__ void __launch_bounds__((TallGeom<W, VPL, NR>::kBlock))
-k_bwd_tall(const RowTable v, const typename T::storage* __restrict__ w,
+k_bwd_tall(const RowTable v, const void* __restrict__ w, int wt,
            const typename T::storage* __restrict__ g, const float* __restrict__ stats,
            const RowTable dv, float* __restrict__ partial, int n_src, int64_t n_tok, int d,
            float inv_d, int n_iter) {
@@ -1235,15 +1252,10 @@ k_bwd_tall(const RowTable v, const typename T::storage* __restrict__ w,
   const int iters = n_iter;  // every slot meets the same barriers
 
   float wf[VPL][CE];
-  i32x4_t wq[VPL];
   {
-    const auto wr = make_rsrc(w, row_bytes);
+    const auto wr = make_rsrc(w, (uint32_t)d * (wt == F32::code ? 4u : 2u));
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      wq[j] = ld16(wr, lane_off + j * kStep);
-#pragma unroll
-      for (int e = 0; e < CE; ++e) wf[j][e] = elem<T>(wq[j], e);
-    }
+    for (int j = 0; j < VPL; ++j) ld_query<CE>(wr, (lane_off + j * kStep) / 16u, wt, wf[j]);
   }
   float dwa[VPL][CE];
 #pragma unroll

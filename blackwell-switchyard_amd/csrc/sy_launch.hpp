@@ -190,6 +190,16 @@ struct BwdBatchedArgs {
 int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_dtype, int aligned,
               sy_plan* out, int has_stats = 1, int matrix_ok = 1);
 
+// make_plan for a launch of the forward or the backward: as make_plan, except that
+// a query of another dtype than the sources (which sy_plan_for reports as generic)
+// runs the plan of the sources' dtype. The vector kernels hold such a query as fp32
+// values: 16-bit D=2048 N=9, 4096 tokens with an fp32 query, forward 230 -> 32 us,
+// backward 354 -> 57 us. The backward needs the forward's stats for it (the
+// recompute tiles keep the query packed in the sources' dtype), and 16-bit rows of
+// more than 1024 chunks stay generic (their eight-wave tile keeps it packed too).
+int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
+                     sy_plan* out, int has_stats = 1);
+
 // Measurement overrides installed with sy_tuning_set (sy_capi.cpp). Returns
 // false (and leaves *out untouched) when none are installed, which is the
 // default: then no launch depends on anything but shape, dtype, alignment
@@ -249,6 +259,9 @@ SY_DECLARE_VEC(bf16)
 SY_DECLARE_VEC(f16)
 SY_DECLARE_VEC(f32)
 #undef SY_DECLARE_VEC
+// launch_fwd_vec_* for 16-bit sources with a query of another dtype.
+hipError_t launch_fwd_wide_bf16(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info);
+hipError_t launch_fwd_wide_f16(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info);
 
 // Merge of two (o, m, l) partial results and its gradient (sy_merge.hip).
 // `vec` selects the 16-byte path (every row start 16-byte aligned).

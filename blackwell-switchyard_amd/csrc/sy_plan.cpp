@@ -252,6 +252,19 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
   return SY_OK;
 }
 
+int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
+                     sy_plan* out, int has_stats) {
+  const int rc = make_plan(op, n_src, 0, d, v_dtype, w_dtype, aligned, out, has_stats);
+  if (rc != SY_OK || out->family != SY_FAMILY_GENERIC || v_dtype == w_dtype || !aligned) return rc;
+  if (op != SY_OP_FWD && !(op == SY_OP_BWD && has_stats)) return rc;
+  sy_plan q;
+  if (make_plan(op, n_src, 0, d, v_dtype, v_dtype, aligned, &q, has_stats) != SY_OK) return rc;
+  const bool packed = op == SY_OP_BWD && q.elems_per_chunk == 8 && q.waves_per_token == 8 &&
+                      q.chunks_per_lane == 4;
+  if (!packed) *out = q;
+  return rc;
+}
+
 bool tile_listed(int op, int w, int vpl, int nr) {
 #define X(W_, V_, N_) \
   if (w == W_ && vpl == V_ && nr == N_) return true;
