@@ -321,16 +321,49 @@ bool vec_rows(bool rows_ok, int64_t d, int dtype) { return rows_ok && (d * esize
 // with m_out/l_out) over any row table. Sizes are already checked.
 int fwd_impl(const RowTable& v, bool v_ok, const void* w, void* out, float* stats, float* m_out,
              float* l_out, int normalize, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
-             int w_dtype, float eps, hipStream_t s) {
+             int w_dtype, float eps, hipStream_t s, int64_t stats_rows = 0) {
   const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out);
   sy_plan p;
   const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p);
   if (rc != SY_OK) return rc;
   apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
   if (n_tok == 0) return SY_OK;
-  const FwdArgs a{v,      w,       out,     stats,   m_out, l_out, normalize, (int)n_src,
-                  n_tok,  (int)d,  v_dtype, w_dtype, eps};
+  FwdArgs a{v,      w,       out,     stats,   m_out, l_out, normalize, (int)n_src,
+            n_tok,  (int)d,  v_dtype, w_dtype, eps};
+  a.stats_rows = (int)stats_rows;
   return status(p.family == SY_FAMILY_GENERIC ? launch_fwd_generic(a, s) : fwd_vec(p, a, s));
+}
+
+// Phase 2 of the two-phase schedule: this group's sources merged with a prior
+// group's (o1, m1, l1). `stats` (or nullptr) receives the group's logits and r in
+// an array whose planes are stats_rows rows apart.
+int merge_impl(RowTable t, bool ok, const void* w, const void* o1, const float* m1, const float* l1,
+               void* out, float* stats, int64_t stats_rows, float* m, float* l, int normalize,
+               int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, float eps,
+               hipStream_t s) {
+  // The prior's o1 rides in the register tile as row n_src: a resident tile
+  // of n_src + 1 rows, addressed through the table's row pointers.
+  const bool aligned = vec_rows(ok, d, v_dtype) && al16(w) && al16(out) && al16(o1);
+  sy_plan p;
+  int rc = make_plan(SY_OP_FWD, n_src + 1, 0, d, v_dtype, w_dtype, aligned, &p);
+  if (rc != SY_OK) return rc;
+  apply_tile_rules(SY_OP_FWD, n_src + 1, n_tok, d, &p, /*chunked_ok=*/false);
+  if (n_tok == 0) return SY_OK;
+  if (p.family == SY_FAMILY_RESIDENT && n_src + 1 <= kTableRows && p.rows_per_tile >= n_src + 1) {
+    t.p[n_src] = const_cast<void*>(o1);
+    FwdArgs a{t,      w,       out,     stats,   m,  l,  normalize, (int)n_src,
+              n_tok,  (int)d,  v_dtype, w_dtype, eps, m1, l1};
+    a.stats_rows = (int)stats_rows;
+    return status(fwd_vec(p, a, s));
+  }
+  // Beyond the resident tiles (more rows, unaligned rows, mixed dtypes): this
+  // group's (o, m, l) into out, m, l, then the merge over them in place.
+  rc = fwd_impl(t, ok, w, out, stats, m, l, 0, n_src, n_tok, d, v_dtype, w_dtype, eps, s, stats_rows);
+  if (rc != SY_OK) return rc;
+  const bool vec = al16(o1) && al16(out) && (d * esize(v_dtype)) % 16 == 0;
+  MergeArgs ma{o1, m1, l1, out, m, l, out, m, l, n_tok, (int)d};
+  ma.normalize = normalize;
+  return status(launch_merge(ma, v_dtype, vec, s));
 }
 
 // Main backward kernel over row tables: dv and the fp32 dw partials.
@@ -488,34 +521,34 @@ int sy_attn_with_stats_merge(const void* v, const void* w, const void* o1, const
   if (n_tok != 0 && (v == nullptr || w == nullptr || o1 == nullptr || m1 == nullptr ||
                      l1 == nullptr || out == nullptr || m == nullptr || l == nullptr))
     return SY_ERR_NULL;
-  int rc = check_common(n_src, n_tok, d, src_stride, v_dtype, w_dtype);
+  const int rc = check_common(n_src, n_tok, d, src_stride, v_dtype, w_dtype);
   if (rc != SY_OK) return rc;
   if (normalize != 0 && normalize != 1) return SY_ERR_OP;
   bool ok = false;
-  RowTable t = stacked(v, n_src, src_stride, v_dtype, &ok);
-  const hipStream_t s = (hipStream_t)stream;
-  // The prior's o1 rides in the register tile as row n_src: a resident tile
-  // of n_src + 1 rows, addressed through the table's row pointers.
-  const bool aligned = vec_rows(ok, d, v_dtype) && al16(w) && al16(out) && al16(o1);
-  sy_plan p;
-  rc = make_plan(SY_OP_FWD, n_src + 1, 0, d, v_dtype, w_dtype, aligned, &p);
+  const RowTable t = stacked(v, n_src, src_stride, v_dtype, &ok);
+  return merge_impl(t, ok, w, o1, m1, l1, out, nullptr, 0, m, l, normalize, n_src, n_tok, d, v_dtype,
+                    w_dtype, eps, (hipStream_t)stream);
+}
+
+int sy_two_phase(const void* v, const void* w, void* o1, float* ml, void* out, float* stats,
+                 int64_t n_src, int64_t split, int64_t n_tok, int64_t d, int64_t src_stride,
+                 int v_dtype, int w_dtype, float eps, void* stream) {
+  if (n_tok != 0 && (v == nullptr || w == nullptr || o1 == nullptr || ml == nullptr || out == nullptr))
+    return SY_ERR_NULL;
+  int rc = check_common(n_src, n_tok, d, src_stride, v_dtype, w_dtype);
   if (rc != SY_OK) return rc;
-  apply_tile_rules(SY_OP_FWD, n_src + 1, n_tok, d, &p, /*chunked_ok=*/false);
+  if (split < 1 || split >= n_src) return SY_ERR_SHAPE;
   if (n_tok == 0) return SY_OK;
-  if (p.family == SY_FAMILY_RESIDENT && n_src + 1 <= kTableRows && p.rows_per_tile >= n_src + 1) {
-    t.p[n_src] = const_cast<void*>(o1);
-    FwdArgs a{t,      w,       out,     nullptr, m,  l,  normalize, (int)n_src,
-              n_tok,  (int)d,  v_dtype, w_dtype, eps, m1, l1};
-    return status(fwd_vec(p, a, s));
-  }
-  // Beyond the resident tiles (more rows, unaligned rows, mixed dtypes): this
-  // group's (o, m, l) into out, m, l, then the merge over them in place.
-  rc = fwd_impl(t, ok, w, out, nullptr, m, l, 0, n_src, n_tok, d, v_dtype, w_dtype, eps, s);
+  const hipStream_t s = (hipStream_t)stream;
+  const void* v2 = static_cast<const char*>(v) + split * src_stride * esize(v_dtype);
+  bool ok1 = false, ok2 = false;
+  const RowTable t1 = stacked(v, split, src_stride, v_dtype, &ok1);
+  const RowTable t2 = stacked(v2, n_src - split, src_stride, v_dtype, &ok2);
+  float *m1 = ml, *l1 = ml + n_tok, *m2 = ml + 2 * n_tok, *l2 = ml + 3 * n_tok;
+  rc = fwd_impl(t1, ok1, w, o1, stats, m1, l1, 0, split, n_tok, d, v_dtype, w_dtype, eps, s, n_src);
   if (rc != SY_OK) return rc;
-  const bool vec = al16(o1) && al16(out) && (d * esize(v_dtype)) % 16 == 0;
-  MergeArgs ma{o1, m1, l1, out, m, l, out, m, l, n_tok, (int)d};
-  ma.normalize = normalize;
-  return status(launch_merge(ma, v_dtype, vec, s));
+  return merge_impl(t2, ok2, w, o1, m1, l1, out, stats ? stats + split * n_tok : nullptr, n_src, m2, l2,
+                    1, n_src - split, n_tok, d, v_dtype, w_dtype, eps, s);
 }
 
 int sy_sol(const void* v, void* out, int64_t n_src, int64_t n_tok, int64_t d, int64_t src_stride,

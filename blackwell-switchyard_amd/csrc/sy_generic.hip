@@ -110,8 +110,8 @@ __device__ void row_scalars(const RowTable& v, const void* w, const void* g, int
 __global__ void __launch_bounds__(kBlock)
 k_fwd_generic(const RowTable v, const void* __restrict__ w, void* __restrict__ out,
               float* __restrict__ stats, float* __restrict__ m_out, float* __restrict__ l_out,
-              int normalize, int n_src, int64_t n_tok, int d, int vt, int wt, float eps,
-              float inv_d) {
+              int normalize, int n_src, int stat_rows, int64_t n_tok, int d, int vt, int wt,
+              float eps, float inv_d) {
   extern __shared__ float sh[];
   float* lg = sh;
   float* ss = sh + n_src;
@@ -139,7 +139,7 @@ k_fwd_generic(const RowTable v, const void* __restrict__ w, void* __restrict__ o
   if (stats) {
     for (int n = tid; n < n_src; n += kBlock) {
       stats[(int64_t)n * n_tok + tok] = lg[n];
-      stats[(int64_t)(n_src + n) * n_tok + tok] = ss[n];
+      stats[(int64_t)(stat_rows + n) * n_tok + tok] = ss[n];
     }
   }
   __syncthreads();
@@ -504,8 +504,8 @@ k_probe_mix(const char* __restrict__ src, char* __restrict__ dst, int64_t out_by
 hipError_t launch_fwd_generic(const FwdArgs& a, hipStream_t s) {
   const size_t lds = (size_t)(2 * a.n_src + 257) * sizeof(float);
   hipLaunchKernelGGL(k_fwd_generic, dim3((unsigned)a.n_tok), dim3(kBlock), lds, s, a.v, a.w, a.out,
-                     a.stats, a.m_out, a.l_out, a.normalize, a.n_src, a.n_tok, a.d, a.v_dtype,
-                     a.w_dtype, a.eps, 1.0f / (float)a.d);
+                     a.stats, a.m_out, a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d,
+                     a.v_dtype, a.w_dtype, a.eps, 1.0f / (float)a.d);
   return hipGetLastError();
 }
 

@@ -78,14 +78,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
           if (n_iter <= 2 && km.blocks_per_cu >= kr.blocks_per_cu) {                         \
             hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true, true>), dim3(grid), dim3(kB), \
                                0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,      \
-                               a.l_out, a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d,    \
+                               a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, \
                                n_iter, a.prior_m, a.prior_l);                                \
             return hipGetLastError();                                                        \
           }                                                                                  \
         }                                                                                    \
         hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true>), dim3(grid), dim3(kB), 0, s, a.v, \
                            a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,            \
-                           a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,         \
+                           a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                            a.prior_m, a.prior_l);                                            \
         return hipGetLastError();                                                            \
       }                                                                                      \
@@ -95,14 +95,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
         if (n_iter <= 2 && kf.blocks_per_cu >= kr.blocks_per_cu) {                           \
           hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, true>), dim3(grid), dim3(kB), 0, \
                              s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,  \
-                             a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,       \
+                             a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                              nullptr, nullptr);                                              \
           return hipGetLastError();                                                          \
         }                                                                                    \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_>), dim3(grid), dim3(kB), 0, s, a.v,        \
                          a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
-                         a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter, nullptr, nullptr);     \
+                         a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, nullptr, nullptr); \
     } else {                                                                                 \
       if (a.prior_m != nullptr) return hipErrorInvalidConfiguration;                         \
       const int64_t grid = cdiv(a.n_tok, kT);                                                \
@@ -113,7 +113,7 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd<T, W_, V_, N_>), dim3((unsigned)grid), dim3(kB), 0, s, a.v,  \
                          a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
-                         a.n_src, a.n_tok, a.d, a.eps, inv_d);                               \
+                         a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);                \
     }                                                                                        \
     return hipGetLastError();                                                                \
   }
@@ -124,18 +124,18 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
 
 hipError_t SY_FN(launch_sol_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_t s) {
   const bool res = p.family == SY_FAMILY_RESIDENT;
-#define X(W_, V_, N_)                                                                          \
-  if (tile_is(p, W_, V_, N_)) {                                                                \
-    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                            \
-    if (res) {                                                                                 \
-      static const KernelRes kr = resources_of(k_sol_res<T, W_, V_, N_>, kB);                  \
-      hipLaunchKernelGGL((k_sol_res<T, W_, V_, N_>), dim3(launch_grid(kr, a.n_tok, kT)),       \
-                         dim3(kB), 0, s, a.v, (St*)a.out, a.n_src, a.n_tok, a.d);              \
-    } else {                                                                                   \
+#define X(W_, V_, N_)                                                                        \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
+    if (res) {                                                                               \
+      static const KernelRes kr = resources_of(k_sol_res<T, W_, V_, N_>, kB);                \
+      hipLaunchKernelGGL((k_sol_res<T, W_, V_, N_>), dim3(launch_grid(kr, a.n_tok, kT)),     \
+                         dim3(kB), 0, s, a.v, (St*)a.out, a.n_src, a.n_tok, a.d);            \
+    } else {                                                                                 \
       hipLaunchKernelGGL((k_sol<T, W_, V_, N_>), dim3((unsigned)cdiv(a.n_tok, kT)), dim3(kB), 0, \
-                         s, a.v, (St*)a.out, a.n_src, a.n_tok, a.d);                           \
-    }                                                                                          \
-    return hipGetLastError();                                                                  \
+                         s, a.v, (St*)a.out, a.n_src, a.n_tok, a.d);                         \
+    }                                                                                        \
+    return hipGetLastError();                                                                \
   }
   SY_TILES(X)
 #undef X
@@ -147,13 +147,13 @@ hipError_t SY_FN(launch_sol_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
 #if SY_PART == 2
 hipError_t SY_FN(launch_batched_vec_)(const sy_plan& p, const BatchedArgs& a, hipStream_t s) {
   const float inv_d = 1.0f / (float)a.d;
-#define X(W_, V_, N_)                                                                            \
-  if (tile_is(p, W_, V_, N_)) {                                                                  \
-    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                              \
+#define X(W_, V_, N_)                                                                        \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
     hipLaunchKernelGGL((k_batched<T, W_, V_, N_>), dim3((unsigned)cdiv(a.n_tok, kT)), dim3(kB), 0, \
-                       s, a.v, (const St*)a.q, (St*)a.out, a.m_out, a.l_out, a.normalize,        \
-                       a.n_src, a.n_q, a.n_tok, a.d, a.eps, inv_d);                              \
-    return hipGetLastError();                                                                    \
+                       s, a.v, (const St*)a.q, (St*)a.out, a.m_out, a.l_out, a.normalize,    \
+                       a.n_src, a.n_q, a.n_tok, a.d, a.eps, inv_d);                          \
+    return hipGetLastError();                                                                \
   }
   SY_TILES(X)
 #undef X
@@ -171,7 +171,7 @@ hipError_t SY_FN(bwd_vec_resources_)(const sy_plan& p, bool stats, int variant, 
   // 32- and 64-row tiles exist for the stacked operator gradient with stats only.
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
-    if (!stats || variant != kBwdStacked) return hipErrorInvalidConfiguration;              \
+    if (!stats || variant != kBwdStacked) return hipErrorInvalidConfiguration;               \
     static const KernelRes r =                                                               \
         resources_of(k_bwd_tall<T, W_, V_, N_>, TallGeom<W_, V_, N_>::kBlock);               \
     *out = r;                                                                                \
@@ -206,9 +206,9 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
   if (tile_is(p, W_, V_, N_)) {                                                              \
     if (a.stats == nullptr || a.listed || a.gm != nullptr) return hipErrorInvalidConfiguration; \
     hipLaunchKernelGGL((k_bwd_tall<T, W_, V_, N_>), dim3(grid), dim3(TallGeom<W_, V_, N_>::kBlock), 0, \
-                       s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.dv, a.partial,       \
-                       a.n_src, a.n_tok, a.d, inv_d, n_iter);                                 \
-    return hipGetLastError();                                                                 \
+                       s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.dv, a.partial,     \
+                       a.n_src, a.n_tok, a.d, inv_d, n_iter);                                \
+    return hipGetLastError();                                                                \
   }
   SY_BWD_TALL_TILES(X)
 #undef X
@@ -218,7 +218,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
                      a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter)
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
-    const int var = a.listed ? kBwdListed : (a.gm != nullptr ? kBwdStatsGrad : kBwdStacked);  \
+    const int var = a.listed ? kBwdListed : (a.gm != nullptr ? kBwdStatsGrad : kBwdStacked); \
     if (a.stats != nullptr) {                                                                \
       if (var == kBwdListed) SY_BWD_LAUNCH(W_, V_, N_, true, kBwdListed);                    \
       else if (var == kBwdStatsGrad) SY_BWD_LAUNCH(W_, V_, N_, true, kBwdStatsGrad);         \
@@ -246,12 +246,12 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
 
 hipError_t SY_FN(bwd_batched_vec_resources_)(const sy_plan& p, KernelRes* out) {
   // Sized by the variant with a runtime row count (the larger footprint).
-#define X(W_, N_)                                                                             \
-  if (tile_is(p, W_, 1, N_)) {                                                                \
-    static const KernelRes kr = resources_of(                                                 \
-        k_bwd_batched<T, W_, N_, (int)kBwdBatchedMaxQ, false>, FwdGeom<W_>::kBlock);            \
-    *out = kr;                                                                                \
-    return hipSuccess;                                                                        \
+#define X(W_, N_)                                                                            \
+  if (tile_is(p, W_, 1, N_)) {                                                               \
+    static const KernelRes kr = resources_of(                                                \
+        k_bwd_batched<T, W_, N_, (int)kBwdBatchedMaxQ, false>, FwdGeom<W_>::kBlock);         \
+    *out = kr;                                                                               \
+    return hipSuccess;                                                                       \
   }
   SY_BB_TILES(X)
 #undef X
@@ -262,15 +262,15 @@ hipError_t SY_FN(launch_bwd_batched_vec_)(const sy_plan& p, const BwdBatchedArgs
                                          hipStream_t s) {
   const float inv_d = 1.0f / (float)a.d;
   const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * p.tokens_per_block);
-#define SY_BB_LAUNCH(W_, N_, EX_)                                                             \
-  hipLaunchKernelGGL((k_bwd_batched<T, W_, N_, (int)kBwdBatchedMaxQ, EX_>), dim3(grid),       \
-                     dim3(FwdGeom<W_>::kBlock), 0, s, a.v, (const St*)a.q, (const St*)a.g,    \
+#define SY_BB_LAUNCH(W_, N_, EX_)                                                            \
+  hipLaunchKernelGGL((k_bwd_batched<T, W_, N_, (int)kBwdBatchedMaxQ, EX_>), dim3(grid),      \
+                     dim3(FwdGeom<W_>::kBlock), 0, s, a.v, (const St*)a.q, (const St*)a.g,   \
                      a.dv, a.partial, a.n_src, a.n_q, a.n_tok, a.d, a.eps, inv_d, n_iter)
-#define X(W_, N_)                                                                             \
-  if (tile_is(p, W_, 1, N_)) {                                                                \
-    if (a.n_src == N_) SY_BB_LAUNCH(W_, N_, true);                                            \
-    else SY_BB_LAUNCH(W_, N_, false);                                                         \
-    return hipGetLastError();                                                                 \
+#define X(W_, N_)                                                                            \
+  if (tile_is(p, W_, 1, N_)) {                                                               \
+    if (a.n_src == N_) SY_BB_LAUNCH(W_, N_, true);                                           \
+    else SY_BB_LAUNCH(W_, N_, false);                                                        \
+    return hipGetLastError();                                                                \
   }
   SY_BB_TILES(X)
 #undef X
@@ -302,7 +302,7 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
       const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * kT);                             \
       hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, true>), dim3(grid),         \
                          dim3(kB), 0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,  \
-                         a.l_out, a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter,  \
+                         a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                          nullptr, nullptr);                                                  \
     } else {                                                                                 \
       const int64_t grid = cdiv(a.n_tok, kT);                                                \
@@ -311,9 +311,9 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
         info->grid = (int)grid;                                                              \
         return hipSuccess;                                                                   \
       }                                                                                      \
-      hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true>), dim3((unsigned)grid), dim3(kB), \
+      hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true>), dim3((unsigned)grid), dim3(kB),       \
                          0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,   \
-                         a.normalize, a.n_src, a.n_tok, a.d, a.eps, inv_d);                  \
+                         a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);   \
     }                                                                                        \
     return hipGetLastError();                                                                \
   }

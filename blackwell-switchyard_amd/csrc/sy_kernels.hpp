@@ -127,7 +127,8 @@ __device__ __forceinline__ void row_sums_transposed(const float (&tv)[P], float 
 // merges chunks with the online-softmax update (running max m, running sum l,
 // accumulator rescaled by exp(m_old - m_new)), which still reads v once.
 //
-// Optional outputs: stats[n*n_tok + t] = logit, stats[(N+n)*n_tok + t] = r_n;
+// Optional outputs: stats[n*n_tok + t] = logit, stats[(stat_rows+n)*n_tok + t] = r_n
+// (stat_rows = N, or the whole source count when this launch takes one group of it);
 // m_out[t] = max logit and l_out[t] = sum_n exp(logit_n - m) (both or neither).
 // normalize = 0 stores the unnormalised o = sum_n exp(logit_n - m) v_n instead
 // of o / l (reference src/switchyard/reference.py:194-215, attn_with_stats).
@@ -138,8 +139,8 @@ template <class T, int W, int VPL, int NR, bool WIDE = false>
 __global__ void __launch_bounds__(FwdGeom<W>::kBlock)
 k_fwd(const RowTable v, const void* __restrict__ w, int wt,
       typename T::storage* __restrict__ out, float* __restrict__ stats, float* __restrict__ m_out,
-      float* __restrict__ l_out, int normalize, int n_src, int64_t n_tok, int d, float eps,
-      float inv_d) {
+      float* __restrict__ l_out, int normalize, int n_src, int stat_rows, int64_t n_tok, int d,
+      float eps, float inv_d) {
   using S = typename T::storage;
   constexpr int CE = T::ce;
   constexpr int TPB = FwdGeom<W>::kTpb;
@@ -233,7 +234,7 @@ k_fwd(const RowTable v, const void* __restrict__ w, int wt,
         cm = fmaxf(cm, lg[n]);
         if (stats != nullptr && seg == 0 && lane == 0 && live) {
           stats[(int64_t)(c0 + n) * n_tok + tok] = lg[n];
-          stats[(int64_t)(n_src + c0 + n) * n_tok + tok] = r;
+          stats[(int64_t)(stat_rows + c0 + n) * n_tok + tok] = r;
         }
       }
     }
@@ -514,7 +515,7 @@ __global__ void __launch_bounds__(FwdGeom<W>::kBlock, WIDE && VPL == 4 && NR == 
 k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
           typename T::storage* __restrict__ out, float* __restrict__ stats,
           float* __restrict__ m_out, float* __restrict__ l_out, int normalize, int n_src,
-          int64_t n_tok, int d, float eps, float inv_d, int n_iter,
+          int stat_rows, int64_t n_tok, int d, float eps, float inv_d, int n_iter,
           const float* __restrict__ pm = nullptr, const float* __restrict__ pl = nullptr) {
   using S = typename T::storage;
   constexpr int CE = T::ce;
@@ -637,7 +638,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
             sv = lane == 32 + n ? rr[n] : sv;
           }
           const int i = lane & 31;
-          if (i < rows) stats[(int64_t)((lane >> 5) * n_src + i) * n_tok + tok] = sv;
+          if (i < rows) stats[(int64_t)((lane >> 5) * stat_rows + i) * n_tok + tok] = sv;
         }
         if (m_out != nullptr && lane == 0) {
           m_out[tok] = m;
@@ -747,7 +748,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
           sv = lane == 32 + n ? part[n] : sv;
         }
         const int i = lane & 31;
-        if (i < rows) stats[(int64_t)((lane >> 5) * n_src + i) * n_tok + tok] = sv;
+        if (i < rows) stats[(int64_t)((lane >> 5) * stat_rows + i) * n_tok + tok] = sv;
       }
       if (m_out != nullptr && seg == 0 && lane == 0) {
         m_out[tok] = m;

@@ -134,6 +134,10 @@ struct FwdArgs {
   // is a prior group's o1, these its m1 and l1 [n_tok]; nullptr otherwise.
   const float* prior_m = nullptr;
   const float* prior_l = nullptr;
+  // Rows between the two planes of `stats`, when the launch fills one group's rows
+  // of a wider array (0: n_src, an array of its own).
+  int stats_rows = 0;
+  int stat_rows() const { return stats_rows > 0 ? stats_rows : n_src; }
 };
 
 struct BwdArgs {

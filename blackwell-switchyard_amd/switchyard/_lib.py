@@ -98,6 +98,7 @@ SIGNATURES = {
                                      ctypes.c_float, _vp]),
     "sy_attn_with_stats_merge": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                                         _i32, _i32, ctypes.c_float, _i32, _vp]),
+    "sy_two_phase": (_i32, [_vp] * 6 + [_i64] * 5 + [_i32, _i32, ctypes.c_float, _vp]),
     "sy_merge_stats": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp]),
     "sy_merge_stats_bwd": (_i32, [_vp] * 15 + [_i64, _i64, _i32, _vp]),
     "sy_bwd_batched_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32]),

@@ -65,6 +65,31 @@ def _validate(v: torch.Tensor, w: torch.Tensor) -> tuple[int, int, int, int]:
     return n, b, t, d
 
 
+def _operator_backward(v, w, stats, grad_out, eps: float):
+    """``(dv, dw)`` of the operator from the forward's saved (contiguous) v and
+    w and its statistics."""
+    n, b, t, d = v.shape
+    n_tok = b * t
+    grad_out = grad_out.to(v.dtype).contiguous()
+    dv = torch.empty_like(v, memory_format=torch.contiguous_format)
+    dw = torch.empty(d, device=v.device, dtype=w.dtype)
+    if d == 0:
+        return dv, dw
+    lib = _lib.lib()
+    vt, wt = _lib.dtype_code(v.dtype), _lib.dtype_code(w.dtype)
+    with torch.cuda.device(v.device):
+        ws_bytes = lib.sy_bwd_workspace_bytes(n, n_tok, d, vt, wt)
+        if ws_bytes < 0:
+            _lib.check(int(ws_bytes), "sy_bwd_workspace_bytes")
+        ws = torch.empty(max(1, (ws_bytes + 3) // 4), device=v.device, dtype=torch.float32)
+        rc = lib.sy_bwd(
+            _ptr(v), _ptr(w), _ptr(grad_out), _ptr(stats), _ptr(dv), _ptr(dw), _ptr(ws),
+            ws.numel() * 4, n, n_tok, d, n_tok * d, vt, wt, eps, _lib.stream_ptr(v.device),
+        )
+    _lib.check(rc, "sy_bwd")
+    return dv, dw
+
+
 class _BlockAttnResHIP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, v: torch.Tensor, w: torch.Tensor, eps: float):
@@ -97,25 +122,7 @@ class _BlockAttnResHIP(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out: torch.Tensor):
         v, w, stats = ctx.saved_tensors
-        n, b, t, d = v.shape
-        n_tok = b * t
-        grad_out = grad_out.to(v.dtype).contiguous()
-        dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-        dw = torch.empty(d, device=v.device, dtype=w.dtype)
-        if d == 0:
-            return dv, dw, None
-        lib = _lib.lib()
-        vt, wt = _lib.dtype_code(v.dtype), _lib.dtype_code(w.dtype)
-        with torch.cuda.device(v.device):
-            ws_bytes = lib.sy_bwd_workspace_bytes(n, n_tok, d, vt, wt)
-            if ws_bytes < 0:
-                _lib.check(int(ws_bytes), "sy_bwd_workspace_bytes")
-            ws = torch.empty(max(1, (ws_bytes + 3) // 4), device=v.device, dtype=torch.float32)
-            rc = lib.sy_bwd(
-                _ptr(v), _ptr(w), _ptr(grad_out), _ptr(stats), _ptr(dv), _ptr(dw), _ptr(ws),
-                ws.numel() * 4, n, n_tok, d, n_tok * d, vt, wt, ctx.eps, _lib.stream_ptr(v.device),
-            )
-        _lib.check(rc, "sy_bwd")
+        dv, dw = _operator_backward(v, w, stats, grad_out, ctx.eps)
         return dv, dw, None
 
 

@@ -29,7 +29,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .hip_op import _ptr, _validate, _validate_batched
+from .hip_op import _operator_backward, _ptr, _validate, _validate_batched
 from .reference import DEFAULT_EPS
 
 __all__ = [
@@ -251,6 +251,48 @@ def block_attn_res_batched_with_stats(v: torch.Tensor, queries: torch.Tensor, ep
     return o, m, ell
 
 
+class _TwoPhase(torch.autograd.Function):
+    """Forward: the schedule's two launches, filling one ``[2, N, B*T]`` statistics
+    array. The output is the operator's output over all sources, so the backward
+    is the operator's: one pass over ``v`` with those statistics, ``dv`` and
+    ``dw`` each written once (through the two phases' own gradients it read ``v``
+    and wrote ``dv`` in slices, filled and added to full-size tensors, and rounded
+    the partial results' gradients: forward + backward at N=9, split 4, T=4096,
+    D=2048 bf16 525-597 us, now 143 us of which the kernels take 100; dw's error
+    against float64 3.5e-3, now 1.7e-3)."""
+
+    @staticmethod
+    def forward(ctx, v: torch.Tensor, w: torch.Tensor, split: int, eps: float):
+        n, b, t, d = _validate(v, w)
+        v = v.contiguous()
+        w = w.contiguous()
+        n_tok = b * t
+        out = torch.empty(b, t, d, device=v.device, dtype=v.dtype)
+        want_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
+        stats = None
+        if n_tok > 0 and d > 0:
+            if want_grad:
+                stats = torch.empty(2, n, n_tok, device=v.device, dtype=torch.float32)
+            o1 = torch.empty_like(out)
+            ml = torch.empty(4, n_tok, device=v.device, dtype=torch.float32)
+            with torch.cuda.device(v.device):
+                rc = _lib.lib().sy_two_phase(
+                    _ptr(v), _ptr(w), _ptr(o1), _ptr(ml), _ptr(out), _ptr(stats), n, split, n_tok, d,
+                    n_tok * d, _lib.dtype_code(v.dtype), _lib.dtype_code(w.dtype), float(eps),
+                    _lib.stream_ptr(v.device),
+                )
+            _lib.check(rc, "sy_two_phase")
+        ctx.save_for_backward(v, w, stats)
+        ctx.eps = float(eps)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out: torch.Tensor):
+        v, w, stats = ctx.saved_tensors
+        dv, dw = _operator_backward(v, w, stats, grad_out, ctx.eps)
+        return dv, dw, None, None
+
+
 def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: float = DEFAULT_EPS):
     """The two-phase schedule for one query: sources ``[0, split)`` reduced to
     their ``(o, m, l)``, then sources ``[split, N)`` reduced and merged with
@@ -260,5 +302,4 @@ def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: 
     n = v.shape[0] if v.ndim == 4 else 0
     if not 0 < split < n:
         raise ValueError(f"split must be in (0, {n}), got {split}")
-    out, _, _ = attn_with_stats_merge(v[split:], w, *attn_with_stats(v[:split], w, eps), eps=eps)
-    return out
+    return _TwoPhase.apply(v, w, int(split), eps)

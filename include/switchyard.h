@@ -170,6 +170,19 @@ int sy_attn_with_stats_merge(const void* v, const void* w, const void* o1, const
                              int64_t n_tok, int64_t d, int64_t src_stride, int v_dtype,
                              int w_dtype, float eps, int normalize, void* stream);
 
+/* The two-phase schedule for one query: attn_with_stats over sources [0, split)
+ * into o1 and ml, then sources [split, n_src) merged with it as
+ * sy_attn_with_stats_merge (normalize = 1) does, into out. Two launches. o1 is
+ * scratch [n_tok][D] of v's dtype, ml scratch fp32 [4][n_tok]. `stats` as in
+ * sy_fwd, over all n_src sources: out is the operator's output, so sy_bwd on
+ * these stats is its gradient (one pass over v). SY_ERR_SHAPE for split outside
+ * [1, n_src). Reference: the paper's Algorithm 1 for one layer
+ * (src/switchyard/reference.py:195-201; tests/test_reference.py:139-150 states
+ * that it equals the single pass). */
+int sy_two_phase(const void* v, const void* w, void* o1, float* ml, void* out, float* stats,
+                 int64_t n_src, int64_t split, int64_t n_tok, int64_t d, int64_t src_stride,
+                 int v_dtype, int w_dtype, float eps, void* stream);
+
 /* Merge two (o, m, l) results of disjoint source groups into their union:
  * m = max(m1, m2), s_i = exp(m_i - m), o = s1 o1 + s2 o2, l = s1 l1 + s2 l2.
  * o may alias o1 or o2 (and m/l likewise). Replaces merge_online_softmax
