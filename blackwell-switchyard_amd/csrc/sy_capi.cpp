@@ -2,6 +2,7 @@
 // Every check that can be made on the host is made before any device work,
 // so bad arguments come back as negative sy_status codes. Nothing here
 // allocates device memory.
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -179,16 +180,31 @@ int bwd_batched_grid(const sy_plan& p, int64_t n_src, int64_t n_q, int64_t n_tok
   return SY_OK;
 }
 
-// Partial-row groups sy_bwd_batched_workspace_bytes provides: the grid of the
-// plan an aligned call takes when the matrix kernel's offsets fit. The other
-// plans (a source stride past the matrix kernel's 32-bit offsets, misaligned
-// buffers) are persistent over tokens at any grid and are capped to it.
-int batched_workspace_rows(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype,
-                           int* rows) {
+// Bytes of workspace of the two-pass kernels: partial rows, then coefficients.
+int64_t two_pass_bytes(const TwoPass& t, int64_t n_q, int64_t n_tok, int64_t d) {
+  return ((int64_t)t.groups * n_q * d + n_tok * t.coef_stride) * (int64_t)sizeof(float);
+}
+
+// What sy_bwd_batched_workspace_bytes provides: partial-row groups (*rows) for the
+// plan an aligned call takes when the matrix kernel's offsets fit, and *bytes with
+// what that plan needs besides. The other plans (a source stride past the matrix
+// kernel's 32-bit offsets, misaligned buffers) are persistent over tokens at any
+// grid and are capped to *rows.
+int batched_workspace(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype, int* rows,
+                      int64_t* bytes) {
   sy_plan p;
-  const int rc = make_plan(SY_OP_BWD_BATCHED, n_src, n_q, d, dtype, dtype, 1, &p, 1, 1);
+  int rc = make_plan(SY_OP_BWD_BATCHED, n_src, n_q, d, dtype, dtype, 1, &p, 1, 1);
   if (rc != SY_OK) return rc;
-  return bwd_batched_grid(p, n_src, n_q, n_tok, d, dtype, rows);
+  rc = bwd_batched_grid(p, n_src, n_q, n_tok, d, dtype, rows);
+  if (rc != SY_OK) return rc;
+  *bytes = *rows * n_q * d * (int64_t)sizeof(float);
+  if (two_pass_wanted(p, n_src, n_q, n_tok, d, dtype)) {
+    TwoPass t{};
+    const hipError_t e = two_pass_shape(n_src, n_q, n_tok, d, dtype, &t);
+    if (e != hipSuccess) return (int)e;
+    *bytes = std::max(*bytes, two_pass_bytes(t, n_q, n_tok, d));
+  }
+  return SY_OK;
 }
 
 
@@ -779,10 +795,9 @@ int64_t sy_bwd_batched_workspace_bytes(int64_t n_src, int64_t n_q, int64_t n_tok
   if (n_q < 1 || n_q > 0x7fffffff) return SY_ERR_SHAPE;
   if (n_tok == 0) return 0;
   int rows = 0;
-  rc = batched_workspace_rows(n_src, n_q, n_tok, d, dtype, &rows);
-  if (rc != SY_OK) return rc;
-  const int64_t g = rows;
-  return g * n_q * d * (int64_t)sizeof(float);
+  int64_t bytes = 0;
+  rc = batched_workspace(n_src, n_q, n_tok, d, dtype, &rows, &bytes);
+  return rc != SY_OK ? rc : bytes;
 }
 
 int sy_bwd_batched(const void* v, const void* queries, const void* grad_out, void* dv, void* dq,
@@ -807,17 +822,31 @@ int sy_bwd_batched(const void* v, const void* queries, const void* grad_out, voi
   if (rc != SY_OK) return rc;
   int grid = 0;
   if (n_tok != 0) {
+    BwdBatchedArgs a{tv,         queries,    grad_out, td,     (float*)workspace,
+                     (int)n_src, (int)n_q,   n_tok,    (int)d, dtype,
+                     eps};
+    if (aligned && two_pass_wanted(p, n_src, n_q, n_tok, d, dtype)) {
+      TwoPass t{};
+      const hipError_t e = two_pass_shape(n_src, n_q, n_tok, d, dtype, &t);
+      if (e != hipSuccess) return (int)e;
+      // A call that missed the matrix kernel by its source stride has a workspace
+      // sized for that kernel; too small for two passes, it takes the plan below.
+      if (workspace != nullptr && workspace_bytes >= two_pass_bytes(t, n_q, n_tok, d)) {
+        t.coef = (float*)workspace + (int64_t)t.groups * n_q * d;
+        const hipError_t el = launch_bwd_two_pass(a, t, s);
+        if (el != hipSuccess) return (int)el;
+        return status(launch_dw_reduce(a.partial, t.groups, (int)(n_q * d), dq, dtype, s));
+      }
+    }
     rc = bwd_batched_grid(p, n_src, n_q, n_tok, d, dtype, &grid);
     if (rc != SY_OK) return rc;
     int cap = 0;
-    rc = batched_workspace_rows(n_src, n_q, n_tok, d, dtype, &cap);
+    int64_t want = 0;
+    rc = batched_workspace(n_src, n_q, n_tok, d, dtype, &cap, &want);
     if (rc != SY_OK) return rc;
     if (grid > cap) grid = cap;
     if (workspace == nullptr || workspace_bytes < (int64_t)grid * n_q * d * (int64_t)sizeof(float))
       return SY_ERR_WORKSPACE;
-    const BwdBatchedArgs a{tv,         queries,    grad_out, td,     (float*)workspace,
-                           (int)n_src, (int)n_q,   n_tok,    (int)d, dtype,
-                           eps};
     hipError_t e;
     if (p.family == SY_FAMILY_GENERIC) {
       e = launch_bwd_batched_generic(a, grid, s);

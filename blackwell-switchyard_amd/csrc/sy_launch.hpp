@@ -105,6 +105,29 @@ inline bool bwd_matrix_offsets_fit(int64_t n_src, int64_t n_tok, int64_t d, int6
   return (n_src - 1) * g_stride < limit && (rpl - 1) * g_stride < limit &&
          (rpl - 1) * v_stride_bytes < limit;
 }
+// Batched backward in two passes (sy_batched.hip): rows of whole 16-byte chunks of
+// any dtype, at most 16 sources and 16 queries.
+inline bool two_pass_fits(int64_t n_src, int64_t n_q, int64_t d, int dtype) {
+  return n_src >= 1 && n_src <= 16 && n_q >= 1 && n_q <= 16 && d % (dtype == SY_F32 ? 4 : 8) == 0;
+}
+// Whether an aligned call of a shape whose plan is `p` runs them. Against the generic
+// kernel always (bf16 N=12 S=4 T=2048 D=1280 1087 -> 68 us, N=16 S=16 T=512 D=2048
+// 2144 -> 71). The register tile (N <= 9, S <= 8) spends reductions and multiply-adds
+// for every (query, source) pair, the two passes read v and g twice and launch once
+// more; both sides in us: bf16 N=9 S=8 T=4096 D=4096 574 vs 290; N=9 S=4 T=64 D=4096
+// 26.2 vs 20.0, D=256 14.4 vs 14.5; N=4 S=4 T=1024 D=1280 28.6 vs 21.0, D=256 12.1 vs
+// 14.2; N=9 S=2 T=8192 D=256 44.6 vs 43.0; N=4 S=2 T=8192 D=1280 93.6 vs 78.5,
+// T=1024 19.7 vs 19.9. fp32 (products of four columns): N=9 T=1024 D=1024 S=6 52.9 vs
+// 43.0, S=4 40.6 vs 37.6; T=64 S=6 20.7 vs 19.4, S=4 16.3 vs 18.3; N=4 S=4 T=8192
+// D=1024 116 vs 158.
+inline bool two_pass_wanted(const sy_plan& p, int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d,
+                            int dtype) {
+  if (p.family == SY_FAMILY_MATRIX || !two_pass_fits(n_src, n_q, d, dtype)) return false;
+  if (p.family == SY_FAMILY_GENERIC) return true;
+  const int64_t pairs = n_src * n_q, elems = n_tok * d;
+  if (dtype == SY_F32) return pairs >= 48;
+  return pairs >= 32 || (n_q >= 2 && ((pairs >= 16 && elems >= (1 << 20)) || elems >= (1 << 23)));
+}
 // Dynamic LDS the generic kernels may request (bytes).
 constexpr int64_t kGenericMaxLds = 64 * 1024;
 // LDS of the generic batched backward: per-(query, row) alpha and da, per-row
@@ -231,6 +254,19 @@ hipError_t launch_batched_matrix(const BatchedArgs& a, hipStream_t s, KernelRes*
 // launches nothing.
 hipError_t launch_bwd_batched_matrix(const BwdBatchedArgs& a, int grid, hipStream_t s,
                                      KernelRes* info);
+
+// Launch shape of the two-pass batched backward: `groups` partial rows a query, then
+// (at `coef`) coef_stride floats a token.
+struct TwoPass {
+  int waves_per_simd;
+  int coef_stride;
+  int slices;
+  int groups;
+  float* coef;
+};
+// Fills the shape for the current device (the arguments must pass two_pass_fits).
+hipError_t two_pass_shape(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype, TwoPass* out);
+hipError_t launch_bwd_two_pass(const BwdBatchedArgs& a, const TwoPass& t, hipStream_t s);
 
 // Device queries, cached per device (sy_capi.cpp).
 hipError_t cu_count(int* out);
