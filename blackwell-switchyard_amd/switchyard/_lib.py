@@ -136,6 +136,32 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The native torch functions over the library (csrc/sy_torch.cpp). Each
+    returns ``None`` for a call it leaves to the Python path."""
+    global _native
+    if _native is None:
+        lib()  # one clear error when nothing is built
+        try:
+            from . import _sy_torch
+        except ImportError as e:
+            raise RuntimeError(
+                f"switchyard's native torch functions did not load ({e}); build them with "
+                "`make -C blackwell-switchyard_amd/csrc` (there is no fallback path)"
+            ) from e
+        _native = _sy_torch
+    return _native
+
+
+def ordinary(*tensors) -> bool:
+    """Whether the native functions may be offered a call: tensors, outside a
+    compiler's trace (which has to see the Python function)."""
+    return not torch.compiler.is_compiling() and all(isinstance(t, torch.Tensor) for t in tensors)
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODES[dtype]

@@ -18,6 +18,10 @@ The backward is one persistent kernel that writes ``dv`` and per-workgroup
 fp32 ``dw`` partials, then a fixed-order reduction writes ``dw`` in
 ``w.dtype``: two kernels, no float atomics, bit-reproducible.
 
+Ordinary calls run as native torch functions (csrc/sy_torch.cpp); the autograd
+functions here state the same operations for everything else -- what the checks
+refuse, function transforms, tensor subclasses and modes, tracing.
+
 There is no fallback: when the HIP library is missing, or a tensor is not on
 a GPU, these functions raise.
 """
@@ -139,6 +143,10 @@ def block_attn_res_hip(v: torch.Tensor, w: torch.Tensor, eps: float = DEFAULT_EP
         ``[B, T, D]`` in ``v.dtype``. Gradients: ``dv`` in ``v.dtype``, ``dw``
         accumulated in fp32 and returned in ``w.dtype``.
     """
+    if _lib.ordinary(v, w):
+        out = _lib.native().block_attn_res(v, w, float(eps))
+        if out is not None:
+            return out
     return _BlockAttnResHIP.apply(v, w, eps)
 
 
@@ -222,6 +230,10 @@ def block_attn_res_batched_train(
     per-workgroup ``dq`` partials, then the fixed-order reduction writes
     ``dq`` -- two kernels, bit-reproducible.
     """
+    if _lib.ordinary(v, queries):
+        out = _lib.native().block_attn_res_batched_train(v, queries, float(eps))
+        if out is not None:
+            return out
     return _BlockAttnResBatched.apply(v, queries, eps)
 
 
@@ -236,6 +248,10 @@ def block_attn_res_batched(
     and S <= 16 one kernel reads ``v`` once; other shapes issue one forward
     launch per query, written straight into ``out[s]`` (no stack).
     """
+    if _lib.ordinary(v, queries):
+        out = _lib.native().block_attn_res_batched(v, queries, float(eps))
+        if out is not None:
+            return out
     _validate_batched(v, queries)
     if v.requires_grad or queries.requires_grad:
         raise RuntimeError(

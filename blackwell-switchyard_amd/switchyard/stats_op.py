@@ -302,4 +302,8 @@ def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: 
     n = v.shape[0] if v.ndim == 4 else 0
     if not 0 < split < n:
         raise ValueError(f"split must be in (0, {n}), got {split}")
+    if _lib.ordinary(v, w):
+        out = _lib.native().block_attn_res_two_phase(v, w, int(split), float(eps))
+        if out is not None:
+            return out
     return _TwoPhase.apply(v, w, int(split), eps)
