@@ -46,7 +46,13 @@ sy_tuning g_tuning{};
 
 // variant: 0 operator over stacked rows, 1 over per-row pointers, 2 the
 // (o, m, l) gradient over stacked rows (BwdVariant in sy_kernels.hpp).
-hipError_t bwd_resources(const sy_plan& p, int dtype, bool stats, int variant, KernelRes* out) {
+hipError_t bwd_resources(const sy_plan& p, bool unal, int dtype, bool stats, int variant,
+                         KernelRes* out) {
+  if (unal) {
+    if (dtype == SY_BF16) return bwd_unal_resources_bf16(p, out);
+    if (dtype == SY_F16) return bwd_unal_resources_f16(p, out);
+    return bwd_unal_resources_f32(p, out);
+  }
   if (dtype == SY_BF16) return bwd_vec_resources_bf16(p, stats, variant, out);
   if (dtype == SY_F16) return bwd_vec_resources_f16(p, stats, variant, out);
   return bwd_vec_resources_f32(p, stats, variant, out);
@@ -56,14 +62,15 @@ hipError_t bwd_resources(const sy_plan& p, int dtype, bool stats, int variant, K
 // kernel's register/LDS occupancy, never more than there are token slots.
 // Deterministic in (plan, n_tok, stats, addressing, device), which keeps dw
 // bit-stable.
-int bwd_grid(const sy_plan& p, int64_t n_tok, int dtype, bool stats, int variant, int* grid) {
+int bwd_grid(const sy_plan& p, bool unal, int64_t n_tok, int dtype, bool stats, int variant,
+             int* grid) {
   int cus = 0;
   hipError_t e = cu_count(&cus);
   if (e != hipSuccess) return e == hipErrorNoDevice ? SY_ERR_DEVICE : (int)e;
   int per_cu = 4;
   if (p.family != SY_FAMILY_GENERIC) {
     KernelRes r;
-    e = bwd_resources(p, dtype, stats, variant, &r);
+    e = bwd_resources(p, unal, dtype, stats, variant, &r);
     if (e != hipSuccess) return (int)e;
     per_cu = r.blocks_per_cu;
   }
@@ -83,9 +90,9 @@ int bwd_grid(const sy_plan& p, int64_t n_tok, int dtype, bool stats, int variant
 // operator gradient with stats only) becomes the generic kernel for every
 // other caller.
 int bwd_plan(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, int aligned,
-             bool stats, int variant, sy_plan* p) {
-  int rc = make_launch_plan(SY_OP_BWD, n_src, d, v_dtype, w_dtype, aligned, p, stats);
-  if (rc != SY_OK) return rc;
+             bool stats, int variant, sy_plan* p, bool* unal) {
+  int rc = make_launch_plan(SY_OP_BWD, n_src, d, v_dtype, w_dtype, aligned, p, unal, stats, variant);
+  if (rc != SY_OK || *unal) return rc;
   apply_tile_rules(SY_OP_BWD, n_src, n_tok, d, p);
   if (p->family != SY_FAMILY_GENERIC && p->rows_per_tile > 16 && (!stats || variant != 0))
     rc = make_plan(SY_OP_BWD, n_src, 0, d, v_dtype, w_dtype, 0, p, stats);
@@ -108,10 +115,11 @@ int workspace_rows(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_d
   for (bool st : {true, false}) {
     for (int var : {0, 1, 2}) {
       sy_plan p;
-      int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, 1, st, var, &p);
+      bool unal = false;
+      int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, 1, st, var, &p, &unal);
       if (rc != SY_OK) return rc;
       int gi = 0;
-      rc = bwd_grid(p, n_tok, v_dtype, st, var, &gi);
+      rc = bwd_grid(p, unal, n_tok, v_dtype, st, var, &gi);
       if (rc != SY_OK) return rc;
       if (gi > g) g = gi;
     }
@@ -120,12 +128,12 @@ int workspace_rows(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_d
   return SY_OK;
 }
 
-// The backward's grid for plan p: bwd_grid, capped to workspace_rows for the
-// generic kernel.
-int bwd_grid_for(const sy_plan& p, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
+// The backward's grid for plan p: bwd_grid, capped to workspace_rows for the generic
+// and the unaligned kernels (which misaligned buffers of any shape may take).
+int bwd_grid_for(const sy_plan& p, bool unal, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
                  int w_dtype, bool stats, int variant, int* grid) {
-  int rc = bwd_grid(p, n_tok, v_dtype, stats, variant, grid);
-  if (rc != SY_OK || p.family != SY_FAMILY_GENERIC) return rc;
+  int rc = bwd_grid(p, unal, n_tok, v_dtype, stats, variant, grid);
+  if (rc != SY_OK || (p.family != SY_FAMILY_GENERIC && !unal)) return rc;
   int rows = 0;
   rc = workspace_rows(n_src, n_tok, d, v_dtype, w_dtype, &rows);
   if (rc != SY_OK) return rc;
@@ -208,7 +216,13 @@ int batched_workspace(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int 
 }
 
 
-hipError_t fwd_vec(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info = nullptr) {
+hipError_t fwd_vec(const sy_plan& p, bool unal, const FwdArgs& a, hipStream_t s,
+                   KernelRes* info = nullptr) {
+  if (unal) {
+    if (a.v_dtype == SY_BF16) return launch_fwd_unal_bf16(p, a, s, info);
+    if (a.v_dtype == SY_F16) return launch_fwd_unal_f16(p, a, s, info);
+    return launch_fwd_unal_f32(p, a, s, info);
+  }
   const bool wide = a.w_dtype != a.v_dtype;
   if (a.v_dtype == SY_BF16)
     return wide ? launch_fwd_wide_bf16(p, a, s, info) : launch_fwd_vec_bf16(p, a, s, info);
@@ -226,7 +240,12 @@ hipError_t batched_vec(const sy_plan& p, const BatchedArgs& a, hipStream_t s) {
   if (a.dtype == SY_F16) return launch_batched_vec_f16(p, a, s);
   return launch_batched_vec_f32(p, a, s);
 }
-hipError_t bwd_vec(const sy_plan& p, const BwdArgs& a, int grid, hipStream_t s) {
+hipError_t bwd_vec(const sy_plan& p, bool unal, const BwdArgs& a, int grid, hipStream_t s) {
+  if (unal) {
+    if (a.v_dtype == SY_BF16) return launch_bwd_unal_bf16(p, a, grid, s);
+    if (a.v_dtype == SY_F16) return launch_bwd_unal_f16(p, a, grid, s);
+    return launch_bwd_unal_f32(p, a, grid, s);
+  }
   if (a.v_dtype == SY_BF16) return launch_bwd_vec_bf16(p, a, grid, s);
   if (a.v_dtype == SY_F16) return launch_bwd_vec_f16(p, a, grid, s);
   return launch_bwd_vec_f32(p, a, grid, s);
@@ -340,14 +359,15 @@ int fwd_impl(const RowTable& v, bool v_ok, const void* w, void* out, float* stat
              int w_dtype, float eps, hipStream_t s, int64_t stats_rows = 0) {
   const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out);
   sy_plan p;
-  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p);
+  bool unal = false;
+  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p, &unal);
   if (rc != SY_OK) return rc;
-  apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
+  if (!unal) apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
   if (n_tok == 0) return SY_OK;
   FwdArgs a{v,      w,       out,     stats,   m_out, l_out, normalize, (int)n_src,
             n_tok,  (int)d,  v_dtype, w_dtype, eps};
   a.stats_rows = (int)stats_rows;
-  return status(p.family == SY_FAMILY_GENERIC ? launch_fwd_generic(a, s) : fwd_vec(p, a, s));
+  return status(p.family == SY_FAMILY_GENERIC ? launch_fwd_generic(a, s) : fwd_vec(p, unal, a, s));
 }
 
 // Phase 2 of the two-phase schedule: this group's sources merged with a prior
@@ -370,7 +390,7 @@ int merge_impl(RowTable t, bool ok, const void* w, const void* o1, const float* 
     FwdArgs a{t,      w,       out,     stats,   m,  l,  normalize, (int)n_src,
               n_tok,  (int)d,  v_dtype, w_dtype, eps, m1, l1};
     a.stats_rows = (int)stats_rows;
-    return status(fwd_vec(p, a, s));
+    return status(fwd_vec(p, false, a, s));
   }
   // Beyond the resident tiles (more rows, unaligned rows, mixed dtypes): this
   // group's (o, m, l) into out, m, l, then the merge over them in place.
@@ -393,17 +413,18 @@ int bwd_main_impl(const RowTable& v, bool v_ok, const void* w, const void* g, co
   const bool aligned = vec_rows(v_ok && dv_ok, d, v_dtype) && al16(w) && al16(g) && al16(workspace);
   sy_plan p;
   const int variant = listed ? 1 : (gm != nullptr ? 2 : 0);
-  int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, stats != nullptr, variant, &p);
+  bool unal = false;
+  int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, stats != nullptr, variant, &p, &unal);
   if (rc != SY_OK) return rc;
   int grid = 0;
-  rc = bwd_grid_for(p, n_src, n_tok, d, v_dtype, w_dtype, stats != nullptr, variant, &grid);
+  rc = bwd_grid_for(p, unal, n_src, n_tok, d, v_dtype, w_dtype, stats != nullptr, variant, &grid);
   if (rc != SY_OK) return rc;
   if (workspace == nullptr || workspace_bytes < (int64_t)grid * d * (int64_t)sizeof(float))
     return SY_ERR_WORKSPACE;
   const BwdArgs a{v,      w,       g,     stats,  gm,      gl,      dv,  (float*)workspace, listed,
                   (int)n_src, n_tok, (int)d, v_dtype, w_dtype, eps};
   const hipError_t e =
-      p.family == SY_FAMILY_GENERIC ? launch_bwd_generic(a, grid, s) : bwd_vec(p, a, grid, s);
+      p.family == SY_FAMILY_GENERIC ? launch_bwd_generic(a, grid, s) : bwd_vec(p, unal, a, grid, s);
   if (e != hipSuccess) return (int)e;
   *rows_out = grid;
   return SY_OK;
@@ -484,9 +505,10 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
   if (out == nullptr) return SY_ERR_NULL;
   if (n_tok < 0) return SY_ERR_SHAPE;
   int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  bool unal = false;
   if (rc == SY_OK && (op == SY_OP_FWD || op == SY_OP_BWD))
-    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out);
-  if (rc != SY_OK) return rc;
+    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal);
+  if (rc != SY_OK || unal) return rc;
   if (op == SY_OP_FWD || op == SY_OP_BWD) apply_tile_rules(op, n_src, n_tok, d, out);
   return SY_OK;
 }
@@ -697,10 +719,11 @@ int64_t sy_bwd_partial_rows(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype
   if (rc != SY_OK) return rc;
   if (n_tok == 0) return 0;
   sy_plan p;
-  rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, has_stats != 0, 0, &p);
+  bool unal = false;
+  rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, has_stats != 0, 0, &p, &unal);
   if (rc != SY_OK) return rc;
   int grid = 0;
-  rc = bwd_grid_for(p, n_src, n_tok, d, v_dtype, w_dtype, has_stats != 0, 0, &grid);
+  rc = bwd_grid_for(p, unal, n_src, n_tok, d, v_dtype, w_dtype, has_stats != 0, 0, &grid);
   return rc != SY_OK ? rc : grid;
 }
 
@@ -711,9 +734,10 @@ int sy_kernel_info(int op, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
   if (rc != SY_OK) return rc;
   if (op != SY_OP_FWD && op != SY_OP_BWD) return SY_ERR_OP;
   sy_plan p;
-  rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, 1, &p);
+  bool unal = false;
+  rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, 1, &p, &unal);
   if (rc != SY_OK) return rc;
-  apply_tile_rules(op, n_src, n_tok, d, &p);
+  if (!unal) apply_tile_rules(op, n_src, n_tok, d, &p);
   out[0] = out[1] = out[2] = out[3] = 0;
   if (p.family == SY_FAMILY_GENERIC) return SY_OK;
   KernelRes r{0, 0, 0, 0};
@@ -721,11 +745,11 @@ int sy_kernel_info(int op, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
   if (op == SY_OP_FWD) {
     const FwdArgs a{RowTable{}, nullptr, nullptr, nullptr, nullptr, nullptr, 1, (int)n_src,
                     n_tok,      (int)d,  v_dtype, w_dtype, 0.0f};
-    e = fwd_vec(p, a, nullptr, &r);
+    e = fwd_vec(p, unal, a, nullptr, &r);
   } else {
-    e = bwd_resources(p, v_dtype, true, 0, &r);
+    e = bwd_resources(p, unal, v_dtype, true, 0, &r);
     if (e == hipSuccess) {
-      rc = bwd_grid(p, n_tok, v_dtype, true, 0, &r.grid);
+      rc = bwd_grid(p, unal, n_tok, v_dtype, true, 0, &r.grid);
       if (rc != SY_OK) return rc;
     }
   }

@@ -296,6 +296,89 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, float x, int dtyp
   }
 }
 
+// ------------------------------------------------------------ row access
+//
+// A lane's 16-byte chunk of a row. UNAL = false: the row starts at a 16-byte
+// boundary and holds whole chunks; the buffer resource masks what lies past it.
+// UNAL = true: a row of at least 16 bytes that starts at any element. The chunk is
+// read and written with unaligned 16-byte global accesses, the last one moved back to
+// end with the row: it overlaps the chunk before it and repeats its last elements.
+// Lanes past the row read that chunk too and store nothing. Everything element-wise
+// (out, dv, dw) then holds the same value in both lanes; only sums over the row have
+// to leave the repeated elements out (TailMask).
+typedef int i32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef int i32x4_f32_t __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ uint32_t tail_off(uint32_t off, uint32_t row_bytes) {
+  return min(off, row_bytes - 16u);
+}
+template <bool UNAL, class S>
+__device__ __forceinline__ i32x4_t ld_row(const S* row, uint32_t row_bytes, uint32_t off) {
+  if constexpr (UNAL) {
+    const char* p = reinterpret_cast<const char*>(row) + tail_off(off, row_bytes);
+    if constexpr (sizeof(S) == 4) return __builtin_nontemporal_load(reinterpret_cast<const i32x4_f32_t*>(p));
+    else return __builtin_nontemporal_load(reinterpret_cast<const i32x4_any_t*>(p));
+  } else {
+    return ld16_stream(make_rsrc(row, row_bytes), off);
+  }
+}
+template <bool UNAL, int AUX, class S>
+__device__ __forceinline__ void st_row(S* row, uint32_t row_bytes, uint32_t off, bool live, i32x4_t x) {
+  if constexpr (UNAL) {
+    if (live && off < row_bytes) {
+      char* p = reinterpret_cast<char*>(row) + tail_off(off, row_bytes);
+      if constexpr (sizeof(S) == 4) __builtin_nontemporal_store(x, reinterpret_cast<i32x4_f32_t*>(p));
+      else __builtin_nontemporal_store(x, reinterpret_cast<i32x4_any_t*>(p));
+    }
+  } else {
+    st16_aux<AUX>(make_rsrc(row, live ? row_bytes : 0u), off, x);
+  }
+}
+// The bits of the chunk at `off` that are not repeats: all of them, or for the row's
+// last chunk its last (row_bytes - off) bytes, or none past the row.
+__device__ __forceinline__ i32x4_t tail_mask(uint32_t off, uint32_t row_bytes) {
+  const int dup = off >= row_bytes ? 16 : max(0, (int)(off + 16u - row_bytes));  // bytes
+  i32x4_t m;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m[k] = dup <= 4 * k ? -1 : dup >= 4 * k + 4 ? 0 : (int)0xffff0000;
+  return m;
+}
+template <bool UNAL, int VPL>
+__device__ __forceinline__ i32x4_t own_part(const i32x4_t& x, int j, const i32x4_t& mask) {
+  if constexpr (UNAL) return j == VPL - 1 ? (x & mask) : x;
+  else return x;
+}
+
+// The query elements of the chunk at `off` of such a row (no alignment assumed).
+template <int CE>
+__device__ __forceinline__ void ld_query_any(const void* w, uint32_t off, uint32_t row_bytes, int wt,
+                                             float* f) {
+  const int64_t c = tail_off(off, row_bytes) / (16 / CE);
+  if (wt == F32::code) {
+#pragma unroll
+    for (int q = 0; q < CE / 4; ++q) {
+      const i32x4_t x = *reinterpret_cast<const i32x4_f32_t*>(static_cast<const float*>(w) + c + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * q + e] = __int_as_float(x[e]);
+    }
+    return;
+  }
+  const uint16_t* h = static_cast<const uint16_t*>(w) + c;
+  uint32_t x[CE];
+  if constexpr (CE == 8) {
+    const i32x4_t t = *reinterpret_cast<const i32x4_any_t*>(h);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (uint32_t)t[e / 2] >> (16 * (e & 1)) & 0xffffu;
+  } else {
+#pragma unroll
+    for (int e = 0; e < CE; ++e) x[e] = h[e];
+  }
+#pragma unroll
+  for (int e = 0; e < CE; ++e)
+    f[e] = wt == BF16::code ? __uint_as_float(x[e] << 16)
+                            : (float)__builtin_bit_cast(_Float16, (uint16_t)x[e]);
+}
+
 // ---------------------------------------------------------------- reductions
 
 template <int CTRL, int ROW_MASK = 0xf>

@@ -1,6 +1,6 @@
-// Generic kernels for shapes the register-tiled kernels do not cover: rows
-// that are not 16-byte aligned (D = 777, D = 63, ...), a query whose dtype
-// differs from v's, N beyond the tile budgets, or very wide D. One 256-thread
+// Generic kernels for shapes the register-tiled kernels do not cover: rows of
+// less than 16 bytes or more than 1024 chunks, odd rows without the forward's
+// stats, N beyond the tile budgets. One 256-thread
 // workgroup per token, element-wise loads, two passes: the first computes the
 // per-row scalars (kept in LDS), the second re-reads v to produce outputs. The
 // second read is served from L2 for all but the widest rows. These are
@@ -334,89 +334,81 @@ k_bwd_batched_generic(const RowTable v, const void* __restrict__ q, const void* 
   }
 }
 
-// dw[c] = sum over rows r of partial[r][c] (scalar path: any D, any
-// alignment), in a fixed order: wave q of the
-// 1024-thread workgroup sums rows [q*rows/16, (q+1)*rows/16) in sequence, then
-// the 16 wave sums are added in wave order. Same inputs, same bits.
-__global__ void __launch_bounds__(1024)
-k_dw_reduce(const float* __restrict__ partial, int rows, int d, void* __restrict__ dw, int wt) {
-  __shared__ float sh[16][64];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = blockIdx.x * 64 + lane;
-  float s = 0.0f;
-  if (col < d) {
-    const int r0 = (int)((int64_t)wave * rows / 16), r1 = (int)((int64_t)(wave + 1) * rows / 16);
-    for (int r = r0; r < r1; ++r) s += partial[(int64_t)r * d + col];
-  }
-  sh[wave][lane] = s;
-  __syncthreads();
-  if (wave == 0 && col < d) {
-    float t = sh[0][lane];
-#pragma unroll
-    for (int q = 1; q < 16; ++q) t += sh[q][lane];
-    store_elem(dw, col, t, wt);
-  }
+// Both halves of a swap end up with (low lanes' value) + (high lanes'), in that
+// order, so the lanes that meet later hold identical bits.
+template <bool ACROSS32>
+__device__ __forceinline__ float pair_sum(float x) {
+  const uint32_t u = __float_as_uint(x);
+  const auto r = ACROSS32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                          : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// dw[c] = sum over rows of partial[r][c], 16-byte path (D % 4 == 0, rows
-// 16-byte aligned). A workgroup owns 64 columns: lane l of wave w is column
-// group l % 16 (four columns) and row lane rl = 4w + l / 16, which sums rows
-// rl, rl + 64, rl + 128, ... in that order (four loads in flight per step).
+// dw[c] = sum over rows of partial[r][c]. A workgroup owns 16 * V columns: lane l of
+// wave w is column group l % 16 (V columns) and row lane rl = 4w + l / 16, which sums
+// rows rl, rl + 64, rl + 128, ... in that order (four loads in flight per step).
 // Each wave then adds its four row lanes with two lane swaps (row lane q takes
 // q ^ 2, then q ^ 1: permlane32 / permlane16), and after one barrier wave 0
-// adds the 16 wave sums in wave order. Same inputs, same bits.
+// adds the 16 wave sums in wave order. Same inputs, same bits. V = 4 loads 16 bytes
+// (D % 4 == 0, rows 16-byte aligned), V = 1 serves any D and alignment (1024 rows of
+// 777: 2.5-3.1 us, against 19.2 with 16 row lanes and one load in flight).
+template <int V>
 __global__ void __launch_bounds__(1024)
-k_dw_reduce4(const float* __restrict__ partial, int rows, int d, void* __restrict__ dw, int wt) {
-  __shared__ float4 sh[16][16];
+k_dw_reduce(const float* __restrict__ partial, int rows, int d, void* __restrict__ dw, int wt) {
+  struct Vec { float x[V]; };
+  typedef float vec_t __attribute__((ext_vector_type(4)));
+  __shared__ Vec sh[16][16];
   const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
   const int cl = lane & 15;
-  const int rl = (threadIdx.x >> 6) * 4 + (lane >> 4);
-  const int n4 = d / 4;
-  const int c4 = blockIdx.x * 16 + cl;
-  const float4* __restrict__ p4 = reinterpret_cast<const float4*>(partial);
-  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (c4 < n4) {
+  const int rl = wave * 4 + (lane >> 4);
+  const int c0 = ((int)blockIdx.x * 16 + cl) * V;  // first column
+  const bool in = c0 < d;
+  auto load = [&](int r) {
+    Vec t;
+    const float* p = partial + (int64_t)r * d + c0;
+    if constexpr (V == 4) {
+      const vec_t q = *reinterpret_cast<const vec_t*>(p);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t.x[k] = q[k];
+    } else {
+      t.x[0] = *p;
+    }
+    return t;
+  };
+  Vec acc;
+#pragma unroll
+  for (int k = 0; k < V; ++k) acc.x[k] = 0.0f;
+  if (in) {
     int r = rl;
     for (; r + 3 * 64 < rows; r += 4 * 64) {
-      const float4 a = p4[(int64_t)r * n4 + c4];
-      const float4 b = p4[(int64_t)(r + 64) * n4 + c4];
-      const float4 c = p4[(int64_t)(r + 128) * n4 + c4];
-      const float4 e = p4[(int64_t)(r + 192) * n4 + c4];
-      acc.x += a.x; acc.y += a.y; acc.z += a.z; acc.w += a.w;
-      acc.x += b.x; acc.y += b.y; acc.z += b.z; acc.w += b.w;
-      acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
-      acc.x += e.x; acc.y += e.y; acc.z += e.z; acc.w += e.w;
+      const Vec a = load(r), b = load(r + 64), c = load(r + 128), e = load(r + 192);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        acc.x[k] += a.x[k];
+        acc.x[k] += b.x[k];
+        acc.x[k] += c.x[k];
+        acc.x[k] += e.x[k];
+      }
     }
     for (; r < rows; r += 64) {
-      const float4 a = p4[(int64_t)r * n4 + c4];
-      acc.x += a.x; acc.y += a.y; acc.z += a.z; acc.w += a.w;
+      const Vec a = load(r);
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc.x[k] += a.x[k];
     }
   }
-  // Both halves of a swap end up with (low lanes' value) + (high lanes'), in
-  // that order, so the lanes that meet later hold identical bits.
-  auto pair = [](float x, bool across32) {
-    const uint32_t u = __float_as_uint(x);
-    const auto r = across32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
-                            : __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  };
-  acc = make_float4(pair(acc.x, true), pair(acc.y, true), pair(acc.z, true), pair(acc.w, true));
-  acc = make_float4(pair(acc.x, false), pair(acc.y, false), pair(acc.z, false), pair(acc.w, false));
-  const int wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < V; ++k) acc.x[k] = pair_sum<false>(pair_sum<true>(acc.x[k]));
   if (lane < 16) sh[wave][cl] = acc;
   __syncthreads();
-  if (wave == 0 && lane < 16 && c4 < n4) {
-    float4 t = sh[0][cl];
+  if (wave == 0 && lane < 16 && in) {
+    Vec t = sh[0][cl];
 #pragma unroll
-    for (int q = 1; q < 16; ++q) {
-      const float4 o = sh[q][cl];
-      t.x += o.x; t.y += o.y; t.z += o.z; t.w += o.w;
-    }
-    store_elem(dw, 4 * (int64_t)c4, t.x, wt);
-    store_elem(dw, 4 * (int64_t)c4 + 1, t.y, wt);
-    store_elem(dw, 4 * (int64_t)c4 + 2, t.z, wt);
-    store_elem(dw, 4 * (int64_t)c4 + 3, t.w, wt);
+    for (int q = 1; q < 16; ++q)
+#pragma unroll
+      for (int k = 0; k < V; ++k) t.x[k] += sh[q][cl].x[k];
+#pragma unroll
+    for (int k = 0; k < V; ++k) store_elem(dw, (int64_t)c0 + k, t.x[k], wt);
   }
 }
 
@@ -533,10 +525,10 @@ hipError_t launch_bwd_batched_generic(const BwdBatchedArgs& a, int grid, hipStre
 hipError_t launch_dw_reduce(const float* partial, int rows, int d, void* dw, int w_dtype,
                             hipStream_t s) {
   if (d % 4 == 0 && ((uintptr_t)partial & 15) == 0) {
-    hipLaunchKernelGGL(k_dw_reduce4, dim3((unsigned)((d / 4 + 15) / 16)), dim3(1024), 0, s, partial,
+    hipLaunchKernelGGL(k_dw_reduce<4>, dim3((unsigned)((d / 4 + 15) / 16)), dim3(1024), 0, s, partial,
                        rows, d, dw, w_dtype);
   } else {
-    hipLaunchKernelGGL(k_dw_reduce, dim3((unsigned)((d + 63) / 64)), dim3(1024), 0, s, partial,
+    hipLaunchKernelGGL(k_dw_reduce<1>, dim3((unsigned)((d + 15) / 16)), dim3(1024), 0, s, partial,
                        rows, d, dw, w_dtype);
   }
   return hipGetLastError();

@@ -2,14 +2,15 @@
 // them. Built per dtype (-DSY_TAG=BF16 -DSY_NAME=bf16, F16/f16, F32/f32) and per
 // part, so that the parts compile side by side: -DSY_PART=0 the forward and the
 // speed-of-light kernels, 1 the backward, 2 the batched kernels, 3 (16-bit
-// dtypes) the forward with a query of another dtype.
+// dtypes) the forward with a query of another dtype, 4 the kernels for rows that are
+// not whole 16-byte chunks at 16-byte boundaries.
 #include <algorithm>
 
 #include "sy_kernels.hpp"
 #include "sy_launch.hpp"
 
 #if !defined(SY_TAG) || !defined(SY_NAME) || !defined(SY_PART)
-#error "build with -DSY_TAG=<BF16|F16|F32> -DSY_NAME=<bf16|f16|f32> -DSY_PART=<0..3>"
+#error "build with -DSY_TAG=<BF16|F16|F32> -DSY_NAME=<bf16|f16|f32> -DSY_PART=<0..4>"
 #endif
 
 #define SY_CAT2(a, b) a##b
@@ -319,6 +320,67 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
   }
   SY_TILES(X)
 #undef X
+  return hipErrorInvalidConfiguration;
+}
+#endif
+
+#if SY_PART == 4
+hipError_t SY_FN(launch_fwd_unal_)(const sy_plan& p, const FwdArgs& a, hipStream_t s,
+                                  KernelRes* info) {
+  const float inv_d = 1.0f / (float)a.d;
+  if (a.prior_m != nullptr) return hipErrorInvalidConfiguration;
+#define XR(W_, V_, N_)                                                                       \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
+    const int64_t grid = cdiv(a.n_tok, kT);                                                  \
+    if (info) {                                                                              \
+      *info = resources_of(k_fwd<T, W_, V_, N_, true, true>, kB);                            \
+      info->grid = (int)grid;                                                                \
+      return hipSuccess;                                                                     \
+    }                                                                                        \
+    hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true, true>), dim3((unsigned)grid), dim3(kB), 0, \
+                       s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,        \
+                       a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);     \
+    return hipGetLastError();                                                                \
+  }
+#define X(W_, V_) XR(W_, V_, 4) XR(W_, V_, 9)
+  SY_UNAL_TILES(X)
+#undef X
+#undef XR
+  return hipErrorInvalidConfiguration;
+}
+
+hipError_t SY_FN(bwd_unal_resources_)(const sy_plan& p, KernelRes* out) {
+#define XR(W_, V_, N_)                                                                       \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    static const KernelRes r =                                                               \
+        resources_of(k_bwd<T, W_, V_, N_, true, kBwdListed, true>, BwdGeom<W_, V_>::kBlock); \
+    *out = r;                                                                                \
+    return hipSuccess;                                                                       \
+  }
+#define X(W_, V_) XR(W_, V_, 4) XR(W_, V_, 9) XR(W_, V_, 16)
+  SY_UNAL_TILES(X)
+#undef X
+#undef XR
+  return hipErrorInvalidConfiguration;
+}
+
+hipError_t SY_FN(launch_bwd_unal_)(const sy_plan& p, const BwdArgs& a, int grid, hipStream_t s) {
+  const float inv_d = 1.0f / (float)a.d;
+  const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * p.tokens_per_block);
+  if (a.stats == nullptr || a.gm != nullptr) return hipErrorInvalidConfiguration;
+#define XR(W_, V_, N_)                                                                       \
+  if (tile_is(p, W_, V_, N_)) {                                                              \
+    hipLaunchKernelGGL((k_bwd<T, W_, V_, N_, true, kBwdListed, true>), dim3(grid),           \
+                       dim3(BwdGeom<W_, V_>::kBlock), 0, s, a.v, a.w, a.w_dtype,             \
+                       (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, a.n_src,        \
+                       a.n_tok, a.d, a.eps, inv_d, n_iter);                                  \
+    return hipGetLastError();                                                                \
+  }
+#define X(W_, V_) XR(W_, V_, 4) XR(W_, V_, 9) XR(W_, V_, 16)
+  SY_UNAL_TILES(X)
+#undef X
+#undef XR
   return hipErrorInvalidConfiguration;
 }
 #endif

@@ -30,6 +30,10 @@ namespace sy {
 // the generic kernel.
 #define SY_BWD_TALL_TILES(X) \
   X(2, 1, 32) X(4, 1, 32) X(2, 2, 32) X(4, 2, 32) X(2, 1, 64) X(4, 1, 64)
+// Tiles (waves, chunks per lane) for rows that are not whole 16-byte chunks at 16-byte
+// boundaries: a row of E chunks takes the first tile with E <= 64 * waves * chunks, and
+// then fills all its slots but the last (the kernels mask only that one).
+#define SY_UNAL_TILES(X) X(1, 1) X(1, 2) X(2, 2) X(4, 2) X(8, 2)
 constexpr int kTallRows = 32;
 constexpr int kTallerRows = 64;
 
@@ -217,15 +221,21 @@ struct BwdBatchedArgs {
 int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_dtype, int aligned,
               sy_plan* out, int has_stats = 1, int matrix_ok = 1);
 
-// make_plan for a launch of the forward or the backward: as make_plan, except that
-// a query of another dtype than the sources (which sy_plan_for reports as generic)
-// runs the plan of the sources' dtype. The vector kernels hold such a query as fp32
-// values: 16-bit D=2048 N=9, 4096 tokens with an fp32 query, forward 230 -> 32 us,
-// backward 354 -> 57 us. The backward needs the forward's stats for it (the
-// recompute tiles keep the query packed in the sources' dtype), and 16-bit rows of
-// more than 1024 chunks stay generic (their eight-wave tile keeps it packed too).
+// make_plan for a launch of the forward or the backward: as make_plan, except for
+// two kinds of calls that sy_plan_for reports as generic.
+//  * A query of another dtype than the sources runs the plan of the sources' dtype.
+//    The vector kernels hold such a query as fp32 values: 16-bit D=2048 N=9, 4096
+//    tokens with an fp32 query, forward 230 -> 32 us, backward 354 -> 57 us. The
+//    backward needs the forward's stats for it (the recompute tiles keep the query
+//    packed in the sources' dtype), and 16-bit rows of more than 1024 chunks stay
+//    generic (their eight-wave tile keeps it packed too).
+//  * Rows that are not whole 16-byte chunks at 16-byte boundaries (odd widths,
+//    misaligned buffers) run the unaligned kernels (*unal = true): rows of 16 bytes to
+//    1024 chunks; the backward with stats, up to 16 sources and not for the (o, m, l)
+//    gradient. N=5 T=1023 D=777 fp16: forward 18.0 -> 6.4 us, backward 46.2 -> 12.0.
+// `variant` as in bwd_plan (backward only).
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
-                     sy_plan* out, int has_stats = 1);
+                     sy_plan* out, bool* unal, int has_stats = 1, int variant = 0);
 
 // Measurement overrides installed with sy_tuning_set (sy_capi.cpp). Returns
 // false (and leaves *out untouched) when none are installed, which is the
@@ -302,6 +312,16 @@ SY_DECLARE_VEC(f32)
 // launch_fwd_vec_* for 16-bit sources with a query of another dtype.
 hipError_t launch_fwd_wide_bf16(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info);
 hipError_t launch_fwd_wide_f16(const sy_plan& p, const FwdArgs& a, hipStream_t s, KernelRes* info);
+// The kernels for unaligned rows, with a query of any dtype.
+#define SY_DECLARE_UNAL(NAME)                                                                  \
+  hipError_t launch_fwd_unal_##NAME(const sy_plan& p, const FwdArgs& a, hipStream_t s,         \
+                                    KernelRes* info);                                          \
+  hipError_t bwd_unal_resources_##NAME(const sy_plan& p, KernelRes* out);                      \
+  hipError_t launch_bwd_unal_##NAME(const sy_plan& p, const BwdArgs& a, int grid, hipStream_t s);
+SY_DECLARE_UNAL(bf16)
+SY_DECLARE_UNAL(f16)
+SY_DECLARE_UNAL(f32)
+#undef SY_DECLARE_UNAL
 
 // Merge of two (o, m, l) partial results and its gradient (sy_merge.hip).
 // `vec` selects the 16-byte path (every row start 16-byte aligned).

@@ -253,15 +253,29 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
 }
 
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
-                     sy_plan* out, int has_stats) {
+                     sy_plan* out, bool* unal, int has_stats, int variant) {
+  *unal = false;
   const int rc = make_plan(op, n_src, 0, d, v_dtype, w_dtype, aligned, out, has_stats);
-  if (rc != SY_OK || out->family != SY_FAMILY_GENERIC || v_dtype == w_dtype || !aligned) return rc;
+  if (rc != SY_OK || out->family != SY_FAMILY_GENERIC) return rc;
   if (op != SY_OP_FWD && !(op == SY_OP_BWD && has_stats)) return rc;
-  sy_plan q;
-  if (make_plan(op, n_src, 0, d, v_dtype, v_dtype, aligned, &q, has_stats) != SY_OK) return rc;
-  const bool packed = op == SY_OP_BWD && q.elems_per_chunk == 8 && q.waves_per_token == 8 &&
-                      q.chunks_per_lane == 4;
-  if (!packed) *out = q;
+  const int ce = v_dtype == SY_F32 ? 4 : 8;
+  if (aligned && d % ce == 0) {
+    if (v_dtype == w_dtype) return rc;
+    sy_plan q;
+    if (make_plan(op, n_src, 0, d, v_dtype, v_dtype, aligned, &q, has_stats) != SY_OK) return rc;
+    const bool packed = op == SY_OP_BWD && q.elems_per_chunk == 8 && q.waves_per_token == 8 &&
+                        q.chunks_per_lane == 4;
+    if (!packed) *out = q;
+    return rc;
+  }
+  const int64_t e = (d + ce - 1) / ce;
+  if (d < ce || e > 1024 || (op == SY_OP_BWD && (n_src > 16 || variant == 2))) return rc;
+  const int w = e <= 128 ? 1 : e <= 256 ? 2 : e <= 512 ? 4 : 8;
+  const int vpl = e <= 64 ? 1 : 2;
+  // Forward over more than 9 rows: online-softmax chunks of four, as rule 3.
+  const int nr = op == SY_OP_BWD ? (n_src <= 4 ? 4 : n_src <= 9 ? 9 : 16) : (n_src <= 4 || n_src > 9 ? 4 : 9);
+  set(out, nr >= n_src ? SY_FAMILY_RESIDENT : SY_FAMILY_CHUNKED, w, vpl, nr, ce, op, n_src);
+  *unal = true;
   return rc;
 }
 

@@ -97,4 +97,4 @@ def test_the_launched_plan_of_a_mixed_query():
     assert _lib.plan(_lib.OP_FWD, 9, 2048, BF, w_dtype=F, n_tok=4096)["family_name"] == "resident"
     assert _lib.plan(_lib.OP_BWD, 9, 2048, BF, w_dtype=F, n_tok=4096)["family_name"] == "resident"
     assert _lib.plan(_lib.OP_BWD, 9, 16384, BF, w_dtype=F, n_tok=64)["family_name"] == "generic"
-    assert _lib.plan(_lib.OP_FWD, 9, 777, BF, w_dtype=F, n_tok=64)["family_name"] == "generic"
+    assert _lib.plan(_lib.OP_FWD, 9, 7, BF, w_dtype=F, n_tok=64)["family_name"] == "generic"
