@@ -917,6 +917,76 @@ int sy_merge_stats_bwd(const void* o1, const float* m1, const float* l1, const v
   return status(launch_merge_bwd(a, dtype, vec, (hipStream_t)stream));
 }
 
+int sy_rms_norm(const void* x, const void* w, void* out, float* rinv, int64_t n_tok, int64_t d,
+                int dtype, float eps, void* stream) {
+  if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
+  if (n_tok < 0 || n_tok > 0x3fffffff || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
+  if (n_tok == 0) return SY_OK;
+  if (!x || !w || !out) return SY_ERR_NULL;
+  if (!al16(x) || !al16(w) || !al16(out)) return SY_ERR_SHAPE;
+  const NormArgs a{x, w, nullptr, out, rinv, nullptr, 0, n_tok, (int)d, eps};
+  return status(launch_rms_norm(a, dtype, (hipStream_t)stream));
+}
+
+int64_t sy_rms_norm_bwd_bytes(int64_t n_tok, int64_t d) {
+  if (n_tok < 0 || d < 1 || d > 0x7fffffff / 16) return SY_ERR_SHAPE;
+  return n_tok == 0 ? 0 : norm_bwd_rows(n_tok) * d * (int64_t)sizeof(float);
+}
+
+int sy_rms_norm_bwd(const void* x, const void* w, const void* grad_out, const float* rinv, void* dx,
+                    void* dw, void* workspace, int64_t workspace_bytes, int64_t n_tok, int64_t d,
+                    int dtype, void* stream) {
+  if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
+  if (n_tok < 0 || n_tok > 0x3fffffff || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
+  if (!dw || (n_tok != 0 && (!x || !w || !grad_out || !rinv || !dx))) return SY_ERR_NULL;
+  if (!al16(x) || !al16(w) || !al16(grad_out) || !al16(dx) || !al16(workspace)) return SY_ERR_SHAPE;
+  const hipStream_t s = (hipStream_t)stream;
+  const int rows = n_tok == 0 ? 0 : norm_bwd_rows(n_tok);
+  if (rows > 0) {
+    if (workspace == nullptr || workspace_bytes < rows * d * (int64_t)sizeof(float)) return SY_ERR_WORKSPACE;
+    const NormArgs a{x,    w,     grad_out, dx, const_cast<float*>(rinv), (float*)workspace,
+                     rows, n_tok, (int)d,   0.0f};
+    const hipError_t e = launch_rms_norm(a, dtype, s);
+    if (e != hipSuccess) return (int)e;
+  }
+  return status(launch_dw_reduce((const float*)workspace, rows, (int)d, dw, dtype, s));
+}
+
+int sy_rope_qkv(void* qkv, void* q, void* k, void* v, const float* cosv, const float* sinv,
+                int64_t n_tok, int64_t seq, int64_t heads, int64_t hd, int dtype, int backward,
+                void* stream) {
+  if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
+  const int64_t ce = dtype == SY_F32 ? 4 : 8;
+  if (n_tok < 0 || seq < 1 || seq > 0x7fffffff || n_tok % seq != 0 || heads < 1 || heads > 0xffff ||
+      hd < 1 || hd > 0xffff || hd % (2 * ce) != 0)
+    return SY_ERR_SHAPE;
+  if (backward != 0 && backward != 1) return SY_ERR_OP;
+  if (n_tok == 0) return SY_OK;
+  if (!qkv || !q || !k || !v || !cosv || !sinv) return SY_ERR_NULL;
+  if (!al16(qkv) || !al16(q) || !al16(k) || !al16(v)) return SY_ERR_SHAPE;
+  const RopeArgs a{qkv, q, k, v, cosv, sinv, n_tok, (int)seq, (int)heads, (int)hd, backward == 1};
+  return status(launch_rope_qkv(a, dtype, (hipStream_t)stream));
+}
+
+int sy_swiglu(const void* gate_up, void* out, int64_t n_tok, int64_t f, int dtype, void* stream) {
+  if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
+  if (n_tok < 0 || f < 1 || f > 0x7fffffff / 16 || f % (dtype == SY_F32 ? 4 : 8) != 0) return SY_ERR_SHAPE;
+  if (n_tok == 0) return SY_OK;
+  if (!gate_up || !out) return SY_ERR_NULL;
+  if (!al16(gate_up) || !al16(out)) return SY_ERR_SHAPE;
+  return status(launch_swiglu(gate_up, nullptr, out, n_tok, (int)f, dtype, (hipStream_t)stream));
+}
+
+int sy_swiglu_bwd(const void* gate_up, const void* grad_out, void* dgate_up, int64_t n_tok, int64_t f,
+                  int dtype, void* stream) {
+  if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
+  if (n_tok < 0 || f < 1 || f > 0x7fffffff / 16 || f % (dtype == SY_F32 ? 4 : 8) != 0) return SY_ERR_SHAPE;
+  if (n_tok == 0) return SY_OK;
+  if (!gate_up || !grad_out || !dgate_up) return SY_ERR_NULL;
+  if (!al16(gate_up) || !al16(grad_out) || !al16(dgate_up)) return SY_ERR_SHAPE;
+  return status(launch_swiglu(gate_up, grad_out, dgate_up, n_tok, (int)f, dtype, (hipStream_t)stream));
+}
+
 int64_t sy_probe_grid(int64_t bytes) {
   // 256 threads x 4 chunks in flight per workgroup; up to 32768 workgroups
   // (the grid that reached the highest read bandwidth on MI355X).

@@ -361,6 +361,39 @@ struct MergeBwdArgs {
 hipError_t launch_merge(const MergeArgs& a, int dtype, bool vec, hipStream_t s);
 hipError_t launch_merge_bwd(const MergeBwdArgs& a, int dtype, bool vec, hipStream_t s);
 
+// The decoder's sublayer kernels (sy_decoder.hip).
+struct NormArgs {  // go == nullptr: forward (out, rinv or nullptr); else out is dx
+  const void* x;
+  const void* w;
+  const void* go;
+  void* out;
+  float* rinv;
+  float* partial;  // backward: [rows][d]
+  int rows;
+  int64_t n_tok;
+  int d;
+  float eps;
+};
+struct RopeArgs {
+  void* qkv;
+  void* q;
+  void* k;
+  void* v;
+  const float* cosv;  // [>= seq][hd / 2]
+  const float* sinv;
+  int64_t n_tok;
+  int seq;
+  int heads;
+  int hd;
+  bool backward;
+};
+bool norm_fits(int64_t d, int dtype);
+int norm_bwd_rows(int64_t n_tok);
+hipError_t launch_rms_norm(const NormArgs& a, int dtype, hipStream_t s);
+hipError_t launch_rope_qkv(const RopeArgs& a, int dtype, hipStream_t s);
+hipError_t launch_swiglu(const void* gu, const void* go, void* out, int64_t n_tok, int f, int dtype,
+                         hipStream_t s);
+
 // Generic kernels, the dw reduction and the probes (sy_generic.hip).
 hipError_t launch_fwd_generic(const FwdArgs& a, hipStream_t s);
 hipError_t launch_sol_generic(const FwdArgs& a, hipStream_t s);

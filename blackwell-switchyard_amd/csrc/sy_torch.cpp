@@ -328,6 +328,146 @@ std::optional<Tensor> block_attn_res_batched_train(const Tensor& v, const Tensor
   return batched_forward(dense(v), dense(q), eps);
 }
 
+// ------------------------------------------------------------ decoder sublayers
+
+bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+int64_t chunk(const Tensor& t) { return 16 / (int64_t)t.element_size(); }
+
+Tensor norm_forward(const Tensor& x, const Tensor& w, double eps, Tensor* rinv) {
+  const c10::DeviceGuard guard(x.device());
+  const int64_t d = w.size(0), tok = x.numel() / d;
+  Tensor out = at::empty(x.sizes(), x.options().requires_grad(false));
+  if (rinv != nullptr) *rinv = at::empty({tok}, f32_on(x));
+  check(sy_rms_norm(x.data_ptr(), w.data_ptr(), out.data_ptr(),
+                    rinv != nullptr ? rinv->data_ptr<float>() : nullptr, tok, d, code_of(x), (float)eps,
+                    stream_of(x)),
+        "sy_rms_norm");
+  return out;
+}
+
+struct RmsNorm : torch::autograd::Function<RmsNorm> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+    Tensor rinv;
+    Tensor out = norm_forward(x, w, eps, &rinv);
+    ctx->save_for_backward({x, w, rinv});
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1];
+    const c10::DeviceGuard guard(x.device());
+    const int64_t d = w.size(0), tok = x.numel() / d;
+    Tensor g = grad_like(grads[0], x);
+    if (!aligned16(g)) g = g.clone();
+    Tensor dx = at::empty(x.sizes(), x.options().requires_grad(false));
+    Tensor dw = at::empty({d}, w.options().requires_grad(false));
+    const int64_t bytes = sy_rms_norm_bwd_bytes(tok, d);
+    if (bytes < 0) check(bytes, "sy_rms_norm_bwd_bytes");
+    const Tensor ws = at::empty({std::max<int64_t>(1, bytes / 4)}, f32_on(x));
+    check(sy_rms_norm_bwd(x.data_ptr(), w.data_ptr(), g.data_ptr(), saved[2].data_ptr<float>(), dx.data_ptr(),
+                          dw.data_ptr(), ws.data_ptr(), ws.numel() * 4, tok, d, code_of(x), stream_of(x)),
+          "sy_rms_norm_bwd");
+    return {dx, dw, Tensor()};
+  }
+};
+
+std::optional<Tensor> rms_norm(const Tensor& x, const Tensor& w, double eps) {
+  if (!ordinary() || !plain(x) || !plain(w) || w.dim() != 1 || x.dim() < 1 || x.numel() == 0 ||
+      x.size(-1) != w.size(0) || x.scalar_type() != w.scalar_type() || x.device() != w.device() ||
+      !x.is_contiguous() || !w.is_contiguous() || !aligned16(x) || !aligned16(w) ||
+      w.size(0) % chunk(x) != 0 || w.size(0) / chunk(x) > 512)
+    return std::nullopt;
+  if (needs_grad(x, w)) return RmsNorm::apply(x, w, eps);
+  return norm_forward(x, w, eps, nullptr);
+}
+
+variable_list rope_forward(const Tensor& qkv, const Tensor& cosv, const Tensor& sinv) {
+  const c10::DeviceGuard guard(qkv.device());
+  const int64_t b = qkv.size(0), t = qkv.size(1), h = qkv.size(3), hd = qkv.size(4);
+  variable_list r;
+  for (int k = 0; k < 3; ++k) r.push_back(at::empty({b, h, t, hd}, qkv.options().requires_grad(false)));
+  check(sy_rope_qkv(qkv.data_ptr(), r[0].data_ptr(), r[1].data_ptr(), r[2].data_ptr(),
+                    cosv.data_ptr<float>(), sinv.data_ptr<float>(), b * t, t, h, hd, code_of(qkv), 0,
+                    stream_of(qkv)),
+        "sy_rope_qkv");
+  return r;
+}
+
+struct RopeQkv : torch::autograd::Function<RopeQkv> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cosv,
+                               const Tensor& sinv) {
+    ctx->save_for_backward({cosv, sinv});
+    return rope_forward(qkv, cosv, sinv);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    for (Tensor& g : grads) {
+      g = dense(g);
+      if (!aligned16(g)) g = g.clone();
+    }
+    const Tensor& q = grads[0];
+    const c10::DeviceGuard guard(q.device());
+    const int64_t b = q.size(0), h = q.size(1), t = q.size(2), hd = q.size(3);
+    Tensor dqkv = at::empty({b, t, 3, h, hd}, q.options().requires_grad(false));
+    check(sy_rope_qkv(dqkv.data_ptr(), q.data_ptr(), grads[1].data_ptr(), grads[2].data_ptr(),
+                      saved[0].data_ptr<float>(), saved[1].data_ptr<float>(), b * t, t, h, hd, code_of(q), 1,
+                      stream_of(q)),
+          "sy_rope_qkv");
+    return {dqkv, Tensor(), Tensor()};
+  }
+};
+
+// qkv [B, T, 3, H, hd], tables [>= T, ..., hd/2] -> (q, k, v), each [B, H, T, hd].
+std::optional<variable_list> rope_qkv(const Tensor& qkv, const Tensor& cosv, const Tensor& sinv) {
+  if (!ordinary() || !plain(qkv) || !plain(cosv) || !plain(sinv) || qkv.dim() != 5 || qkv.size(2) != 3 ||
+      qkv.numel() == 0 || !qkv.is_contiguous() || !aligned16(qkv) || qkv.size(4) % (2 * chunk(qkv)) != 0 ||
+      qkv.size(3) > 0xffff || qkv.size(4) > 0xffff)
+    return std::nullopt;
+  for (const Tensor* t : {&cosv, &sinv})
+    if (t->scalar_type() != at::kFloat || t->device() != qkv.device() || !t->is_contiguous() ||
+        t->requires_grad() || t->dim() < 2 || t->size(-1) != qkv.size(4) / 2 || t->size(0) < qkv.size(1) ||
+        t->numel() != t->size(0) * t->size(-1))
+      return std::nullopt;
+  if (at::GradMode::is_enabled() && qkv.requires_grad()) return RopeQkv::apply(qkv, cosv, sinv);
+  return rope_forward(qkv, cosv, sinv);
+}
+
+struct SwiGlu : torch::autograd::Function<SwiGlu> {
+  static Tensor run(const Tensor& gu) {
+    const c10::DeviceGuard guard(gu.device());
+    auto sizes = gu.sizes().vec();
+    const int64_t f = sizes.back() / 2;
+    sizes.back() = f;
+    Tensor out = at::empty(sizes, gu.options().requires_grad(false));
+    check(sy_swiglu(gu.data_ptr(), out.data_ptr(), out.numel() / f, f, code_of(gu), stream_of(gu)), "sy_swiglu");
+    return out;
+  }
+  static Tensor forward(AutogradContext* ctx, const Tensor& gu) {
+    ctx->save_for_backward({gu});
+    return run(gu);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor gu = ctx->get_saved_variables()[0];
+    const c10::DeviceGuard guard(gu.device());
+    Tensor g = grad_like(grads[0], gu);
+    if (!aligned16(g)) g = g.clone();
+    Tensor d = at::empty(gu.sizes(), gu.options().requires_grad(false));
+    const int64_t f = gu.size(-1) / 2;
+    check(sy_swiglu_bwd(gu.data_ptr(), g.data_ptr(), d.data_ptr(), g.numel() / f, f, code_of(gu),
+                        stream_of(gu)),
+          "sy_swiglu_bwd");
+    return {d};
+  }
+};
+
+std::optional<Tensor> swiglu(const Tensor& gu) {
+  if (!ordinary() || !plain(gu) || gu.dim() < 1 || gu.numel() == 0 || !gu.is_contiguous() || !aligned16(gu) ||
+      gu.size(-1) % (2 * chunk(gu)) != 0)
+    return std::nullopt;
+  if (at::GradMode::is_enabled() && gu.requires_grad()) return SwiGlu::apply(gu);
+  return SwiGlu::run(gu);
+}
+
 }  // namespace
 
 // The interpreter's lock is released during a call, as ctypes does.
@@ -338,4 +478,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("block_attn_res_two_phase", &block_attn_res_two_phase, free_lock);
   m.def("block_attn_res_batched", &block_attn_res_batched, free_lock);
   m.def("block_attn_res_batched_train", &block_attn_res_batched_train, free_lock);
+  m.def("rms_norm", &rms_norm, free_lock);
+  m.def("rope_qkv", &rope_qkv, free_lock);
+  m.def("swiglu", &swiglu, free_lock);
 }

@@ -104,6 +104,12 @@ SIGNATURES = {
     "sy_bwd_batched_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32]),
     "sy_bwd_batched": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
                               ctypes.c_float, _vp]),
+    "sy_rms_norm": (_i32, [_vp, _vp, _vp, _vp, _i64, _i64, _i32, ctypes.c_float, _vp]),
+    "sy_rms_norm_bwd_bytes": (_i64, [_i64, _i64]),
+    "sy_rms_norm_bwd": (_i32, [_vp] * 7 + [_i64, _i64, _i64, _i32, _vp]),
+    "sy_rope_qkv": (_i32, [_vp] * 6 + [_i64] * 4 + [_i32, _i32, _vp]),
+    "sy_swiglu": (_i32, [_vp, _vp, _i64, _i64, _i32, _vp]),
+    "sy_swiglu_bwd": (_i32, [_vp, _vp, _vp, _i64, _i64, _i32, _vp]),
     "sy_bw_probe": (_i32, [_i32, _vp, _vp, _i64, _vp]),
     "sy_probe_grid": (_i64, [_i64]),
     "sy_tuning_set": (_i32, [ctypes.POINTER(Tuning)]),

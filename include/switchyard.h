@@ -307,6 +307,34 @@ int sy_bwd_batched(const void* v, const void* queries, const void* grad_out, voi
                    int64_t n_tok, int64_t d, int64_t src_stride, int dtype, float eps,
                    void* stream);
 
+/* The decoder's sublayer work between its GEMMs and attention (the reference's
+ * decoder evaluates these operation by operation, src/switchyard/model.py:238-319).
+ * All tensors dense and 16-byte aligned, one dtype per call (cos, sin, rinv and
+ * partials fp32); SY_ERR_SHAPE for sizes outside the stated ones.
+ *
+ * RMSNorm: out = x r w, r = 1/sqrt(mean(x^2) + eps), over [n_tok][d]; d a multiple
+ * of a 16-byte chunk, at most 512 chunks. rinv [n_tok] (or NULL) receives r. The
+ * gradient takes that rinv and a workspace of sy_rms_norm_bwd_bytes bytes. */
+int sy_rms_norm(const void* x, const void* w, void* out, float* rinv, int64_t n_tok, int64_t d,
+                int dtype, float eps, void* stream);
+int64_t sy_rms_norm_bwd_bytes(int64_t n_tok, int64_t d);
+int sy_rms_norm_bwd(const void* x, const void* w, const void* grad_out, const float* rinv, void* dx,
+                    void* dw, void* workspace, int64_t workspace_bytes, int64_t n_tok, int64_t d,
+                    int dtype, void* stream);
+/* Rotary embedding and split of a fused projection: qkv [n_tok][3][heads][hd],
+ * n_tok a multiple of seq, to q, k, v [n_tok/seq][heads][seq][hd], where channel i
+ * of a q or k head's first half turns with channel i of its second half by
+ * cos/sin[t][i] ([>= seq][hd/2]); hd/2 a multiple of a 16-byte chunk. backward = 1
+ * is the transpose: from the gradients in q, k, v to qkv's. */
+int sy_rope_qkv(void* qkv, void* q, void* k, void* v, const float* cosv, const float* sinv,
+                int64_t n_tok, int64_t seq, int64_t heads, int64_t hd, int dtype, int backward,
+                void* stream);
+/* SwiGLU: out [n_tok][f] = silu(gate) * up over gate_up [n_tok][2 f], gate first;
+ * f a multiple of a 16-byte chunk. The gradient writes d gate_up [n_tok][2 f]. */
+int sy_swiglu(const void* gate_up, void* out, int64_t n_tok, int64_t f, int dtype, void* stream);
+int sy_swiglu_bwd(const void* gate_up, const void* grad_out, void* dgate_up, int64_t n_tok, int64_t f,
+                  int dtype, void* stream);
+
 /* Speed-of-light ceiling: out[t] = sum_n v_n[t] with the forward's geometry and
  * bytes but no softmax. Replaces speed_of_light (src/switchyard/triton_op.py:153-191). */
 int sy_sol(const void* v, void* out, int64_t n_src, int64_t n_tok, int64_t d,

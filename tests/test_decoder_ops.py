@@ -1,0 +1,127 @@
+"""The decoder's fused sublayer kernels (RMSNorm, rotary with the QKV split, SwiGLU)
+forward and backward against float64 torch, at rows of one chunk, partial lanes, the
+widest row, one token and several per wave; and what is left to the plain operations."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("needs a HIP device", allow_module_level=True)
+
+from oracle.reference import dtype_floor, rel_l2  # noqa: E402
+from switchyard import _lib  # noqa: E402
+from switchyard.model import ModelConfig, Rotary, Transformer  # noqa: E402
+
+DEV = "cuda"
+BF, HF, F = torch.bfloat16, torch.float16, torch.float32
+DTYPES = [BF, HF, F]
+
+
+def _rand(*shape, dtype, seed):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV)
+
+
+def _close(got, ref, dtype):
+    # one rounding of each output; fp32: sums of up to 4096 products
+    assert rel_l2(got, ref.cpu()) <= (2e-6 if dtype == F else 1.10 * dtype_floor(ref.cpu(), dtype))
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (5, 64), (3, 520), (2, 7, 1032), (2100, 512), (33, 2048), (9, 4096)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rms_norm(shape, dtype):
+    d = shape[-1] // 2 if dtype == F else shape[-1]
+    shape = (*shape[:-1], d)
+    x, w, g = _rand(*shape, dtype=dtype, seed=1), _rand(d, dtype=dtype, seed=2), _rand(*shape, dtype=dtype, seed=3)
+    xx, ww = x.clone().requires_grad_(), w.clone().requires_grad_()
+    out = _lib.native().rms_norm(xx, ww, 1e-6)
+    dx, dw = torch.autograd.grad(out, (xx, ww), g)
+    x6, w6 = x.double().requires_grad_(), w.double().requires_grad_()
+    ref = x6 * torch.rsqrt(x6.square().mean(-1, keepdim=True) + 1e-6) * w6
+    rdx, rdw = torch.autograd.grad(ref, (x6, w6), g.double())
+    for got, want in ((out.detach(), ref.detach()), (dx, rdx), (dw, rdw)):
+        assert got.dtype == dtype and got.shape == want.shape
+        _close(got, want, dtype)
+    with torch.no_grad():
+        assert torch.equal(_lib.native().rms_norm(x, w, 1e-6), out)
+
+
+@pytest.mark.parametrize("bthd", [(1, 1, 1, 16), (2, 33, 3, 64), (3, 7, 2, 48), (1, 300, 4, 128)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rope_qkv(bthd, dtype):
+    b, t, h, hd = bthd
+    rot = Rotary(hd, 512, 10000.0).to(DEV)
+    qkv = _rand(b, t, 3, h, hd, dtype=dtype, seed=4)
+    gs = [_rand(b, h, t, hd, dtype=dtype, seed=5 + k) for k in range(3)]
+    gs[1] = gs[1].transpose(1, 2).contiguous().transpose(1, 2)  # a strided gradient
+    xx = qkv.clone().requires_grad_()
+    out = _lib.native().rope_qkv(xx, rot.cos, rot.sin)
+    dq = torch.autograd.grad(out, xx, gs)[0]
+    x6 = qkv.double().requires_grad_()
+    cos, sin = rot.cos[:t].double(), rot.sin[:t].double()
+
+    def turn(x):
+        lo, hi = x.chunk(2, -1)
+        return torch.cat((lo * cos - hi * sin, lo * sin + hi * cos), -1)
+
+    q, k, v = x6.unbind(2)
+    ref = [y.transpose(1, 2) for y in (turn(q), turn(k), v)]
+    rdq = torch.autograd.grad(ref, x6, [g.double() for g in gs])[0]
+    for got, want in (*zip(out, ref), (dq, rdq)):
+        assert got.is_contiguous() and got.shape == want.shape
+        _close(got.detach(), want.detach(), dtype)
+
+
+@pytest.mark.parametrize("shape", [(1, 16), (3, 5, 2816), (700, 208)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_swiglu(shape, dtype):
+    x = _rand(*shape, dtype=dtype, seed=8) * 3
+    x[0, ..., 0] = 90.0  # saturated gates
+    x[0, ..., 1] = -90.0
+    g = _rand(*shape[:-1], shape[-1] // 2, dtype=dtype, seed=9)
+    xx = x.clone().requires_grad_()
+    out = _lib.native().swiglu(xx)
+    dx = torch.autograd.grad(out, xx, g)[0]
+    x6 = x.double().requires_grad_()
+    a, u = x6.chunk(2, -1)
+    ref = torch.nn.functional.silu(a) * u
+    _close(out.detach(), ref.detach(), dtype)
+    _close(dx, torch.autograd.grad(ref, x6, g.double())[0], dtype)
+
+
+def test_other_tensors_are_left_to_the_plain_operations():
+    m = _lib.native()
+    x, w = _rand(4, 64, dtype=BF, seed=1), _rand(64, dtype=BF, seed=2)
+    assert m.rms_norm(x, w.float(), 1e-6) is None and m.rms_norm(x.t(), w[:4], 1e-6) is None
+    assert m.rms_norm(x[:, :63], w[:63], 1e-6) is None and m.rms_norm(x.cpu(), w.cpu(), 1e-6) is None
+    assert m.swiglu(x[:, ::2]) is None and m.swiglu(x[:, :24].contiguous()) is None
+    rot = Rotary(16, 8, 1e4).to(DEV)
+    qkv = _rand(1, 9, 3, 2, 16, dtype=BF, seed=3)  # more positions than the tables hold
+    assert m.rope_qkv(qkv, rot.cos, rot.sin) is None
+    assert m.rope_qkv(qkv[:, :8], rot.cos.double(), rot.sin) is None
+
+
+@pytest.mark.parametrize("residual", ["standard", "switchyard"])
+def test_the_decoder_agrees_with_its_plain_operations(residual, monkeypatch):
+    """Loss and gradients of a small fp32 decoder with the kernels and without."""
+    cfg = ModelConfig(vocab_size=128, d_model=64, n_heads=2, d_ff=128, n_layers=2, n_blocks=2, max_seq_len=32,
+                      residual=residual)
+    torch.manual_seed(0)
+    model = Transformer(cfg).to(DEV)
+    if model.attn_res is not None:
+        for site in model.attn_res:
+            torch.nn.init.normal_(site.w, std=0.3)
+    idx = torch.randint(0, 128, (2, 32), generator=torch.Generator().manual_seed(1)).to(DEV)
+    got = []
+    for plain in (False, True):
+        if plain:
+            monkeypatch.setattr(_lib, "ordinary", lambda *t: False)
+        loss = model(idx, idx)[1]
+        got.append([loss.detach(), *torch.autograd.grad(loss, list(model.parameters()))])
+        with torch.no_grad():
+            got[-1].append(model(idx))
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=2e-4, atol=2e-5)  # fp32 sums in another order, two layers deep
