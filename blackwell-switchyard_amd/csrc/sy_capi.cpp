@@ -90,8 +90,8 @@ int bwd_grid(const sy_plan& p, bool unal, int64_t n_tok, int dtype, bool stats, 
 // operator gradient with stats only) becomes the generic kernel for every
 // other caller.
 int bwd_plan(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, int aligned,
-             bool stats, int variant, sy_plan* p, bool* unal) {
-  int rc = make_launch_plan(SY_OP_BWD, n_src, d, v_dtype, w_dtype, aligned, p, unal, stats, variant);
+             bool stats, int variant, sy_plan* p, bool* unal, bool gain = false) {
+  int rc = make_launch_plan(SY_OP_BWD, n_src, d, v_dtype, w_dtype, aligned, p, unal, stats, variant, gain);
   if (rc != SY_OK || *unal) return rc;
   apply_tile_rules(SY_OP_BWD, n_src, n_tok, d, p);
   if (p->family != SY_FAMILY_GENERIC && p->rows_per_tile > 16 && (!stats || variant != 0))
@@ -223,7 +223,7 @@ hipError_t fwd_vec(const sy_plan& p, bool unal, const FwdArgs& a, hipStream_t s,
     if (a.v_dtype == SY_F16) return launch_fwd_unal_f16(p, a, s, info);
     return launch_fwd_unal_f32(p, a, s, info);
   }
-  const bool wide = a.w_dtype != a.v_dtype;
+  const bool wide = a.w_dtype != a.v_dtype || a.gain != nullptr;
   if (a.v_dtype == SY_BF16)
     return wide ? launch_fwd_wide_bf16(p, a, s, info) : launch_fwd_vec_bf16(p, a, s, info);
   if (a.v_dtype == SY_F16)
@@ -356,17 +356,20 @@ bool vec_rows(bool rows_ok, int64_t d, int dtype) { return rows_ok && (d * esize
 // with m_out/l_out) over any row table. Sizes are already checked.
 int fwd_impl(const RowTable& v, bool v_ok, const void* w, void* out, float* stats, float* m_out,
              float* l_out, int normalize, int64_t n_src, int64_t n_tok, int64_t d, int v_dtype,
-             int w_dtype, float eps, hipStream_t s, int64_t stats_rows = 0) {
-  const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out);
+             int w_dtype, float eps, hipStream_t s, int64_t stats_rows = 0,
+             const void* gain = nullptr) {
+  const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out) && al16(gain);
   sy_plan p;
   bool unal = false;
-  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p, &unal);
+  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p, &unal, 1, 0,
+                                  gain != nullptr);
   if (rc != SY_OK) return rc;
   if (!unal) apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
   if (n_tok == 0) return SY_OK;
   FwdArgs a{v,      w,       out,     stats,   m_out, l_out, normalize, (int)n_src,
             n_tok,  (int)d,  v_dtype, w_dtype, eps};
   a.stats_rows = (int)stats_rows;
+  a.gain = gain;
   return status(p.family == SY_FAMILY_GENERIC ? launch_fwd_generic(a, s) : fwd_vec(p, unal, a, s));
 }
 
@@ -407,22 +410,31 @@ int merge_impl(RowTable t, bool ok, const void* w, const void* o1, const float* 
 int bwd_main_impl(const RowTable& v, bool v_ok, const void* w, const void* g, const float* stats,
                   const float* gm, const float* gl, const RowTable& dv, bool dv_ok, bool listed,
                   void* workspace, int64_t workspace_bytes, int64_t n_src, int64_t n_tok,
-                  int64_t d, int v_dtype, int w_dtype, float eps, hipStream_t s, int* rows_out) {
+                  int64_t d, int v_dtype, int w_dtype, float eps, hipStream_t s, int* rows_out,
+                  const void* gain = nullptr) {
   *rows_out = 0;
   if (n_tok == 0) return SY_OK;
-  const bool aligned = vec_rows(v_ok && dv_ok, d, v_dtype) && al16(w) && al16(g) && al16(workspace);
+  const bool aligned = vec_rows(v_ok && dv_ok, d, v_dtype) && al16(w) && al16(g) && al16(workspace) &&
+                       al16(gain);
   sy_plan p;
   const int variant = listed ? 1 : (gm != nullptr ? 2 : 0);
   bool unal = false;
-  int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, stats != nullptr, variant, &p, &unal);
+  int rc = bwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, stats != nullptr, variant, &p, &unal,
+                    gain != nullptr);
   if (rc != SY_OK) return rc;
   int grid = 0;
   rc = bwd_grid_for(p, unal, n_src, n_tok, d, v_dtype, w_dtype, stats != nullptr, variant, &grid);
   if (rc != SY_OK) return rc;
+  // A two-factor query may take the generic kernel where the workspace was sized for
+  // the packed one's tile: persistent over tokens, it runs on what there is.
+  if (gain != nullptr && p.family == SY_FAMILY_GENERIC && workspace != nullptr)
+    grid = (int)std::min<int64_t>(grid, workspace_bytes / (d * (int64_t)sizeof(float)));
+  if (grid < 1) return SY_ERR_WORKSPACE;
   if (workspace == nullptr || workspace_bytes < (int64_t)grid * d * (int64_t)sizeof(float))
     return SY_ERR_WORKSPACE;
-  const BwdArgs a{v,      w,       g,     stats,  gm,      gl,      dv,  (float*)workspace, listed,
-                  (int)n_src, n_tok, (int)d, v_dtype, w_dtype, eps};
+  BwdArgs a{v,      w,       g,     stats,  gm,      gl,      dv,  (float*)workspace, listed,
+            (int)n_src, n_tok, (int)d, v_dtype, w_dtype, eps};
+  a.gain = gain;
   const hipError_t e =
       p.family == SY_FAMILY_GENERIC ? launch_bwd_generic(a, grid, s) : bwd_vec(p, unal, a, grid, s);
   if (e != hipSuccess) return (int)e;
@@ -435,12 +447,13 @@ int bwd_main_impl(const RowTable& v, bool v_ok, const void* w, const void* g, co
 int bwd_impl(const RowTable& v, bool v_ok, const void* w, const void* g, const float* stats,
              const float* gm, const float* gl, const RowTable& dv, bool dv_ok, bool listed, void* dw,
              void* workspace, int64_t workspace_bytes, int64_t n_src, int64_t n_tok, int64_t d,
-             int v_dtype, int w_dtype, float eps, hipStream_t s) {
+             int v_dtype, int w_dtype, float eps, hipStream_t s, const void* gain = nullptr,
+             void* dgain = nullptr) {
   int rows = 0;
   const int rc = bwd_main_impl(v, v_ok, w, g, stats, gm, gl, dv, dv_ok, listed, workspace,
-                               workspace_bytes, n_src, n_tok, d, v_dtype, w_dtype, eps, s, &rows);
+                               workspace_bytes, n_src, n_tok, d, v_dtype, w_dtype, eps, s, &rows, gain);
   if (rc != SY_OK) return rc;
-  return status(launch_dw_reduce((const float*)workspace, rows, (int)d, dw, w_dtype, s));
+  return status(launch_dw_reduce((const float*)workspace, rows, (int)d, dw, w_dtype, s, w, gain, dgain));
 }
 
 // Batched forward: the resident kernel, else one forward launch per query
@@ -523,6 +536,18 @@ int sy_fwd(const void* v, const void* w, void* out, float* stats, int64_t n_src,
   const RowTable t = stacked(v, n_src, src_stride, v_dtype, &ok);
   return fwd_impl(t, ok, w, out, stats, nullptr, nullptr, 1, n_src, n_tok, d, v_dtype, w_dtype, eps,
                   (hipStream_t)stream);
+}
+
+int sy_fwd_gain(const void* v, const void* w, const void* gain, void* out, float* stats,
+                int64_t n_src, int64_t n_tok, int64_t d, int64_t src_stride, int v_dtype, int w_dtype,
+                float eps, void* stream) {
+  if (n_tok != 0 && (v == nullptr || w == nullptr || gain == nullptr || out == nullptr)) return SY_ERR_NULL;
+  const int rc = check_common(n_src, n_tok, d, src_stride, v_dtype, w_dtype);
+  if (rc != SY_OK) return rc;
+  bool ok = false;
+  const RowTable t = stacked(v, n_src, src_stride, v_dtype, &ok);
+  return fwd_impl(t, ok, w, out, stats, nullptr, nullptr, 1, n_src, n_tok, d, v_dtype, w_dtype, eps,
+                  (hipStream_t)stream, 0, gain);
 }
 
 int sy_fwd_table(const void* const* v_rows, const void* w, void* out, float* stats, int64_t n_src,
@@ -631,6 +656,21 @@ int sy_bwd(const void* v, const void* w, const void* grad_out, const float* stat
   const RowTable td = stacked(dv, n_src, n_tok * d, v_dtype, &dok);
   return bwd_impl(tv, vok, w, grad_out, stats, nullptr, nullptr, td, dok, false, dw, workspace,
                   workspace_bytes, n_src, n_tok, d, v_dtype, w_dtype, eps, (hipStream_t)stream);
+}
+
+int sy_bwd_gain(const void* v, const void* w, const void* gain, const void* grad_out,
+                const float* stats, void* dv, void* dw, void* dgain, void* workspace,
+                int64_t workspace_bytes, int64_t n_src, int64_t n_tok, int64_t d, int64_t src_stride,
+                int v_dtype, int w_dtype, float eps, void* stream) {
+  if (dw == nullptr || dgain == nullptr || w == nullptr || gain == nullptr) return SY_ERR_NULL;
+  if (n_tok != 0 && (v == nullptr || grad_out == nullptr || dv == nullptr)) return SY_ERR_NULL;
+  const int rc = check_common(n_src, n_tok, d, src_stride, v_dtype, w_dtype);
+  if (rc != SY_OK) return rc;
+  bool vok = false, dok = false;
+  const RowTable tv = stacked(v, n_src, src_stride, v_dtype, &vok);
+  const RowTable td = stacked(dv, n_src, n_tok * d, v_dtype, &dok);
+  return bwd_impl(tv, vok, w, grad_out, stats, nullptr, nullptr, td, dok, false, dw, workspace,
+                  workspace_bytes, n_src, n_tok, d, v_dtype, w_dtype, eps, (hipStream_t)stream, gain, dgain);
 }
 
 int sy_bwd_static(const void* v, const void* w, const void* grad_out, const float* stats, void* dv,

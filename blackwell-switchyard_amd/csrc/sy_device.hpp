@@ -233,6 +233,21 @@ __device__ __forceinline__ void ld_query(__amdgpu_buffer_rsrc_t r, uint32_t c, i
   }
 }
 
+// The same of w * gain, a query given as its two factors (gain may be nullptr): the
+// product is formed in fp32 and never rounded.
+template <int CE>
+__device__ __forceinline__ void ld_query_gain(const void* w, const void* gain, int wt, uint32_t d,
+                                              uint32_t c, float* f) {
+  const uint32_t bytes = d * (wt == F32::code ? 4u : 2u);
+  ld_query<CE>(make_rsrc(w, bytes), c, wt, f);
+  if (gain != nullptr) {
+    float g[CE];
+    ld_query<CE>(make_rsrc(gain, bytes), c, wt, g);
+#pragma unroll
+    for (int e = 0; e < CE; ++e) f[e] *= g[e];
+  }
+}
+
 // acc + sum_e x[e] * f[e] with an fp32 query chunk.
 template <class T>
 __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, float acc) {
@@ -242,18 +257,18 @@ __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, floa
 }
 
 // A lane's query chunks: packed in the sources' dtype, or (WIDE) as fp32 values
-// when the query has another dtype. fp32 sources hold any query as fp32 chunks.
+// when the query has another dtype or a gain. fp32 sources hold any query as fp32
+// chunks.
 template <class T, bool WIDE, int VPL>
 struct Query {
   i32x4_t q[VPL];
-  __device__ __forceinline__ void load(const void* w, int wt, uint32_t d, uint32_t lane_off,
-                                       uint32_t step) {
+  __device__ __forceinline__ void load(const void* w, const void* gain, int wt, uint32_t d,
+                                       uint32_t lane_off, uint32_t step) {
     if constexpr (T::code == F32::code) {
-      const auto r = make_rsrc(w, d * (wt == F32::code ? 4u : 2u));
 #pragma unroll
       for (int j = 0; j < VPL; ++j) {
         float f[4];
-        ld_query<4>(r, (lane_off + j * step) / 16u, wt, f);
+        ld_query_gain<4>(w, gain, wt, d, (lane_off + j * step) / 16u, f);
         q[j] = pack<T>(f);
       }
     } else {
@@ -269,11 +284,10 @@ struct Query {
 template <class T, int VPL>
 struct Query<T, true, VPL> {
   float f[VPL][T::ce];
-  __device__ __forceinline__ void load(const void* w, int wt, uint32_t d, uint32_t lane_off,
-                                       uint32_t step) {
-    const auto r = make_rsrc(w, d * (wt == F32::code ? 4u : 2u));
+  __device__ __forceinline__ void load(const void* w, const void* gain, int wt, uint32_t d,
+                                       uint32_t lane_off, uint32_t step) {
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) ld_query<T::ce>(r, (lane_off + j * step) / 16u, wt, f[j]);
+    for (int j = 0; j < VPL; ++j) ld_query_gain<T::ce>(w, gain, wt, d, (lane_off + j * step) / 16u, f[j]);
   }
   __device__ __forceinline__ float dot(const i32x4_t& x, int j, float acc) const {
     return dot_wide<T>(x, f[j], acc);
@@ -349,11 +363,9 @@ __device__ __forceinline__ i32x4_t own_part(const i32x4_t& x, int j, const i32x4
   else return x;
 }
 
-// The query elements of the chunk at `off` of such a row (no alignment assumed).
+// The query elements from element c on (no alignment assumed).
 template <int CE>
-__device__ __forceinline__ void ld_query_any(const void* w, uint32_t off, uint32_t row_bytes, int wt,
-                                             float* f) {
-  const int64_t c = tail_off(off, row_bytes) / (16 / CE);
+__device__ __forceinline__ void ld_query_at(const void* w, int64_t c, int wt, float* f) {
   if (wt == F32::code) {
 #pragma unroll
     for (int q = 0; q < CE / 4; ++q) {
@@ -377,6 +389,20 @@ __device__ __forceinline__ void ld_query_any(const void* w, uint32_t off, uint32
   for (int e = 0; e < CE; ++e)
     f[e] = wt == BF16::code ? __uint_as_float(x[e] << 16)
                             : (float)__builtin_bit_cast(_Float16, (uint16_t)x[e]);
+}
+
+// Those of the chunk at `off` of an unaligned row, times the gain's.
+template <int CE>
+__device__ __forceinline__ void ld_query_any(const void* w, const void* gain, uint32_t off,
+                                             uint32_t row_bytes, int wt, float* f) {
+  const int64_t c = tail_off(off, row_bytes) / (16 / CE);
+  ld_query_at<CE>(w, c, wt, f);
+  if (gain != nullptr) {
+    float g[CE];
+    ld_query_at<CE>(gain, c, wt, g);
+#pragma unroll
+    for (int e = 0; e < CE; ++e) f[e] *= g[e];
+  }
 }
 
 // ---------------------------------------------------------------- reductions

@@ -52,8 +52,8 @@ __device__ float block_max(float x, float* scr) {
 // Pass 1 for one token: per-row (sum of squares, query dot[, grad dot]) for
 // every row, written to ss[], qd[] and gd[] in LDS. Rows go in groups of 8 so
 // a thread carries 16-24 partial sums.
-__device__ void row_scalars(const RowTable& v, const void* w, const void* g, int n_src,
-                            int64_t tok, int d, int vt, int wt, float* ss, float* qd, float* gd,
+__device__ void row_scalars(const RowTable& v, const void* w, const void* gain, const void* g,
+                            int n_src, int64_t tok, int d, int vt, int wt, float* ss, float* qd, float* gd,
                             float* scr) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -64,7 +64,7 @@ __device__ void row_scalars(const RowTable& v, const void* w, const void* g, int
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = b[r] = c[r] = 0.0f;
     for (int k = tid; k < d; k += kBlock) {
-      const float wk = load_elem(w, k, wt);
+      const float wk = load_elem(w, k, wt) * (gain ? load_elem(gain, k, wt) : 1.0f);
       const float gk = g ? load_elem(g, tok * d + k, vt) : 0.0f;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -108,7 +108,8 @@ __device__ void row_scalars(const RowTable& v, const void* w, const void* g, int
 
 // LDS layout (floats): [0, n) lg, [n, 2n) ss/r, [2n, 3n) gd, then 257 scratch.
 __global__ void __launch_bounds__(kBlock)
-k_fwd_generic(const RowTable v, const void* __restrict__ w, void* __restrict__ out,
+k_fwd_generic(const RowTable v, const void* __restrict__ w, const void* __restrict__ gain,
+              void* __restrict__ out,
               float* __restrict__ stats, float* __restrict__ m_out, float* __restrict__ l_out,
               int normalize, int n_src, int stat_rows, int64_t n_tok, int d, int vt, int wt,
               float eps, float inv_d) {
@@ -118,7 +119,7 @@ k_fwd_generic(const RowTable v, const void* __restrict__ w, void* __restrict__ o
   float* scr = sh + 2 * n_src;
   const int tid = threadIdx.x;
   const int64_t tok = blockIdx.x;
-  row_scalars(v, w, nullptr, n_src, tok, d, vt, wt, ss, lg, nullptr, scr);
+  row_scalars(v, w, gain, nullptr, n_src, tok, d, vt, wt, ss, lg, nullptr, scr);
 
   float m = -INFINITY;
   for (int n = tid; n < n_src; n += kBlock) {
@@ -167,7 +168,8 @@ k_sol_generic(const RowTable v, void* __restrict__ out, int n_src, int64_t n_tok
 // own fp32 row partial[b][:] (no other workgroup touches it). gm != nullptr
 // selects the gradient of the unnormalised (o, m, l) triple, as in k_bwd.
 __global__ void __launch_bounds__(kBlock)
-k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restrict__ g,
+k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restrict__ gain,
+              const void* __restrict__ g,
               const float* __restrict__ gm, const float* __restrict__ gl, const RowTable dv,
               float* __restrict__ partial, int n_src, int64_t n_tok, int d, int vt, int wt,
               float eps, float inv_d) {
@@ -181,7 +183,7 @@ k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restri
   for (int k = tid; k < d; k += kBlock) prow[k] = 0.0f;
 
   for (int64_t tok = blockIdx.x; tok < n_tok; tok += gridDim.x) {
-    row_scalars(v, w, g, n_src, tok, d, vt, wt, da, al, gc, scr);
+    row_scalars(v, w, gain, g, n_src, tok, d, vt, wt, da, al, gc, scr);
     float m = -INFINITY;
     for (int n = tid; n < n_src; n += kBlock) {
       const float r = rsqrtf(fmaf(da[n], inv_d, eps));
@@ -235,7 +237,7 @@ k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restri
     __syncthreads();
     for (int k = tid; k < d; k += kBlock) {
       const float gk = load_elem(g, tok * d + k, vt);
-      const float wk = load_elem(w, k, wt);
+      const float wk = load_elem(w, k, wt) * (gain ? load_elem(gain, k, wt) : 1.0f);
       float dwk = 0.0f;
       for (int n = 0; n < n_src; ++n) {
         const float x = load_elem(row_of<const char>(v, n), tok * d + k, vt);
@@ -279,7 +281,7 @@ k_bwd_batched_generic(const RowTable v, const void* __restrict__ q, const void* 
     for (int s = 0; s < n_q; ++s) {
       const char* qs = static_cast<const char*>(q) + (int64_t)s * d * es;
       const char* gs = static_cast<const char*>(g) + (int64_t)s * n_tok * d * es;
-      row_scalars(v, qs, gs, nn, tok, d, vt, vt, ss, qd, gd, scr);
+      row_scalars(v, qs, nullptr, gs, nn, tok, d, vt, vt, ss, qd, gd, scr);
       float m = -INFINITY;
       for (int n = tid; n < nn; n += kBlock) {
         const float r = rsqrtf(fmaf(ss[n], inv_d, eps));
@@ -354,7 +356,8 @@ __device__ __forceinline__ float pair_sum(float x) {
 // 777: 2.5-3.1 us, against 19.2 with 16 row lanes and one load in flight).
 template <int V>
 __global__ void __launch_bounds__(1024)
-k_dw_reduce(const float* __restrict__ partial, int rows, int d, void* __restrict__ dw, int wt) {
+k_dw_reduce(const float* __restrict__ partial, int rows, int d, void* __restrict__ dw, int wt,
+            const void* __restrict__ w, const void* __restrict__ gain, void* __restrict__ dgain) {
   struct Vec { float x[V]; };
   typedef float vec_t __attribute__((ext_vector_type(4)));
   __shared__ Vec sh[16][16];
@@ -408,7 +411,14 @@ k_dw_reduce(const float* __restrict__ partial, int rows, int d, void* __restrict
 #pragma unroll
       for (int k = 0; k < V; ++k) t.x[k] += sh[q][cl].x[k];
 #pragma unroll
-    for (int k = 0; k < V; ++k) store_elem(dw, (int64_t)c0 + k, t.x[k], wt);
+    for (int k = 0; k < V; ++k) {
+      const int64_t c = (int64_t)c0 + k;
+      if (dgain != nullptr) {
+        store_elem(dgain, c, t.x[k] * load_elem(w, c, wt), wt);
+        t.x[k] *= load_elem(gain, c, wt);
+      }
+      store_elem(dw, c, t.x[k], wt);
+    }
   }
 }
 
@@ -495,7 +505,7 @@ k_probe_mix(const char* __restrict__ src, char* __restrict__ dst, int64_t out_by
 
 hipError_t launch_fwd_generic(const FwdArgs& a, hipStream_t s) {
   const size_t lds = (size_t)(2 * a.n_src + 257) * sizeof(float);
-  hipLaunchKernelGGL(k_fwd_generic, dim3((unsigned)a.n_tok), dim3(kBlock), lds, s, a.v, a.w, a.out,
+  hipLaunchKernelGGL(k_fwd_generic, dim3((unsigned)a.n_tok), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.out,
                      a.stats, a.m_out, a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d,
                      a.v_dtype, a.w_dtype, a.eps, 1.0f / (float)a.d);
   return hipGetLastError();
@@ -509,7 +519,7 @@ hipError_t launch_sol_generic(const FwdArgs& a, hipStream_t s) {
 
 hipError_t launch_bwd_generic(const BwdArgs& a, int grid, hipStream_t s) {
   const size_t lds = (size_t)(3 * a.n_src + 257) * sizeof(float);
-  hipLaunchKernelGGL(k_bwd_generic, dim3(grid), dim3(kBlock), lds, s, a.v, a.w, a.g, a.gm, a.gl,
+  hipLaunchKernelGGL(k_bwd_generic, dim3(grid), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.g, a.gm, a.gl,
                      a.dv, a.partial, a.n_src, a.n_tok, a.d, a.v_dtype, a.w_dtype, a.eps,
                      1.0f / (float)a.d);
   return hipGetLastError();
@@ -523,13 +533,13 @@ hipError_t launch_bwd_batched_generic(const BwdBatchedArgs& a, int grid, hipStre
 }
 
 hipError_t launch_dw_reduce(const float* partial, int rows, int d, void* dw, int w_dtype,
-                            hipStream_t s) {
+                            hipStream_t s, const void* w, const void* gain, void* dgain) {
   if (d % 4 == 0 && ((uintptr_t)partial & 15) == 0) {
     hipLaunchKernelGGL(k_dw_reduce<4>, dim3((unsigned)((d / 4 + 15) / 16)), dim3(1024), 0, s, partial,
-                       rows, d, dw, w_dtype);
+                       rows, d, dw, w_dtype, w, gain, dgain);
   } else {
     hipLaunchKernelGGL(k_dw_reduce<1>, dim3((unsigned)((d + 15) / 16)), dim3(1024), 0, s, partial,
-                       rows, d, dw, w_dtype);
+                       rows, d, dw, w_dtype, w, gain, dgain);
   }
   return hipGetLastError();
 }

@@ -78,14 +78,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
           static const KernelRes km = resources_of(k_fwd_res<T, W_, V_, N_, true, true>, kB); \
           if (n_iter <= 2 && km.blocks_per_cu >= kr.blocks_per_cu) {                         \
             hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true, true>), dim3(grid), dim3(kB), \
-                               0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,      \
+                               0, s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, \
                                a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, \
                                n_iter, a.prior_m, a.prior_l);                                \
             return hipGetLastError();                                                        \
           }                                                                                  \
         }                                                                                    \
         hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, true>), dim3(grid), dim3(kB), 0, s, a.v, \
-                           a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,            \
+                           a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,    \
                            a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                            a.prior_m, a.prior_l);                                            \
         return hipGetLastError();                                                            \
@@ -95,14 +95,14 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
         static const KernelRes kf = resources_of(k_fwd_res<T, W_, V_, N_, false, true>, kB); \
         if (n_iter <= 2 && kf.blocks_per_cu >= kr.blocks_per_cu) {                           \
           hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, true>), dim3(grid), dim3(kB), 0, \
-                             s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,  \
+                             s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, \
                              a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                              nullptr, nullptr);                                              \
           return hipGetLastError();                                                          \
         }                                                                                    \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_>), dim3(grid), dim3(kB), 0, s, a.v,        \
-                         a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
+                         a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
                          a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, nullptr, nullptr); \
     } else {                                                                                 \
       if (a.prior_m != nullptr) return hipErrorInvalidConfiguration;                         \
@@ -113,7 +113,7 @@ hipError_t SY_FN(launch_fwd_vec_)(const sy_plan& p, const FwdArgs& a, hipStream_
         return hipSuccess;                                                                   \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd<T, W_, V_, N_>), dim3((unsigned)grid), dim3(kB), 0, s, a.v,  \
-                         a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
+                         a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, a.normalize, \
                          a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);                \
     }                                                                                        \
     return hipGetLastError();                                                                \
@@ -207,7 +207,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
   if (tile_is(p, W_, V_, N_)) {                                                              \
     if (a.stats == nullptr || a.listed || a.gm != nullptr) return hipErrorInvalidConfiguration; \
     hipLaunchKernelGGL((k_bwd_tall<T, W_, V_, N_>), dim3(grid), dim3(TallGeom<W_, V_, N_>::kBlock), 0, \
-                       s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.dv, a.partial,     \
+                       s, a.v, a.w, a.gain, a.w_dtype, (const St*)a.g, a.stats, a.dv, a.partial, \
                        a.n_src, a.n_tok, a.d, inv_d, n_iter);                                \
     return hipGetLastError();                                                                \
   }
@@ -215,7 +215,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
 #undef X
 #define SY_BWD_LAUNCH(W_, V_, N_, ST_, LI_)                                                  \
   hipLaunchKernelGGL((k_bwd<T, W_, V_, N_, ST_, LI_>), dim3(grid), dim3(BwdGeom<W_, V_>::kBlock), 0, \
-                     s, a.v, a.w, a.w_dtype, (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, \
+                     s, a.v, a.w, a.gain, a.w_dtype, (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, \
                      a.n_src, a.n_tok, a.d, a.eps, inv_d, n_iter)
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
@@ -302,7 +302,7 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
       }                                                                                      \
       const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * kT);                             \
       hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, true>), dim3(grid),         \
-                         dim3(kB), 0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out,  \
+                         dim3(kB), 0, s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, \
                          a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                          nullptr, nullptr);                                                  \
     } else {                                                                                 \
@@ -313,7 +313,7 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
         return hipSuccess;                                                                   \
       }                                                                                      \
       hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true>), dim3((unsigned)grid), dim3(kB),       \
-                         0, s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,   \
+                         0, s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, \
                          a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);   \
     }                                                                                        \
     return hipGetLastError();                                                                \
@@ -339,7 +339,7 @@ hipError_t SY_FN(launch_fwd_unal_)(const sy_plan& p, const FwdArgs& a, hipStream
       return hipSuccess;                                                                     \
     }                                                                                        \
     hipLaunchKernelGGL((k_fwd<T, W_, V_, N_, true, true>), dim3((unsigned)grid), dim3(kB), 0, \
-                       s, a.v, a.w, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out,        \
+                       s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, a.l_out, \
                        a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d);     \
     return hipGetLastError();                                                                \
   }
@@ -372,7 +372,7 @@ hipError_t SY_FN(launch_bwd_unal_)(const sy_plan& p, const BwdArgs& a, int grid,
 #define XR(W_, V_, N_)                                                                       \
   if (tile_is(p, W_, V_, N_)) {                                                              \
     hipLaunchKernelGGL((k_bwd<T, W_, V_, N_, true, kBwdListed, true>), dim3(grid),           \
-                       dim3(BwdGeom<W_, V_>::kBlock), 0, s, a.v, a.w, a.w_dtype,             \
+                       dim3(BwdGeom<W_, V_>::kBlock), 0, s, a.v, a.w, a.gain, a.w_dtype,     \
                        (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, a.n_src,        \
                        a.n_tok, a.d, a.eps, inv_d, n_iter);                                  \
     return hipGetLastError();                                                                \

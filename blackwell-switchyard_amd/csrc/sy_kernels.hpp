@@ -141,7 +141,8 @@ __device__ __forceinline__ void row_sums_transposed(const float (&tv)[P], float 
 // N=9 T=4096 D=2047 bf16 45.5 against 238 (3.7 TB/s: a misaligned chunk spans two lines).
 template <class T, int W, int VPL, int NR, bool WIDE = false, bool UNAL = false>
 __global__ void __launch_bounds__(FwdGeom<W>::kBlock)
-k_fwd(const RowTable v, const void* __restrict__ w, int wt,
+k_fwd(const RowTable v, const void* __restrict__ w,
+      const void* __restrict__ gain, int wt,
       typename T::storage* __restrict__ out, float* __restrict__ stats, float* __restrict__ m_out,
       float* __restrict__ l_out, int normalize, int n_src, int stat_rows, int64_t n_tok, int d,
       float eps, float inv_d) {
@@ -170,10 +171,10 @@ k_fwd(const RowTable v, const void* __restrict__ w, int wt,
   if constexpr (UNAL) {
     static_assert(WIDE, "unaligned rows hold the query as fp32 values");
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, lane_off + j * kStep, row_bytes, wt, wq.f[j]);
+    for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, gain, lane_off + j * kStep, row_bytes, wt, wq.f[j]);
     own = tail_mask(lane_off + (VPL - 1) * kStep, row_bytes);
   } else {
-    wq.load(w, wt, (uint32_t)d, lane_off, kStep);
+    wq.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
   }
 
   float m_run = -INFINITY, l_run = 0.0f;
@@ -525,7 +526,8 @@ k_batched(const RowTable v, const typename T::storage* __restrict__ q,
 // held to 256, two waves a SIMD like the packed query's (239).
 template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false, bool WIDE = false>
 __global__ void __launch_bounds__(FwdGeom<W>::kBlock, WIDE && VPL == 4 && NR == 9 ? 2 : 1)
-k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
+k_fwd_res(const RowTable v, const void* __restrict__ w,
+      const void* __restrict__ gain, int wt,
           typename T::storage* __restrict__ out, float* __restrict__ stats,
           float* __restrict__ m_out, float* __restrict__ l_out, int normalize, int n_src,
           int stat_rows, int64_t n_tok, int d, float eps, float inv_d, int n_iter,
@@ -558,7 +560,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w, int wt,
   const float* pstat_src = (lane & 1) ? pl : pm;
 
   Query<T, WIDE, VPL> wq;
-  wq.load(w, wt, (uint32_t)d, lane_off, kStep);
+  wq.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
   i32x4_t x[NR][VPL];
   float pstat = 0.0f;
   {
@@ -880,7 +882,8 @@ enum BwdVariant { kBwdStacked = 0, kBwdListed = 1, kBwdStatsGrad = 2 };
 
 template <class T, int W, int VPL, int NR, bool STATS, int VAR, bool UNAL = false>
 __global__ void __launch_bounds__((BwdGeom<W, VPL, NR>::kBlock))
-k_bwd(const RowTable v, const void* __restrict__ w, int wt,
+k_bwd(const RowTable v, const void* __restrict__ w,
+      const void* __restrict__ gain, int wt,
       const typename T::storage* __restrict__ g, const float* __restrict__ stats,
       const float* __restrict__ gm, const float* __restrict__ gl, const RowTable dv,
       float* __restrict__ partial, int n_src, int64_t n_tok, int d, float eps, float inv_d,
@@ -942,12 +945,12 @@ k_bwd(const RowTable v, const void* __restrict__ w, int wt,
   if constexpr (UNAL) {
     static_assert(STATS && !kLean, "unaligned rows: with the forward's stats");
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, lane_off + j * kStep, row_bytes, wt, wf[j]);
+    for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, gain, lane_off + j * kStep, row_bytes, wt, wf[j]);
     own = tail_mask(lane_off + (VPL - 1) * kStep, row_bytes);
   } else if constexpr (STATS && !kLean) {
-    const auto wr = make_rsrc(w, (uint32_t)d * (wt == F32::code ? 4u : 2u));
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) ld_query<CE>(wr, (lane_off + j * kStep) / 16u, wt, wf[j]);
+    for (int j = 0; j < VPL; ++j)
+      ld_query_gain<CE>(w, gain, wt, (uint32_t)d, (lane_off + j * kStep) / 16u, wf[j]);
   } else {
     const auto wr = make_rsrc(w, row_bytes);
 #pragma unroll
@@ -1260,7 +1263,8 @@ struct TallGeom {
 
 template <class T, int W, int VPL, int NR>
 __global__ void __launch_bounds__((TallGeom<W, VPL, NR>::kBlock))
-k_bwd_tall(const RowTable v, const void* __restrict__ w, int wt,
+k_bwd_tall(const RowTable v, const void* __restrict__ w,
+      const void* __restrict__ gain, int wt,
            const typename T::storage* __restrict__ g, const float* __restrict__ stats,
            const RowTable dv, float* __restrict__ partial, int n_src, int64_t n_tok, int d,
            float inv_d, int n_iter) {
@@ -1291,9 +1295,9 @@ k_bwd_tall(const RowTable v, const void* __restrict__ w, int wt,
 
   float wf[VPL][CE];
   {
-    const auto wr = make_rsrc(w, (uint32_t)d * (wt == F32::code ? 4u : 2u));
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) ld_query<CE>(wr, (lane_off + j * kStep) / 16u, wt, wf[j]);
+    for (int j = 0; j < VPL; ++j)
+      ld_query_gain<CE>(w, gain, wt, (uint32_t)d, (lane_off + j * kStep) / 16u, wf[j]);
   }
   float dwa[VPL][CE];
 #pragma unroll

@@ -164,6 +164,7 @@ struct FwdArgs {
   // Rows between the two planes of `stats`, when the launch fills one group's rows
   // of a wider array (0: n_src, an array of its own).
   int stats_rows = 0;
+  const void* gain = nullptr;  // [d] in w's dtype: the query is w * gain
   int stat_rows() const { return stats_rows > 0 ? stats_rows : n_src; }
 };
 
@@ -183,6 +184,7 @@ struct BwdArgs {
   int v_dtype;
   int w_dtype;
   float eps;
+  const void* gain = nullptr;  // as in FwdArgs
 };
 
 struct BatchedArgs {
@@ -233,9 +235,10 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
 //    misaligned buffers) run the unaligned kernels (*unal = true): rows of 16 bytes to
 //    1024 chunks; the backward with stats, up to 16 sources and not for the (o, m, l)
 //    gradient. N=5 T=1023 D=777 fp16: forward 18.0 -> 6.4 us, backward 46.2 -> 12.0.
+// A query given as two factors (`gain`) is held as fp32 values too, whatever its dtype.
 // `variant` as in bwd_plan (backward only).
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
-                     sy_plan* out, bool* unal, int has_stats = 1, int variant = 0);
+                     sy_plan* out, bool* unal, int has_stats = 1, int variant = 0, bool gain = false);
 
 // Measurement overrides installed with sy_tuning_set (sy_capi.cpp). Returns
 // false (and leaves *out untouched) when none are installed, which is the
@@ -399,8 +402,11 @@ hipError_t launch_fwd_generic(const FwdArgs& a, hipStream_t s);
 hipError_t launch_sol_generic(const FwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_generic(const BwdArgs& a, int grid, hipStream_t s);
 hipError_t launch_bwd_batched_generic(const BwdBatchedArgs& a, int grid, hipStream_t s);
+// With `dgain` the column sums are the gradient of w * gain: dw = sum * gain,
+// dgain = sum * w.
 hipError_t launch_dw_reduce(const float* partial, int rows, int d, void* dw, int w_dtype,
-                            hipStream_t s);
+                            hipStream_t s, const void* w = nullptr, const void* gain = nullptr,
+                            void* dgain = nullptr);
 hipError_t launch_probe(int kind, const void* src, void* dst, int64_t bytes, int grid,
                         hipStream_t s);
 

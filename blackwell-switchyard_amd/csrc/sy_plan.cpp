@@ -253,8 +253,9 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
 }
 
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
-                     sy_plan* out, bool* unal, int has_stats, int variant) {
+                     sy_plan* out, bool* unal, int has_stats, int variant, bool gain) {
   *unal = false;
+  if (gain) w_dtype = v_dtype == SY_F32 ? SY_BF16 : SY_F32;  // plans as another dtype does
   const int rc = make_plan(op, n_src, 0, d, v_dtype, w_dtype, aligned, out, has_stats);
   if (rc != SY_OK || out->family != SY_FAMILY_GENERIC) return rc;
   if (op != SY_OP_FWD && !(op == SY_OP_BWD && has_stats)) return rc;

@@ -151,6 +151,59 @@ std::optional<Tensor> block_attn_res(const Tensor& v, const Tensor& w, double ep
   return operator_forward(dense(v), dense(w), s, eps, nullptr);
 }
 
+// ------------------------------------------- the module: a query and its gain
+
+Tensor gain_forward(const Tensor& v, const Tensor& w, const Tensor& g, double eps, Tensor* stats) {
+  const c10::DeviceGuard guard(v.device());
+  const int64_t n = v.size(0), b = v.size(1), t = v.size(2), d = v.size(3), tok = b * t;
+  Tensor out = at::empty({b, t, d}, v.options().requires_grad(false));
+  if (stats != nullptr) *stats = at::empty({2, n, tok}, f32_on(v));
+  check(sy_fwd_gain(v.data_ptr(), w.data_ptr(), g.data_ptr(), out.data_ptr(),
+                    stats != nullptr ? stats->data_ptr<float>() : nullptr, n, tok, d, tok * d, code_of(v),
+                    code_of(w), (float)eps, stream_of(v)),
+        "sy_fwd_gain");
+  return out;
+}
+
+struct BlockAttnResGain : torch::autograd::Function<BlockAttnResGain> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& v_in, const Tensor& w_in, const Tensor& g_in,
+                        double eps) {
+    const Tensor v = dense(v_in), w = dense(w_in), g = dense(g_in);
+    Tensor stats;
+    Tensor out = gain_forward(v, w, g, eps, &stats);
+    ctx->save_for_backward({v, w, g, stats});
+    ctx->saved_data["eps"] = eps;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &v = saved[0], &w = saved[1];
+    const c10::DeviceGuard guard(v.device());
+    const int64_t n = v.size(0), d = v.size(3), tok = v.size(1) * v.size(2);
+    const int vt = code_of(v), wt = code_of(w);
+    const Tensor go = grad_like(grads[0], v);
+    Tensor dv = at::empty(v.sizes(), v.options().requires_grad(false));
+    Tensor dw = at::empty({d}, w.options().requires_grad(false));
+    Tensor dg = at::empty({d}, w.options().requires_grad(false));
+    const Tensor ws = bwd_workspace(v, n, tok, d, vt, wt);
+    check(sy_bwd_gain(v.data_ptr(), w.data_ptr(), saved[2].data_ptr(), go.data_ptr(),
+                      saved[3].data_ptr<float>(), dv.data_ptr(), dw.data_ptr(), dg.data_ptr(), ws.data_ptr(),
+                      ws.numel() * 4, n, tok, d, tok * d, vt, wt, (float)ctx->saved_data["eps"].toDouble(),
+                      stream_of(v)),
+          "sy_bwd_gain");
+    return {dv, dw, dg, Tensor()};
+  }
+};
+
+std::optional<Tensor> block_attn_res_gain(const Tensor& v, const Tensor& w, const Tensor& g, double eps) {
+  if (!sizes_of(v, w, 1).ok || !plain(g) || g.sizes() != w.sizes() || g.scalar_type() != w.scalar_type() ||
+      g.device() != w.device())
+    return std::nullopt;
+  if (needs_grad(v, w) || (at::GradMode::is_enabled() && g.requires_grad()))
+    return BlockAttnResGain::apply(v, w, g, eps);
+  return gain_forward(dense(v), dense(w), dense(g), eps, nullptr);
+}
+
 // --------------------------------------------------- sources as separate tensors
 
 struct BlockAttnResSources : torch::autograd::Function<BlockAttnResSources> {
@@ -474,6 +527,7 @@ std::optional<Tensor> swiglu(const Tensor& gu) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   const auto free_lock = py::call_guard<py::gil_scoped_release>();
   m.def("block_attn_res", &block_attn_res, free_lock);
+  m.def("block_attn_res_gain", &block_attn_res_gain, free_lock);
   m.def("block_attn_res_sources", &block_attn_res_sources, free_lock);
   m.def("block_attn_res_two_phase", &block_attn_res_two_phase, free_lock);
   m.def("block_attn_res_batched", &block_attn_res_batched, free_lock);

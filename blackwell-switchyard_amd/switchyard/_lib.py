@@ -83,6 +83,8 @@ SIGNATURES = {
     "sy_dw_reduce": (_i32, [_vp, _i64, _i64, _vp, _i32, _vp]),
     "sy_fwd_batched": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, ctypes.c_float, _vp]),
     "sy_sol": (_i32, [_vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp]),
+    "sy_fwd_gain": (_i32, [_vp] * 5 + [_i64] * 4 + [_i32, _i32, ctypes.c_float, _vp]),
+    "sy_bwd_gain": (_i32, [_vp] * 9 + [_i64] * 5 + [_i32, _i32, ctypes.c_float, _vp]),
     "sy_fwd_table": (_i32, [_vpp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, ctypes.c_float, _vp]),
     "sy_bwd_static": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32,
                              ctypes.c_float, _vp]),

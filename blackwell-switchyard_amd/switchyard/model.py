@@ -449,6 +449,16 @@ def _hip_stacked(v: Tensor, q: Tensor, eps: float) -> Tensor:
     return block_attn_res_hip(v, q, eps)
 
 
+def _hip_module(v: Tensor, site: BlockAttnRes, eps: float) -> Tensor:
+    """The operator at ``site`` with no backward to come; the kernel multiplies the
+    query by the gain."""
+    if site.g is not None and _lib.ordinary(v):
+        out = _lib.native().block_attn_res_gain(v, site.w, site.g, float(eps))
+        if out is not None:
+            return out
+    return _hip_stacked(v, site.effective_query(), eps)
+
+
 def _hip_table(sources: list[Tensor], q: Tensor, eps: float) -> Tensor:
     from .table_op import MAX_SOURCES, block_attn_res_sources
 
@@ -553,12 +563,15 @@ class Transformer(nn.Module):
 
     def _site(self, i: int, stream: _Stream, collect_alphas: bool) -> Tensor:
         cfg = self.cfg
-        q = self.attn_res[i].effective_query()
         sources = stream.sources()
         n = len(sources)
+        hip = cfg.residual == "switchyard"
+        if hip and stream.buf is not None and not torch.is_grad_enabled() and not collect_alphas:
+            with self._region("attnres_op"):
+                return _hip_module(stream.buf.slots[:n], self.attn_res[i], cfg.norm_eps)
+        q = self.attn_res[i].effective_query()
         if collect_alphas:
             self.last_alphas.append(_mean_alpha(sources, q, cfg.norm_eps))
-        hip = cfg.residual == "switchyard"
         if cfg.sources == "stack":
             with self._region("attnres_stage"):
                 v = torch.stack(sources)
@@ -568,8 +581,6 @@ class Transformer(nn.Module):
             with self._region("attnres_op"):
                 return _hip_table(sources, q, cfg.norm_eps)
         with self._region("attnres_op"):
-            if hip and not torch.is_grad_enabled():
-                return _hip_stacked(stream.buf.slots[:n], q, cfg.norm_eps)
             if hip:
                 return _SlotSiteHIP.apply(q, stream, n, cfg.norm_eps, *sources)
             with stream.saving():

@@ -137,6 +137,18 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
 int sy_fwd(const void* v, const void* w, void* out, float* stats, int64_t n_src, int64_t n_tok,
            int64_t d, int64_t src_stride, int v_dtype, int w_dtype, float eps, void* stream);
 
+/* sy_fwd and sy_bwd with the query given as two factors of one dtype, w * gain
+ * (a module's pseudo-query and its RMSNorm gain, src/switchyard/triton_op.py:597-609,
+ * which forms the product first): the kernels multiply in fp32, and the dw reduction
+ * writes both factors' gradients. stats, workspace and strides as in sy_fwd / sy_bwd. */
+int sy_fwd_gain(const void* v, const void* w, const void* gain, void* out, float* stats,
+                int64_t n_src, int64_t n_tok, int64_t d, int64_t src_stride, int v_dtype, int w_dtype,
+                float eps, void* stream);
+int sy_bwd_gain(const void* v, const void* w, const void* gain, const void* grad_out,
+                const float* stats, void* dv, void* dw, void* dgain, void* workspace,
+                int64_t workspace_bytes, int64_t n_src, int64_t n_tok, int64_t d, int64_t src_stride,
+                int v_dtype, int w_dtype, float eps, void* stream);
+
 /* sy_fwd with the sources given as a host array of n_src <= SY_MAX_TABLE_ROWS
  * device pointers, v_rows[n] -> [n_tok][D]. The reference takes only a stacked
  * tensor and names a per-source pointer table (fla's API) as the better design

@@ -1,0 +1,55 @@
+"""The module's query as two factors, multiplied in the kernels: outputs and the
+gradients of both factors on every family a two-factor query takes, against the
+float64 oracle of the product."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():  # pragma: no cover
+    pytest.skip("needs a HIP device", allow_module_level=True)
+
+from oracle.reference import block_attn_res_oracle, dtype_floor, oracle_grads, rel_l2  # noqa: E402
+from switchyard.triton_op import BlockAttnResTriton  # noqa: E402
+
+DEV = "cuda"
+BF, HF, F = torch.bfloat16, torch.float16, torch.float32
+
+# (N, T, D): resident, chunked and tall tiles, the eight-wave row (element-wise
+# backward), unaligned rows, and rows under 16 bytes (element-wise both ways)
+SHAPES = [(9, 1100, 2048), (4, 3, 64), (16, 40, 1024), (32, 24, 2048), (3, 8, 16384), (5, 70, 777), (4, 20, 7)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("dtypes", [(BF, BF), (BF, F), (HF, HF), (F, F)])
+@pytest.mark.parametrize("wants", ["all", "w"])
+def test_module_with_a_gain(shape, dtypes, wants):
+    vdt, wdt = dtypes
+    n, t, d = shape
+    print(f"gain {shape} {dtypes}", flush=True)
+    g = torch.Generator().manual_seed(d)
+    v = torch.randn(n, 1, t, d, generator=g).to(vdt)
+    w = (torch.randn(d, generator=g) * d**-0.5).to(wdt)
+    gain = (1 + 0.3 * torch.randn(d, generator=g)).to(wdt)
+    go = torch.randn(1, t, d, generator=g).to(vdt)
+    mod = BlockAttnResTriton(d).to(DEV).to(wdt)
+    with torch.no_grad():
+        mod.w.copy_(w)
+        mod.g.copy_(gain)
+    vv = v.to(DEV).requires_grad_(wants == "all")
+    mod.g.requires_grad_(wants == "all")
+    out = mod(vv)
+    leaves = [x for x in (vv, mod.w, mod.g) if x.requires_grad]
+    grads = torch.autograd.grad(out, leaves, go.to(DEV))
+    q = w.double() * gain.double()
+    rdv, rdq = oracle_grads(v.double(), q, go.double())
+    ref = {id(vv): (rdv, vdt), id(mod.w): (rdq * gain.double(), wdt), id(mod.g): (rdq * w.double(), wdt)}
+    for got, (want, dt) in ((out.detach(), (block_attn_res_oracle(v.double(), q), vdt)),
+                            *((x, ref[id(leaf)]) for x, leaf in zip(grads, leaves))):
+        assert got.dtype == dt
+        assert rel_l2(got, want) <= (1e-5 if dt == F else 1.10 * dtype_floor(want, dt))
+    with torch.no_grad():
+        assert torch.equal(mod(vv), out)
