@@ -199,6 +199,27 @@ template <> __device__ __forceinline__ float dot<F32>(const i32x4_t& a, const i3
   return acc;
 }
 
+// The same with the chunk summed from zero before it joins acc, fp32 in two halves: a
+// lane's chunks would else be one long chain. Rows of any start and queries of another
+// dtype use it; their error against float64 is then that of a block a row, whose threads
+// sum a few elements each (gradients: fp32 N=5 T=300 D=777 8.9e-7 -> 6.0e-7, the block
+// 6.4e-7; bf16 rows, fp32 query with a gain, N=9 T=300 D=2048 2.2e-6 -> 1.7e-6, 1.6e-6).
+template <class T> __device__ __forceinline__ float dot_short(const i32x4_t& a, const i32x4_t& b, float acc) {
+  if constexpr (T::code == F32::code) {
+    const float lo = fmaf(__int_as_float(a[1]), __int_as_float(b[1]), __int_as_float(a[0]) * __int_as_float(b[0]));
+    const float hi = fmaf(__int_as_float(a[3]), __int_as_float(b[3]), __int_as_float(a[2]) * __int_as_float(b[2]));
+    return acc + (lo + hi);
+  } else {
+    return acc + dot<T>(a, b, 0.0f);
+  }
+}
+
+template <class T, bool SHORT>
+__device__ __forceinline__ float row_dot(const i32x4_t& a, const i32x4_t& b, float acc) {
+  if constexpr (SHORT) return dot_short<T>(a, b, acc);
+  else return dot<T>(a, b, acc);
+}
+
 // The CE elements of chunk c of a query row of dtype wt (0 fp32, 1 fp16, 2 bf16,
 // uniform over the launch) as fp32. r covers the row, so elements past its end
 // read 0. A query may have another dtype than the sources (fp32 parameters with
@@ -252,7 +273,11 @@ __device__ __forceinline__ void ld_query_gain(const void* w, const void* gain, i
 template <class T>
 __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, float acc) {
 #pragma unroll
-  for (int e = 0; e < T::ce; ++e) acc = fmaf(elem<T>(x, e), f[e], acc);
+  for (int e = 0; e < T::ce; e += 4) {
+    const float lo = fmaf(elem<T>(x, e + 1), f[e + 1], elem<T>(x, e) * f[e]);
+    const float hi = fmaf(elem<T>(x, e + 3), f[e + 3], elem<T>(x, e + 2) * f[e + 2]);
+    acc += lo + hi;
+  }
   return acc;
 }
 
@@ -280,6 +305,9 @@ struct Query {
   __device__ __forceinline__ float dot(const i32x4_t& x, int j, float acc) const {
     return sy::dot<T>(x, q[j], acc);
   }
+  __device__ __forceinline__ float dot_short(const i32x4_t& x, int j, float acc) const {
+    return sy::dot_short<T>(x, q[j], acc);
+  }
 };
 template <class T, int VPL>
 struct Query<T, true, VPL> {
@@ -290,6 +318,9 @@ struct Query<T, true, VPL> {
     for (int j = 0; j < VPL; ++j) ld_query_gain<T::ce>(w, gain, wt, d, (lane_off + j * step) / 16u, f[j]);
   }
   __device__ __forceinline__ float dot(const i32x4_t& x, int j, float acc) const {
+    return dot_wide<T>(x, f[j], acc);
+  }
+  __device__ __forceinline__ float dot_short(const i32x4_t& x, int j, float acc) const {
     return dot_wide<T>(x, f[j], acc);
   }
 };

@@ -211,8 +211,8 @@ k_fwd(const RowTable v, const void* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             const i32x4_t xo = own_part<UNAL, VPL>(x[n][j], j, own);
-            ss = dot<T>(xo, xo, ss);
-            dt = wq.dot(xo, j, dt);
+            ss = row_dot<T, UNAL || WIDE>(xo, xo, ss);
+            dt = UNAL ? wq.dot_short(xo, j, dt) : wq.dot(xo, j, dt);
             reconvert<WIDE>(x[n][j]);
           }
           tv[n] = ss;
@@ -228,8 +228,8 @@ k_fwd(const RowTable v, const void* __restrict__ w,
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
             const i32x4_t xo = own_part<UNAL, VPL>(x[n][j], j, own);
-            ss = dot<T>(xo, xo, ss);
-            dt = wq.dot(xo, j, dt);
+            ss = row_dot<T, UNAL || WIDE>(xo, xo, ss);
+            dt = UNAL ? wq.dot_short(xo, j, dt) : wq.dot(xo, j, dt);
             reconvert<WIDE>(x[n][j]);
           }
           part[n] = wave_sum(ss);
@@ -611,7 +611,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
               float ss = 0.0f, dt = 0.0f;
 #pragma unroll
               for (int j = 0; j < VPL; ++j) {
-                ss = dot<T>(x[n][j], x[n][j], ss);
+                ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
                 dt = wq.dot(x[n][j], j, dt);
                 reconvert<WIDE>(x[n][j]);
             reconvert<WIDE>(x[n][j]);
@@ -684,7 +684,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
           float ss = 0.0f, dt = 0.0f;
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
-            ss = dot<T>(x[n][j], x[n][j], ss);
+            ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
             dt = wq.dot(x[n][j], j, dt);
             reconvert<WIDE>(x[n][j]);
           }
@@ -700,7 +700,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
           float ss = 0.0f, dt = 0.0f;
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
-            ss = dot<T>(x[n][j], x[n][j], ss);
+            ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
             dt = wq.dot(x[n][j], j, dt);
             reconvert<WIDE>(x[n][j]);
           }
@@ -1030,14 +1030,14 @@ k_bwd(const RowTable v, const void* __restrict__ w,
         if (live_row(n)) {
           float gg = 0.0f;
 #pragma unroll
-          for (int j = 0; j < VPL; ++j) gg = dot<T>(own_part<UNAL, VPL>(x[n][j], j, own), gq[j], gg);
+          for (int j = 0; j < VPL; ++j) gg = row_dot<T, UNAL>(own_part<UNAL, VPL>(x[n][j], j, own), gq[j], gg);
           tv[n] = gg;
           if constexpr (!STATS) {
             float dt = 0.0f, ss = 0.0f;
 #pragma unroll
             for (int j = 0; j < VPL; ++j) {
-              dt = dot<T>(x[n][j], wq[j], dt);
-              ss = dot<T>(x[n][j], x[n][j], ss);
+              dt = row_dot<T, UNAL>(x[n][j], wq[j], dt);
+              ss = row_dot<T, UNAL>(x[n][j], x[n][j], ss);
             }
             tv[NR + n] = dt;
             tv[2 * NR + n] = ss;
@@ -1051,14 +1051,14 @@ k_bwd(const RowTable v, const void* __restrict__ w,
         if (live_row(n)) {
           float gg = 0.0f;
 #pragma unroll
-          for (int j = 0; j < VPL; ++j) gg = dot<T>(own_part<UNAL, VPL>(x[n][j], j, own), gq[j], gg);
+          for (int j = 0; j < VPL; ++j) gg = row_dot<T, UNAL>(own_part<UNAL, VPL>(x[n][j], j, own), gq[j], gg);
           part[n] = wave_sum(gg);
           if constexpr (!STATS) {
             float dt = 0.0f, ss = 0.0f;
 #pragma unroll
             for (int j = 0; j < VPL; ++j) {
-              dt = dot<T>(x[n][j], wq[j], dt);
-              ss = dot<T>(x[n][j], x[n][j], ss);
+              dt = row_dot<T, UNAL>(x[n][j], wq[j], dt);
+              ss = row_dot<T, UNAL>(x[n][j], x[n][j], ss);
             }
             part[NR + n] = wave_sum(dt);
             part[2 * NR + n] = wave_sum(ss);
