@@ -1,4 +1,7 @@
-// Batched backward in two passes: any row of 16-byte chunks, 16-bit or fp32, up to
+// The batched operator for rows and counts that the matrix-core kernels of
+// sy_matrix.hip do not take.
+//
+// Backward in two passes: any row of 16-byte chunks, 16-bit or fp32, up to
 // 16 sources and 16 queries (the gradient's algebra is at k_bwd_batched_mx in
 // sy_matrix.hip, whose single pass needs g, the queries and the sources of a token
 // in one CU's LDS and serves 16-bit D <= 2048 with S <= 8).
@@ -18,6 +21,7 @@
 // Reference: the batched forward is src/switchyard/triton_op.py:378-501; it has no
 // backward (the single-query derivation is at :205-214).
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "sy_launch.hpp"
@@ -471,6 +475,179 @@ k_bb_apply(const RowTable v, const typename T::storage* __restrict__ q,
   }
 }
 
+// ------------------------------------------------------------------ forward
+//
+// S <= 16 queries, N <= NR sources, rows of any start and of at least one chunk. A
+// token is a workgroup's (W = 4: each wave a quarter of the columns) or a wave's
+// (W = 1). First the logits, straight from memory on MFMA as in k_bb_coef (queries as
+// B), summed over the waves through LDS; every wave then forms the softmax and keeps
+// the token's weights [n][s] as A operands, one value a lane, and in a second walk over
+// the token's rows -- now in L2 -- out_s = sum_n P_sn v_n on v_mfma_f32_4x4x1 as in
+// k_bb_apply: whole chunks in and out, exact fp32 weights. Memory-bound: v is read
+// from HBM once (the register tile computes S dots and S sums a row on the VALU).
+// bf16 T=4096: N=9 S=8 D=1280 74 -> 62 us, D=2560 144 -> 108; N=12 S=8 D=1280 159 (a
+// launch a query) -> 64; N=9 S=8 T=1023 D=777 195 -> 17.5. Its two walks do not
+// overlap within a wave, which leaves it at 1.5-1.8x the bytes' time.
+template <class T, int NR, int SG, int W>
+__global__ void __launch_bounds__(64 * kCoefWaves)
+k_batched_any(const RowTable v, const typename T::storage* __restrict__ q,
+              typename T::storage* __restrict__ out, float* __restrict__ m_out,
+              float* __restrict__ l_out, int normalize, int n_src, int n_q, int64_t n_tok, int d,
+              float eps, float inv_d) {
+  using S = typename T::storage;
+  constexpr int CE = T::ce;
+  constexpr int NG = (NR + 3) / 4, kS = 4 * SG;
+  constexpr int kCols = 4 * CE;  // columns of a logit step
+  constexpr int kU = 4;
+  constexpr int kTpb = kCoefWaves / W;
+  constexpr int kVgprs = (4 * NG * kS + 63) / 64;
+  constexpr int kEpd = CE / 4;
+  __shared__ __align__(16) float xl[W > 1 ? W : 1][64][4];
+  __shared__ __align__(16) float xs[kTpb][W][16];
+  __shared__ __align__(16) float tab[kCoefWaves][64 * kVgprs];
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int slot = wave / W, w = wave % W;
+  const int qi = lane & 15, grp = lane >> 4;
+  const uint32_t row_bytes = (uint32_t)d * sizeof(S);
+  using any_t = std::conditional_t<sizeof(S) == 4, i32x4_f32_t, i32x4_any_t>;
+  const int64_t hop = (int64_t)gridDim.x * kTpb;
+  for (int64_t tok = (int64_t)blockIdx.x * kTpb + slot; tok < n_tok; tok += hop) {
+    // 1. Logit and sum-of-squares partials over this wave's columns.
+    const S* pa = row_of<const S>(v, min(qi, n_src - 1)) + tok * d + grp * CE;
+    const S* pb = q + (int64_t)min(qi, n_q - 1) * d + grp * CE;
+    const int full = d / kCols;
+    const int beg = (int)((int64_t)full * w / W), end = (int)((int64_t)full * (w + 1) / W);
+    f32x4_t acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    f32x4_t accn[2];     // one group of queries: no second product
+    const i32x4_t none[1] = {};
+    float ss[2] = {0.0f, 0.0f};
+    auto ld = [](const S* p) { return (i32x4_t)*reinterpret_cast<const any_t*>(p); };
+    int k = beg;
+    for (; k < end; k += kU) {
+      i32x4_t a[kU], b[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        a[u] = b[u] = i32x4_t{0, 0, 0, 0};
+        if (k + u < end) {
+          a[u] = ld(pa + (k + u) * kCols);
+          b[u] = ld(pb + (k + u) * kCols);
+        }
+      }
+      add_batch<T, kU, false>(a, b, none, acc, accn, ss);
+    }
+    if (w == W - 1 && full * kCols < d) {
+      // The row's partial step: a partial chunk is read back to end with the row, less
+      // the elements the chunk before it holds.
+      const int c0 = full * kCols + grp * CE;  // this lane's first column
+      i32x4_t a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+      if (c0 < d) {
+        const int back = max(0, c0 + CE - d);
+        a = ld(pa + full * kCols - back) & tail_mask((uint32_t)c0 * sizeof(S), row_bytes);
+        b = ld(pb + full * kCols - back);
+        if (back > 0) b = b & tail_mask((uint32_t)c0 * sizeof(S), row_bytes);
+      }
+      ss[0] = dot<T>(a, a, ss[0]);
+      acc[0] = mma<T>(a, b, acc[0]);
+    }
+    f32x4_t lt = acc[0] + acc[1];
+    const float sw = sum_groups(ss[0] + ss[1]);
+    if (lane < 16) xs[slot][w][lane] = sw;
+    if constexpr (W > 1) {
+      *(f32x4_t*)&xl[w][lane][0] = lt;
+      __syncthreads();
+      lt = *(const f32x4_t*)&xl[0][lane][0];
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    f32x4_t sq = *(const f32x4_t*)&xs[slot][0][4 * grp];
+#pragma unroll
+    for (int ww = 1; ww < W; ++ww) {
+      lt += *(const f32x4_t*)&xl[ww][lane][0];
+      sq += *(const f32x4_t*)&xs[slot][ww][4 * grp];
+    }
+
+    // 2. Softmax of query qi over rows n = 4 grp + j; the weights as a table [n][s].
+    float lg[4], p[4], mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lg[j] = lt[j] * rsqrtf(fmaf(sq[j], inv_d, eps));
+      if (4 * grp + j < n_src) mx = fmaxf(mx, lg[j]);
+    }
+    mx = max_groups(mx);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = 4 * grp + j < n_src ? expf(lg[j] - mx) : 0.0f;
+    const float l = sum_groups((p[0] + p[1]) + (p[2] + p[3]));
+    if (m_out != nullptr && w == 0 && grp == 0 && qi < n_q) {
+      m_out[(int64_t)qi * n_tok + tok] = mx;
+      l_out[(int64_t)qi * n_tok + tok] = l;
+    }
+    const float inv_l = normalize ? 1.0f / l : 1.0f;
+    if (grp < NG && qi < kS) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tab[wave][(4 * grp + j) * kS + qi] = p[j] * inv_l;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float cf[kVgprs];
+#pragma unroll
+    for (int i = 0; i < kVgprs; ++i) cf[i] = tab[wave][64 * i + lane];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    // 3. The outputs, 64 chunks a wave at a time.
+    for (uint32_t base = (uint32_t)w * 1024u; base < row_bytes; base += 1024u * W) {
+      const uint32_t off = base + lane * 16u;
+      i32x4_t x[NR];
+#pragma unroll
+      for (int n = 0; n < NR; ++n) {
+        x[n] = i32x4_t{0, 0, 0, 0};
+        if (n < n_src) x[n] = ld_row<true>(row_of<const S>(v, n) + tok * d, row_bytes, off);
+      }
+      i32x4_t o[kS];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        float res[kS][2];
+#pragma unroll
+        for (int h = 0; h < kEpd; ++h) {
+          f32x4_t y[SG];
+#pragma unroll
+          for (int g = 0; g < SG; ++g) y[g] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+          static_for<NR>([&](auto NI) {
+            const float xe = elem<T>(x[NI.value], kk * kEpd + h);
+            static_for<SG>([&](auto GI) {
+              constexpr int op = NI.value * SG + GI.value;
+              y[GI.value] = __builtin_amdgcn_mfma_f32_4x4x1f32(cf[op / 16], xe, y[GI.value], 4, op % 16, 0);
+            });
+          });
+#pragma unroll
+          for (int s = 0; s < kS; ++s) res[s][h] = y[s / 4][s % 4];
+        }
+#pragma unroll
+        for (int s = 0; s < kS; ++s) {
+          if constexpr (T::code == F32::code) {
+            o[s][kk] = __float_as_int(res[s][0]);
+          } else {
+            const f32x2_t two = {res[s][0], res[s][1]};
+            if constexpr (T::code == BF16::code)
+              o[s][kk] = __builtin_bit_cast(int, __builtin_convertvector(two, bf16x2_t));
+            else
+              o[s][kk] = __builtin_bit_cast(int, __builtin_convertvector(two, f16x2_t));
+          }
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < kS; ++s)
+        if (s < n_q)
+          st_row<true, 0>(out + ((int64_t)s * n_tok + tok) * d, row_bytes, off, true, o[s]);
+    }
+    if constexpr (W > 1) {
+      if (tok + hop < n_tok) __syncthreads();  // the exchange is rewritten
+    }
+  }
+}
+
 // ------------------------------------------------------------------- launch
 
 template <class T, int NR, int SG>
@@ -537,7 +714,52 @@ hipError_t two_pass_t(int dtype, int n_src, int n_q, const BwdBatchedArgs* a, co
   return two_pass_n<F32>(n_src, n_q, a, t, s, info);
 }
 
+template <class T, int NR, int SG>
+hipError_t any_w(const BatchedArgs& a, hipStream_t s) {
+  using St = typename T::storage;
+  // A wave per token once the device is full of them and a row is at most four
+  // 64-chunk walks; else four waves share it. bf16, us, four waves -> one: N=9 S=8
+  // T=8192 D=256 52.1 -> 25.9, T=4096 D=768 44.3 -> 35.9, N=12 D=1280 87.0 -> 63.6;
+  // N=9 D=2560 108 -> 117, T=64 D=1280 7.2 -> 13.9.
+  int cus = 0;
+  if (cu_count(&cus) != hipSuccess || cus < 1) cus = 1;
+  const bool wave_token = a.n_tok >= 4 * (int64_t)cus && a.d <= 256 * T::ce;
+  const int tpb = wave_token ? kCoefWaves : 1;
+  const dim3 grid((unsigned)std::min<int64_t>((a.n_tok + tpb - 1) / tpb, 1 << 20));
+  const float inv_d = 1.0f / (float)a.d;
+  if (wave_token)
+    hipLaunchKernelGGL((k_batched_any<T, NR, SG, 1>), grid, dim3(64 * kCoefWaves), 0, s, a.v, (const St*)a.q,
+                       (St*)a.out, a.m_out, a.l_out, a.normalize, a.n_src, a.n_q, a.n_tok, a.d, a.eps, inv_d);
+  else
+    hipLaunchKernelGGL((k_batched_any<T, NR, SG, kCoefWaves>), grid, dim3(64 * kCoefWaves), 0, s, a.v,
+                       (const St*)a.q, (St*)a.out, a.m_out, a.l_out, a.normalize, a.n_src, a.n_q, a.n_tok,
+                       a.d, a.eps, inv_d);
+  return hipGetLastError();
+}
+
+template <class T, int NR>
+hipError_t any_q(const BatchedArgs& a, hipStream_t s) {
+  if (a.n_q <= 4) return any_w<T, NR, 1>(a, s);
+  if (a.n_q <= 8) return any_w<T, NR, 2>(a, s);
+  return any_w<T, NR, 4>(a, s);
+}
+
+template <class T>
+hipError_t any_n(const BatchedArgs& a, hipStream_t s) {
+  if (a.n_src <= 4) return any_q<T, 4>(a, s);
+  if (a.n_src <= 9) return any_q<T, 9>(a, s);
+  return any_q<T, 16>(a, s);
+}
+
 }  // namespace
+
+hipError_t launch_batched_any(const BatchedArgs& a, hipStream_t s) {
+  if (!batched_any_fits(a.n_src, a.n_q, a.d, a.dtype)) return hipErrorInvalidConfiguration;
+  if (a.n_tok == 0) return hipSuccess;
+  if (a.dtype == SY_BF16) return any_n<BF16>(a, s);
+  if (a.dtype == SY_F16) return any_n<F16>(a, s);
+  return any_n<F32>(a, s);
+}
 
 hipError_t two_pass_shape(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype, TwoPass* out) {
   hipError_t e = two_pass_t(dtype, (int)n_src, (int)n_q, nullptr, *out, nullptr, out);

@@ -470,6 +470,15 @@ int batched_impl(const RowTable& v, bool v_ok, const void* q, void* out, float* 
   // The matrix kernel's store offsets are 32-bit; past that, per-query launches.
   if (p.family == SY_FAMILY_MATRIX && !matrix_batched_offsets_fit(n_q, n_tok, d))
     p.family = SY_FAMILY_PER_QUERY;
+  int cus = 0;
+  if (cu_count(&cus) != hipSuccess) cus = 1;
+  sy_tuning forced;  // a measurement override of the register tile is kept
+  const bool tile = tuning_snapshot(&forced) && forced.batched_tile[0] != 0;
+  if (!tile && batched_any_wanted(p, n_src, n_q, n_tok, d, dtype, cus)) {
+    const BatchedArgs a{v,          q,        out,   m_out,  l_out, normalize,
+                        (int)n_src, (int)n_q, n_tok, (int)d, dtype, eps};
+    return status(launch_batched_any(a, s));
+  }
   if (p.family == SY_FAMILY_RESIDENT || p.family == SY_FAMILY_MATRIX) {
     const BatchedArgs a{v,          q,        out,   m_out,  l_out, normalize,
                         (int)n_src, (int)n_q, n_tok, (int)d, dtype, eps};

@@ -132,6 +132,30 @@ inline bool two_pass_wanted(const sy_plan& p, int64_t n_src, int64_t n_q, int64_
   if (dtype == SY_F32) return pairs >= 48;
   return pairs >= 32 || (n_q >= 2 && ((pairs >= 16 && elems >= (1 << 20)) || elems >= (1 << 23)));
 }
+// Batched forward for rows of any start and width of at least one chunk, at most 16
+// sources and 16 queries (k_batched_any in sy_batched.hip). Whether a launch whose plan
+// is `p` runs it, both sides in us: instead of a launch a query from three queries on
+// (bf16 N=12 S=8 T=4096 D=1280 159 vs 64, odd D=2313 N=9 S=10 T=512 118 vs 28; N=12 S=2
+// T=4096 D=2048 71 vs 75). Instead of the
+// register tile for 16-bit rows with many (query, source) pairs, or fewer where few
+// tokens leave that tile's waves idle (N=9 S=8 T=4096 D=768 44 vs 36, S=6 T=1024 D=1280
+// 20.4 vs 14.9, N=3 S=9 T=4944 D=640 22 vs 29, N=9 S=3 T=4096 D=1280 37 vs 40; N=4 S=4
+// T=64 8.1 vs 5.7, T=4096 21 vs 31; N=9 S=2 T=512 9.8 vs 8.1). fp32 register tiles stay
+// (N=9 S=8 T=2048 D=2048 70 vs 78, N=12 S=4 T=4096 D=512 39 vs 41) but for the 16-row one,
+// whose rows leave one wave a SIMD, with many pairs (N=12 S=8 T=2048 D=2048 143 vs 104, N=16
+// S=8 T=2048 D=1024 90 vs 58, N=16 S=16 T=512 D=1024 69 vs 18.5).
+inline bool batched_any_fits(int64_t n_src, int64_t n_q, int64_t d, int dtype) {
+  return n_src >= 1 && n_src <= 16 && n_q >= 1 && n_q <= 16 && d >= (dtype == SY_F32 ? 4 : 8) &&
+         d <= 0x7fffffff / 16;
+}
+inline bool batched_any_wanted(const sy_plan& p, int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d,
+                               int dtype, int cus) {
+  if (p.family == SY_FAMILY_MATRIX || !batched_any_fits(n_src, n_q, d, dtype)) return false;
+  if (p.family != SY_FAMILY_RESIDENT) return n_q >= 3;
+  const int64_t pairs = n_src * n_q;
+  if (dtype == SY_F32) return pairs >= 64 && n_src > 9;
+  return pairs >= 48 || (pairs >= 16 && n_tok <= 2 * (int64_t)cus);
+}
 // Dynamic LDS the generic kernels may request (bytes).
 constexpr int64_t kGenericMaxLds = 64 * 1024;
 // LDS of the generic batched backward: per-(query, row) alpha and da, per-row
@@ -280,6 +304,8 @@ struct TwoPass {
 // Fills the shape for the current device (the arguments must pass two_pass_fits).
 hipError_t two_pass_shape(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype, TwoPass* out);
 hipError_t launch_bwd_two_pass(const BwdBatchedArgs& a, const TwoPass& t, hipStream_t s);
+
+hipError_t launch_batched_any(const BatchedArgs& a, hipStream_t s);
 
 // Device queries, cached per device (sy_capi.cpp).
 hipError_t cu_count(int* out);
