@@ -107,7 +107,10 @@ typedef struct sy_plan {
  * fp32 forwards take four waves a token up to one token per CU (10-16 rows:
  * two), and 16-bit D = 4096 up to one token per CU runs the forward on four
  * waves and the backward on eight;
- * sy_kernel_info and sy_plan_for_tokens report
+ * some shapes reported as generic, per-query or resident launch a faster kernel
+ * with the same results: a query of another dtype, rows that start at no
+ * 16-byte boundary or have an odd D, and batched shapes outside the matrix
+ * tiles; sy_kernel_info and sy_plan_for_tokens report
  * the launched tile, this function, having no token count, does not.
  * Replaces the dispatch helpers _launch_config, _bwd_launch and
  * _batched_launch (src/switchyard/triton_op.py:130-150, :267-276, :420-435). */
@@ -303,7 +306,8 @@ int sy_batched_with_stats(const void* v, const void* queries, void* o, float* m,
                           int dtype, float eps, void* stream);
 
 /* Bytes of workspace sy_bwd_batched needs (fp32 dq partials, one row of
- * n_q*D per workgroup of its persistent grid), or < 0 on bad input. */
+ * n_q*D per workgroup of its persistent grid; where it runs in two passes also
+ * every token's fp32 coefficients between them), or < 0 on bad input. */
 int64_t sy_bwd_batched_workspace_bytes(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d,
                                        int dtype);
 
