@@ -386,6 +386,19 @@ std::optional<Tensor> block_attn_res_batched_train(const Tensor& v, const Tensor
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 int64_t chunk(const Tensor& t) { return 16 / (int64_t)t.element_size(); }
 
+// The gradients of a backward that is itself recorded (create_graph): the kernels'
+// results carry no graph, so there the same sublayer is evaluated from torch operations
+// in fp32 and differentiated. `y` is formed from `inputs`.
+variable_list recorded_grads(const Tensor& y, const variable_list& inputs, const Tensor& g) {
+  variable_list need, all(inputs.size());
+  for (const Tensor& x : inputs)
+    if (x.requires_grad()) need.push_back(x);
+  const variable_list r = torch::autograd::grad({y}, need, {g}, /*retain_graph=*/true, /*create_graph=*/true);
+  for (size_t k = 0, j = 0; k < inputs.size(); ++k)
+    if (inputs[k].requires_grad()) all[k] = r[j++];
+  return all;
+}
+
 Tensor norm_forward(const Tensor& x, const Tensor& w, double eps, Tensor* rinv) {
   const c10::DeviceGuard guard(x.device());
   const int64_t d = w.size(0), tok = x.numel() / d;
@@ -403,12 +416,20 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
     Tensor rinv;
     Tensor out = norm_forward(x, w, eps, &rinv);
     ctx->save_for_backward({x, w, rinv});
+    ctx->saved_data["eps"] = eps;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w = saved[1];
     const c10::DeviceGuard guard(x.device());
+    if (at::GradMode::is_enabled()) {
+      const Tensor xf = x.to(at::kFloat);
+      const Tensor r = xf.square().mean(-1, /*keepdim=*/true).add(ctx->saved_data["eps"].toDouble()).rsqrt();
+      const Tensor y = (xf * r * w.to(at::kFloat)).to(x.scalar_type());
+      const variable_list d = recorded_grads(y, {x, w}, grads[0]);
+      return {d[0], d[1], Tensor()};
+    }
     const int64_t d = w.size(0), tok = x.numel() / d;
     Tensor g = grad_like(grads[0], x);
     if (!aligned16(g)) g = g.clone();
@@ -454,6 +475,20 @@ struct RopeQkv : torch::autograd::Function<RopeQkv> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
+    if (at::GradMode::is_enabled()) {  // the kernel's inverse rotation, recorded
+      const int64_t t = grads[0].size(2), half = grads[0].size(3) / 2;
+      const Tensor c = saved[0].reshape({-1, half}).slice(0, 0, t), s = saved[1].reshape({-1, half}).slice(0, 0, t);
+      variable_list d;
+      for (int k = 0; k < 3; ++k) {
+        Tensor g = grads[k];
+        if (k < 2) {
+          const auto p = g.to(at::kFloat).chunk(2, -1);
+          g = at::cat({p[0] * c + p[1] * s, p[1] * c - p[0] * s}, -1).to(g.scalar_type());
+        }
+        d.push_back(g.transpose(1, 2));
+      }
+      return {at::stack(d, 2), Tensor(), Tensor()};
+    }
     for (Tensor& g : grads) {
       g = dense(g);
       if (!aligned16(g)) g = g.clone();
@@ -502,6 +537,10 @@ struct SwiGlu : torch::autograd::Function<SwiGlu> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor gu = ctx->get_saved_variables()[0];
     const c10::DeviceGuard guard(gu.device());
+    if (at::GradMode::is_enabled()) {
+      const auto p = gu.to(at::kFloat).chunk(2, -1);
+      return recorded_grads((at::silu(p[0]) * p[1]).to(gu.scalar_type()), {gu}, grads[0]);
+    }
     Tensor g = grad_like(grads[0], gu);
     if (!aligned16(g)) g = g.clone();
     Tensor d = at::empty(gu.sizes(), gu.options().requires_grad(false));

@@ -92,6 +92,39 @@ def test_swiglu(shape, dtype):
     _close(dx, torch.autograd.grad(ref, x6, g.double())[0], dtype)
 
 
+@pytest.mark.parametrize("op", ["rms_norm", "frozen_norm", "swiglu", "rope_qkv"])
+def test_second_derivatives(op):
+    """A recorded backward (create_graph) can itself be differentiated, as through the
+    plain operations; fp32 sums of at most 64 products and their products: 1e-5."""
+    print(f"second derivatives {op}", flush=True)
+    m = _lib.native()
+    rot = Rotary(16, 8, 1e4).to(DEV)
+    shape = (2, 8, 3, 2, 16) if op == "rope_qkv" else (5, 64)
+    x, w = _rand(*shape, dtype=F, seed=1), _rand(64, dtype=F, seed=2)
+
+    def call(x, w):
+        if op in ("rms_norm", "frozen_norm"):
+            return [m.rms_norm(x, w, 1e-6)] if x.dtype == F else [x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w]
+        if op == "swiglu":
+            a, u = x.chunk(2, -1)
+            return [m.swiglu(x)] if x.dtype == F else [torch.nn.functional.silu(a) * u]
+        if x.dtype == F:
+            return m.rope_qkv(x, rot.cos, rot.sin)
+        lo, hi = x[:, :, :2].chunk(2, -1)
+        c, s = (y[:8].reshape(8, 1, 1, 8).double() for y in (rot.cos, rot.sin))
+        qk = torch.cat((lo * c - hi * s, lo * s + hi * c), -1)
+        return [y.transpose(1, 2) for y in (*qk.unbind(2), x[:, :, 2])]
+
+    got = []
+    for dtype in (F, torch.float64):
+        xx, ww = x.to(dtype).requires_grad_(), w.to(dtype).requires_grad_(op != "frozen_norm")
+        leaves = [xx, ww] if op == "rms_norm" else [xx]
+        first = torch.autograd.grad(sum(y.pow(3).sum() for y in call(xx, ww)), leaves, create_graph=True)
+        got.append([*first, *torch.autograd.grad(sum(y.square().sum() for y in first), leaves)])
+    for a, b in zip(*got):
+        assert rel_l2(a.detach().cpu(), b.detach().cpu()) <= 1e-5
+
+
 def test_other_tensors_are_left_to_the_plain_operations():
     m = _lib.native()
     x, w = _rand(4, 64, dtype=BF, seed=1), _rand(64, dtype=BF, seed=2)
