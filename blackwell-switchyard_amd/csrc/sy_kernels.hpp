@@ -614,7 +614,6 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
                 ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
                 dt = wq.dot(x[n][j], j, dt);
                 reconvert<WIDE>(x[n][j]);
-            reconvert<WIDE>(x[n][j]);
               }
               const float pv[2] = {ss, dt};
               const float s2 = tsum<2>(pv, lane);  // lanes 0..31: ss, 32..63: dt
@@ -948,9 +947,7 @@ k_bwd(const RowTable v, const void* __restrict__ w,
     for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, gain, lane_off + j * kStep, row_bytes, wt, wf[j]);
     own = tail_mask(lane_off + (VPL - 1) * kStep, row_bytes);
   } else if constexpr (STATS && !kLean) {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j)
-      ld_query_gain<CE>(w, gain, wt, (uint32_t)d, (lane_off + j * kStep) / 16u, wf[j]);
+    ld_query_row(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
   } else {
     const auto wr = make_rsrc(w, row_bytes);
 #pragma unroll
@@ -1294,11 +1291,7 @@ k_bwd_tall(const RowTable v, const void* __restrict__ w,
   const int iters = n_iter;  // every slot meets the same barriers
 
   float wf[VPL][CE];
-  {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j)
-      ld_query_gain<CE>(w, gain, wt, (uint32_t)d, (lane_off + j * kStep) / 16u, wf[j]);
-  }
+  ld_query_row(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
   float dwa[VPL][CE];
 #pragma unroll
   for (int j = 0; j < VPL; ++j)
