@@ -175,7 +175,9 @@ def slab_copies(n_sublayers: int, n_blocks: int, sources: str) -> int:
 # whole 16-byte chunks), operation by operation otherwise. The kernels compute in fp32
 # and round once, where the operations round every intermediate to the activations'
 # dtype. Prefill of the small decoder (8 layers, 4 x 512 tokens of 512, bf16) was bound
-# by ~700 launches: 4.2-4.7 ms, with the kernels 1.7 ms.
+# by ~700 launches: 4.2-4.7 ms, with the kernels 1.7 ms. Symbolic tracing (whose proxies
+# are no tensors, and are asked nothing about their device) and scripting see the plain
+# operations.
 
 
 class RMSNorm(nn.Module):
@@ -187,10 +189,11 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(d))
 
     def forward(self, x: Tensor) -> Tensor:
-        if x.is_cuda and _lib.ordinary(x):
-            out = _lib.native().rms_norm(x, self.weight, self.eps)
-            if out is not None:
-                return out
+        if not torch.jit.is_scripting():
+            if _lib.ordinary(x) and x.is_cuda:
+                out = _lib.native().rms_norm(x, self.weight, self.eps)
+                if out is not None:
+                    return out
         inv = x.float().square().mean(dim=-1, keepdim=True).add(self.eps).rsqrt()
         return x * inv.to(x.dtype) * self.weight
 
@@ -229,7 +232,7 @@ class Attention(nn.Module):
         b, t, d = x.shape
         qkv = self.qkv(x).view(b, t, 3, self.heads, self.hd)
         split = None
-        if qkv.is_cuda and _lib.ordinary(qkv):
+        if _lib.ordinary(qkv) and qkv.is_cuda:
             split = _lib.native().rope_qkv(qkv, rotary.cos, rotary.sin)
         if split is None:
             q, k, v = qkv.unbind(2)
@@ -250,7 +253,7 @@ class GatedMLP(nn.Module):
 
     def forward(self, x: Tensor, rotary: Rotary | None = None) -> Tensor:
         y = self.gate_up(x)
-        if y.is_cuda and _lib.ordinary(y):
+        if _lib.ordinary(y) and y.is_cuda:
             h = _lib.native().swiglu(y)
             if h is not None:
                 return self.down(h)
