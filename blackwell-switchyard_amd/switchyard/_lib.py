@@ -164,10 +164,15 @@ def native():
     return _native
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def ordinary(*tensors) -> bool:
-    """Whether the native functions may be offered a call: tensors, outside a
-    compiler's trace (which has to see the Python function)."""
-    return not torch.compiler.is_compiling() and all(isinstance(t, torch.Tensor) for t in tensors)
+    """Whether the native functions may be offered a call: plain tensors, outside a
+    compiler's trace. Tracers have to see the Python function, and so have subclasses:
+    one that only overrides ``__torch_function__`` looks like any tensor to native
+    code and would come out a plain one."""
+    return not torch.compiler.is_compiling() and all(type(t) in _PLAIN for t in tensors)
 
 
 def dtype_code(dtype: torch.dtype) -> int:

@@ -277,7 +277,7 @@ class BlockAttnResHIP(torch.nn.Module):
         self.g = torch.nn.Parameter(torch.ones(d_model)) if norm_affine else None
 
     def forward(self, v: torch.Tensor) -> torch.Tensor:
-        if self.g is not None and _lib.ordinary(v):
+        if self.g is not None and _lib.ordinary(v, self.w, self.g):
             out = _lib.native().block_attn_res_gain(v, self.w, self.g, float(self.eps))
             if out is not None:
                 return out

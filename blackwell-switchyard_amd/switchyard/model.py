@@ -190,7 +190,7 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: Tensor) -> Tensor:
         if not torch.jit.is_scripting():
-            if _lib.ordinary(x) and x.is_cuda:
+            if _lib.ordinary(x, self.weight) and x.is_cuda:
                 out = _lib.native().rms_norm(x, self.weight, self.eps)
                 if out is not None:
                     return out
@@ -455,7 +455,7 @@ def _hip_stacked(v: Tensor, q: Tensor, eps: float) -> Tensor:
 def _hip_module(v: Tensor, site: BlockAttnRes, eps: float) -> Tensor:
     """The operator at ``site`` with no backward to come; the kernel multiplies the
     query by the gain."""
-    if site.g is not None and _lib.ordinary(v):
+    if site.g is not None and _lib.ordinary(v, site.w, site.g):
         out = _lib.native().block_attn_res_gain(v, site.w, site.g, float(eps))
         if out is not None:
             return out

@@ -46,3 +46,27 @@ def test_a_norm_can_be_scripted():
     norm = RMSNorm(64, 1e-6)
     x = torch.randn(2, 8, 64, generator=torch.Generator().manual_seed(0))
     assert torch.equal(torch.jit.script(norm)(x), norm(x))
+
+
+class _Tagged(torch.Tensor):
+    """A subclass with nothing of its own but the default ``__torch_function__``, which
+    keeps results in the subclass."""
+
+
+def test_a_subclass_is_left_to_the_plain_operations():
+    from switchyard import _lib
+
+    x = torch.zeros(2)
+    assert _lib.ordinary(x, torch.nn.Parameter(x)) and not _lib.ordinary(x, x.as_subclass(_Tagged))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tagged", ["input", "weight"])
+def test_a_subclass_comes_out_of_the_sublayers(tagged):
+    x = torch.randn(2, 8, 64, generator=torch.Generator().manual_seed(0)).cuda()
+    norm, mlp = RMSNorm(64, 1e-6).cuda(), GatedMLP(CFG).cuda()
+    if tagged == "weight":
+        norm.weight = torch.nn.Parameter(norm.weight.data.as_subclass(_Tagged))
+        assert type(norm(x)) is _Tagged
+    else:
+        assert type(norm(x.as_subclass(_Tagged))) is _Tagged and type(mlp(x.as_subclass(_Tagged))) is _Tagged
