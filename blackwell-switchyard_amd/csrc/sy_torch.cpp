@@ -505,7 +505,7 @@ struct RopeQkv : torch::autograd::Function<RopeQkv> {
   }
 };
 
-// qkv [B, T, 3, H, hd], tables [>= T, ..., hd/2] -> (q, k, v), each [B, H, T, hd].
+// qkv [B, T, 3, H, hd], tables [>= T, 1, hd/2] -> (q, k, v), each [B, H, T, hd].
 std::optional<variable_list> rope_qkv(const Tensor& qkv, const Tensor& cosv, const Tensor& sinv) {
   if (!ordinary() || !plain(qkv) || !plain(cosv) || !plain(sinv) || qkv.dim() != 5 || qkv.size(2) != 3 ||
       qkv.numel() == 0 || !qkv.is_contiguous() || !aligned16(qkv) || qkv.size(4) % (2 * chunk(qkv)) != 0 ||
@@ -513,8 +513,8 @@ std::optional<variable_list> rope_qkv(const Tensor& qkv, const Tensor& cosv, con
     return std::nullopt;
   for (const Tensor* t : {&cosv, &sinv})
     if (t->scalar_type() != at::kFloat || t->device() != qkv.device() || !t->is_contiguous() ||
-        t->requires_grad() || t->dim() < 2 || t->size(-1) != qkv.size(4) / 2 || t->size(0) < qkv.size(1) ||
-        t->numel() != t->size(0) * t->size(-1))
+        t->requires_grad() || t->dim() != 3 || t->size(1) != 1 || t->size(2) != qkv.size(4) / 2 ||
+        t->size(0) < qkv.size(1))
       return std::nullopt;
   if (at::GradMode::is_enabled() && qkv.requires_grad()) return RopeQkv::apply(qkv, cosv, sinv);
   return rope_forward(qkv, cosv, sinv);

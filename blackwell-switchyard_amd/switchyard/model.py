@@ -180,6 +180,14 @@ def slab_copies(n_sublayers: int, n_blocks: int, sources: str) -> int:
 # operations.
 
 
+def _only_forward(m: nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` would run ``cls.forward`` and nothing else: no subclass, no
+    replaced ``forward``, no hooks. Only then may a kernel stand in for the call."""
+    return (type(m) is cls and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and not nn.modules.module._has_any_global_hook())
+
+
 class RMSNorm(nn.Module):
     """``x / rms(x) * weight``, the statistic in fp32."""
 
@@ -232,7 +240,7 @@ class Attention(nn.Module):
         b, t, d = x.shape
         qkv = self.qkv(x).view(b, t, 3, self.heads, self.hd)
         split = None
-        if _lib.ordinary(qkv) and qkv.is_cuda:
+        if _lib.ordinary(qkv) and qkv.is_cuda and _only_forward(rotary, Rotary) and _lib.ordinary(rotary.cos, rotary.sin):
             split = _lib.native().rope_qkv(qkv, rotary.cos, rotary.sin)
         if split is None:
             q, k, v = qkv.unbind(2)

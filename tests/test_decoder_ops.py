@@ -14,7 +14,7 @@ if not torch.cuda.is_available():  # pragma: no cover
 
 from oracle.reference import dtype_floor, rel_l2  # noqa: E402
 from switchyard import _lib  # noqa: E402
-from switchyard.model import ModelConfig, Rotary, Transformer  # noqa: E402
+from switchyard.model import Attention, ModelConfig, Rotary, Transformer  # noqa: E402
 
 DEV = "cuda"
 BF, HF, F = torch.bfloat16, torch.float16, torch.float32
@@ -158,3 +158,36 @@ def test_the_decoder_agrees_with_its_plain_operations(residual, monkeypatch):
             got[-1].append(model(idx))
     for a, b in zip(*got):
         torch.testing.assert_close(a, b, rtol=2e-4, atol=2e-5)  # fp32 sums in another order, two layers deep
+
+
+class _Turned(Rotary):
+    def forward(self, x):
+        return super().forward(x) * 2
+
+
+def test_attention_calls_a_rotary_that_is_more_than_its_tables():
+    """Hooks, a subclass, a replaced forward and tables that broadcast otherwise all act
+    as they do on the plain operations; the plain rotary's kernel agrees with them."""
+    torch.manual_seed(0)
+    cfg = ModelConfig(vocab_size=128, d_model=64, n_heads=2, d_ff=128, n_layers=2, n_blocks=2, max_seq_len=32)
+    attn, rot, x = Attention(cfg).to(DEV), Rotary(32, 32, 1e4).to(DEV), _rand(2, 8, 64, dtype=F, seed=1)
+    ref, calls = attn(x, rot), []
+    hook = rot.register_forward_hook(lambda *a: calls.append(1))
+    torch.testing.assert_close(attn(x, rot), ref)
+    hook.remove()
+    assert len(calls) == 2
+    hook = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: calls.append(1) if m is rot else None)
+    attn(x, rot)
+    hook.remove()
+    assert len(calls) == 4
+    sub = _Turned(32, 32, 1e4).to(DEV)
+    replaced = Rotary(32, 32, 1e4).to(DEV)
+    replaced.forward = lambda y: Rotary.forward(replaced, y) * 2
+    torch.testing.assert_close(attn(x, sub), attn(x, replaced))
+    assert not torch.allclose(attn(x, sub), ref)
+    with torch.no_grad():
+        assert torch.equal(attn(x, rot), ref) and not calls[4:]
+    # positions along the batch, as broadcasting has it: refused by the plain operations
+    rot.cos, rot.sin = rot.cos[:, 0], rot.sin[:, 0]
+    with pytest.raises(RuntimeError):
+        attn(x, rot)
