@@ -50,11 +50,15 @@ void* stream_of(const Tensor& t) {
 }
 
 // A dense GPU tensor of a supported dtype that nothing intercepts: no tensor subclass
-// with its own dispatch, no lazy negation or conjugation, no forward-mode tangent.
+// with its own dispatch, no transform's wrapper, no lazy negation or conjugation, no
+// forward-mode tangent.
 bool plain(const Tensor& t) {
+  using c10::DispatchKey;
+  constexpr c10::DispatchKeySet wrapped{DispatchKey::FuncTorchBatched, DispatchKey::FuncTorchGradWrapper,
+                                        DispatchKey::Batched, DispatchKey::Functionalize};
   return t.defined() && t.is_cuda() && t.layout() == at::kStrided && code_of(t) >= 0 &&
-         !t.unsafeGetTensorImpl()->is_python_dispatch() && !t.is_neg() && !t.is_conj() &&
-         !t._fw_grad(0).defined();
+         !t.unsafeGetTensorImpl()->is_python_dispatch() && !t.key_set().has_any(wrapped) && !t.is_neg() &&
+         !t.is_conj() && !t._fw_grad(0).defined();
 }
 
 // No function transform (vmap, grad, jvp), torch dispatch or function mode, nor tracer
@@ -386,17 +390,15 @@ std::optional<Tensor> block_attn_res_batched_train(const Tensor& v, const Tensor
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 int64_t chunk(const Tensor& t) { return 16 / (int64_t)t.element_size(); }
 
-// The gradients of a backward that is itself recorded (create_graph): the kernels'
-// results carry no graph, so there the same sublayer is evaluated from torch operations
-// in fp32 and differentiated. `y` is formed from `inputs`.
-variable_list recorded_grads(const Tensor& y, const variable_list& inputs, const Tensor& g) {
-  variable_list need, all(inputs.size());
-  for (const Tensor& x : inputs)
-    if (x.requires_grad()) need.push_back(x);
-  const variable_list r = torch::autograd::grad({y}, need, {g}, /*retain_graph=*/true, /*create_graph=*/true);
-  for (size_t k = 0, j = 0; k < inputs.size(); ++k)
-    if (inputs[k].requires_grad()) all[k] = r[j++];
-  return all;
+// Whether a backward may launch its kernel. A recorded one (create_graph) may not, as
+// the kernels' results carry no graph, nor one inside a transform or mode or given a
+// wrapped gradient (is_grads_batched): those evaluate the same gradient from torch
+// operations in fp32.
+bool kernel_backward(const variable_list& grads) {
+  if (at::GradMode::is_enabled() || !ordinary()) return false;
+  for (const Tensor& g : grads)
+    if (!plain(g)) return false;
+  return true;
 }
 
 Tensor norm_forward(const Tensor& x, const Tensor& w, double eps, Tensor* rinv) {
@@ -423,12 +425,12 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w = saved[1];
     const c10::DeviceGuard guard(x.device());
-    if (at::GradMode::is_enabled()) {
-      const Tensor xf = x.to(at::kFloat);
+    if (!kernel_backward(grads)) {
+      const Tensor xf = x.to(at::kFloat), gf = grads[0].to(at::kFloat), gw = gf * w.to(at::kFloat);
       const Tensor r = xf.square().mean(-1, /*keepdim=*/true).add(ctx->saved_data["eps"].toDouble()).rsqrt();
-      const Tensor y = (xf * r * w.to(at::kFloat)).to(x.scalar_type());
-      const variable_list d = recorded_grads(y, {x, w}, grads[0]);
-      return {d[0], d[1], Tensor()};
+      const Tensor dx = r * gw - xf * (r.pow(3) * (gw * xf).mean(-1, /*keepdim=*/true));
+      const Tensor dw = (gf * xf * r).reshape({-1, w.size(0)}).sum(0);
+      return {dx.to(x.scalar_type()), dw.to(w.scalar_type()), Tensor()};
     }
     const int64_t d = w.size(0), tok = x.numel() / d;
     Tensor g = grad_like(grads[0], x);
@@ -475,7 +477,7 @@ struct RopeQkv : torch::autograd::Function<RopeQkv> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    if (at::GradMode::is_enabled()) {  // the kernel's inverse rotation, recorded
+    if (!kernel_backward(grads)) {  // the kernel's inverse rotation
       const int64_t t = grads[0].size(2), half = grads[0].size(3) / 2;
       const Tensor c = saved[0].reshape({-1, half}).slice(0, 0, t), s = saved[1].reshape({-1, half}).slice(0, 0, t);
       variable_list d;
@@ -537,9 +539,10 @@ struct SwiGlu : torch::autograd::Function<SwiGlu> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor gu = ctx->get_saved_variables()[0];
     const c10::DeviceGuard guard(gu.device());
-    if (at::GradMode::is_enabled()) {
+    if (!kernel_backward(grads)) {
       const auto p = gu.to(at::kFloat).chunk(2, -1);
-      return recorded_grads((at::silu(p[0]) * p[1]).to(gu.scalar_type()), {gu}, grads[0]);
+      const Tensor gf = grads[0].to(at::kFloat), s = at::sigmoid(p[0]);
+      return {at::cat({gf * p[1] * s * (1 + p[0] * (1 - s)), gf * p[0] * s}, -1).to(gu.scalar_type())};
     }
     Tensor g = grad_like(grads[0], gu);
     if (!aligned16(g)) g = g.clone();

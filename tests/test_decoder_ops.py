@@ -191,3 +191,57 @@ def test_attention_calls_a_rotary_that_is_more_than_its_tables():
     rot.cos, rot.sin = rot.cos[:, 0], rot.sin[:, 0]
     with pytest.raises(RuntimeError):
         attn(x, rot)
+
+
+def _sublayer(op):
+    """(function of the sublayer's inputs, inputs, the same from plain operations)."""
+    m = _lib.native()
+    if op == "rms_norm":
+        leaves = [_rand(5, 64, dtype=F, seed=1), _rand(64, dtype=F, seed=2)]
+        return (lambda x, w: m.rms_norm(x, w, 1e-6)), leaves, lambda x, w: (
+            x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w)
+    if op == "swiglu":
+        return m.swiglu, [_rand(5, 64, dtype=F, seed=1)], lambda x: torch.nn.functional.silu(x[:, :32]) * x[:, 32:]
+    rot = Rotary(16, 8, 1e4).to(DEV)
+
+    def plain(x):
+        q, k, v = x.unbind(2)
+        return torch.stack([y.transpose(1, 2) for y in (rot(q), rot(k), v)])
+
+    return (lambda x: torch.stack(m.rope_qkv(x, rot.cos, rot.sin))), [_rand(2, 8, 3, 2, 16, dtype=F, seed=1)], plain
+
+
+@pytest.mark.parametrize("op", ["rms_norm", "swiglu", "rope_qkv"])
+def test_a_backward_inside_a_transform_or_mode(op):
+    """Ordinary forwards whose backward is not: batched gradients, a dispatch mode, a
+    gradient with a tangent. fp32 sums of at most 64 products on both sides: 1e-5."""
+    print(f"backward inside a transform {op}", flush=True)
+    fused, leaves, plain = _sublayer(op)
+    leaves = [x.requires_grad_() for x in leaves]
+    out, ref = fused(*leaves), plain(*leaves)
+    g = _rand(3, *out.shape, dtype=F, seed=5)
+    got = torch.autograd.grad(out, leaves, g, is_grads_batched=True, retain_graph=True)
+    for k in range(3):
+        want = torch.autograd.grad(ref, leaves, g[k], retain_graph=True)
+        for a, b in zip(got, want):
+            assert rel_l2(a[k].cpu(), b.cpu()) <= 1e-5
+    jac = torch.autograd.functional.jacobian(lambda x: fused(x, *leaves[1:])[:1].flatten()[:4], leaves[0], vectorize=True)
+    assert jac.shape == (4, *leaves[0].shape)
+
+    class Seen(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    seen = []
+    with Seen():
+        got = torch.autograd.grad(out, leaves, g[0], retain_graph=True)
+    assert any("mul" in str(f) for f in seen)
+    for a, b in zip(got, torch.autograd.grad(ref, leaves, g[0], retain_graph=True)):
+        assert rel_l2(a.cpu(), b.cpu()) <= 1e-5
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(g[0].clone(), g[1])
+        got = torch.autograd.grad(out, leaves, dual, retain_graph=True)
+        tangent = torch.autograd.forward_ad.unpack_dual(got[0]).tangent
+    want = torch.autograd.grad(ref, leaves, g[1])[0]  # the gradient is linear in g
+    assert rel_l2(tangent.cpu(), want.cpu()) <= 1e-5
