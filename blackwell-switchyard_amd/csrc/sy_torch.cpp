@@ -183,6 +183,14 @@ struct BlockAttnResGain : torch::autograd::Function<BlockAttnResGain> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &v = saved[0], &w = saved[1];
     const c10::DeviceGuard guard(v.device());
+    if (at::GradMode::is_enabled()) {
+      // Recorded: the product's own gradients are torch operations, through which the
+      // factors can be differentiated again (the operator's carry no graph).
+      const Tensor wf = w.to(at::kFloat), gf = saved[2].to(at::kFloat);
+      const auto r = operator_backward(v, (wf * gf).detach(), saved[3], grads[0],
+                                       ctx->saved_data["eps"].toDouble());
+      return {r[0], (r[1] * gf).to(w.scalar_type()), (r[1] * wf).to(w.scalar_type()), Tensor()};
+    }
     const int64_t n = v.size(0), d = v.size(3), tok = v.size(1) * v.size(2);
     const int vt = code_of(v), wt = code_of(w);
     const Tensor go = grad_like(grads[0], v);

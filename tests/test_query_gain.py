@@ -53,3 +53,25 @@ def test_module_with_a_gain(shape, dtypes, wants):
         assert rel_l2(got, want) <= (1e-5 if dt == F else 1.10 * dtype_floor(want, dt))
     with torch.no_grad():
         assert torch.equal(mod(vv), out)
+
+
+@pytest.mark.parametrize("wdt", [BF, F])
+def test_a_recorded_backward_can_be_differentiated_by_the_factors(wdt):
+    """The operator's gradients carry no graph, the product's do: dw = dq g, dg = dq w."""
+    n, t, d = 4, 40, 256
+    gen = torch.Generator().manual_seed(3)
+    v, go = torch.randn(n, 1, t, d, generator=gen).to(BF).to(DEV), torch.randn(1, t, d, generator=gen).to(BF).to(DEV)
+    mod = BlockAttnResTriton(d).to(DEV).to(wdt)
+    with torch.no_grad():
+        mod.w.copy_(torch.randn(d, generator=gen) * d**-0.5)
+        mod.g.copy_(1 + 0.3 * torch.randn(d, generator=gen))
+    leaves = [mod.w, mod.g]
+    plain = torch.autograd.grad(mod(v), leaves, go)
+    dw, dg = torch.autograd.grad(mod(v), leaves, go, create_graph=True)
+    for a, b in zip((dw, dg), plain):  # one rounding each of sums in the same order
+        assert rel_l2(a.detach(), b.cpu().double()) <= (1e-6 if wdt == F else 4e-3)
+    ww, gg = torch.autograd.grad((dw.float().sum() + 2 * dg.float().sum()), leaves)
+    with torch.no_grad():
+        dq = dg.double() / mod.w.double()
+    for got, want in ((gg, dq), (ww, 2 * dq)):  # dg's rounding, and one of the result
+        assert got.dtype == wdt and rel_l2(got, want.cpu()) <= (1e-5 if wdt == F else 1e-2)
