@@ -126,8 +126,9 @@ def block_attn_res_sources(
     its own ``[B, T, D]`` gradient; ``dw`` is reduced in fp32 and returned in
     ``w.dtype``. ``1 <= N <= 16``.
     """
+    sources = list(sources)  # any iterable, also one that can be walked only once
     if _lib.ordinary(w, *sources):
-        out = _lib.native().block_attn_res_sources(list(sources), w, float(eps))
+        out = _lib.native().block_attn_res_sources(sources, w, float(eps))
         if out is not None:
             return out
     return _BlockAttnResSources.apply(w, eps, *sources)

@@ -99,3 +99,11 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, "bench.py", "--gpus", "2"], capture_output=True, text=True,
                        cwd=str(__import__("pathlib").Path(__file__).resolve().parents[1]), timeout=120)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def test_sources_may_come_from_an_iterator():
+    from switchyard.table_op import block_attn_res_sources
+
+    v, w = torch.randn(3, 1, 4, 8), torch.randn(8)
+    with pytest.raises(ValueError, match="CUDA"):  # past the checks of the list's length and shapes
+        block_attn_res_sources((s for s in v), w)
