@@ -26,6 +26,8 @@ Per token, with ``p_n = exp(logit_n - m)``: ``m = max_n logit_n``,
 
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from . import _lib
@@ -302,8 +304,9 @@ def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: 
     n = v.shape[0] if v.ndim == 4 else 0
     if not 0 < split < n:
         raise ValueError(f"split must be in (0, {n}), got {split}")
+    split = operator.index(split)  # a fraction is no source index
     if _lib.ordinary(v, w):
-        out = _lib.native().block_attn_res_two_phase(v, w, int(split), float(eps))
+        out = _lib.native().block_attn_res_two_phase(v, w, split, float(eps))
         if out is not None:
             return out
-    return _TwoPhase.apply(v, w, int(split), eps)
+    return _TwoPhase.apply(v, w, split, eps)

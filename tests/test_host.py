@@ -107,3 +107,14 @@ def test_sources_may_come_from_an_iterator():
     v, w = torch.randn(3, 1, 4, 8), torch.randn(8)
     with pytest.raises(ValueError, match="CUDA"):  # past the checks of the list's length and shapes
         block_attn_res_sources((s for s in v), w)
+
+
+def test_a_fractional_split_is_refused():
+    from switchyard.stats_op import block_attn_res_two_phase
+
+    v, w = torch.randn(4, 1, 3, 8), torch.randn(8)
+    for split in (2.5, 2.0):
+        with pytest.raises(TypeError):
+            block_attn_res_two_phase(v, w, split)
+    with pytest.raises(ValueError, match="CUDA"):  # any integer type is one
+        block_attn_res_two_phase(v, w, torch.tensor(2))
