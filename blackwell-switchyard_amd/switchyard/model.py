@@ -332,8 +332,10 @@ class _Stream:
     def accumulate(self, y: Tensor, region=contextlib.nullcontext) -> None:
         """Add a sublayer output to the running sum; in arena mode also copy
         the new sum into its slot (the staging cost, inside ``region``). With
-        no backward to come the sum is formed in its slot: one launch."""
-        if self.buf is not None and not torch.is_grad_enabled() and y.dtype == self.buf.slots.dtype:
+        no backward to come a sum of the slots' dtype is formed in its slot: one
+        launch. (A wider one stays outside: each sum would be rounded.)"""
+        if (self.buf is not None and not torch.is_grad_enabled() and y.dtype == self.buf.slots.dtype
+                and (self.running is None or self.running.dtype == y.dtype)):
             k = len(self.blocks)
             slot = self.buf.slots[k]
             with region():

@@ -16,6 +16,7 @@ from switchyard.hip_op import BlockAttnResHIP, block_attn_res_batched, block_att
 from switchyard.triton_op import BlockAttnResTriton, block_attn_res_triton
 
 F64 = dict(dtype=torch.float64)
+BF = torch.bfloat16
 
 
 def test_alias_module_exposes_the_reference_names():
@@ -118,3 +119,19 @@ def test_a_fractional_split_is_refused():
             block_attn_res_two_phase(v, w, split)
     with pytest.raises(ValueError, match="CUDA"):  # any integer type is one
         block_attn_res_two_phase(v, w, torch.tensor(2))
+
+
+def test_a_running_sum_wider_than_the_slots_keeps_its_dtype():
+    from switchyard.model import _Stream
+
+    gen = torch.Generator().manual_seed(0)
+    x0, y1, y2, y3 = (torch.randn(1, 4, 8, generator=gen).to(d) for d in (BF, torch.float32, BF, BF))
+    sums = []
+    for arena in (True, False):
+        with torch.no_grad():
+            stream = _Stream(x0, 2, arena=arena)
+            for y in (y1, y2, y3):
+                stream.accumulate(y)
+        sums.append(stream.running)
+    assert sums[0].dtype == torch.float32 and torch.equal(*sums)
+    assert torch.equal(sums[0], (y1 + y2) + y3)
