@@ -462,16 +462,6 @@ def _hip_stacked(v: Tensor, q: Tensor, eps: float) -> Tensor:
     return block_attn_res_hip(v, q, eps)
 
 
-def _hip_module(v: Tensor, site: BlockAttnRes, eps: float) -> Tensor:
-    """The operator at ``site`` with no backward to come; the kernel multiplies the
-    query by the gain."""
-    if site.g is not None and _lib.ordinary(v, site.w, site.g):
-        out = _lib.native().block_attn_res_gain(v, site.w, site.g, float(eps))
-        if out is not None:
-            return out
-    return _hip_stacked(v, site.effective_query(), eps)
-
-
 def _hip_table(sources: list[Tensor], q: Tensor, eps: float) -> Tensor:
     from .table_op import MAX_SOURCES, block_attn_res_sources
 
@@ -562,27 +552,38 @@ class Transformer(nn.Module):
         with self._region("attnres_stage"):
             stream = _Stream(x0, cfg.n_blocks, arena=cfg.sources == "arena")
         counts = []
+        queries = self._queries()
         for i, (norm, fn) in enumerate(self._sublayers()):
             if i > 0 and i % cfg.block_size == 0:
                 stream.close_block()
-            h = self._site(i, stream, collect_alphas)
+            h = self._site(i, stream, collect_alphas, queries)
             counts.append(len(stream.sources()))
             y = fn(norm(h), self.rotary)
             stream.accumulate(y, lambda: self._region("attnres_stage"))
         stream.close_block()
         counts.append(len(stream.sources()))
         self.last_source_counts = counts
-        return self._site(cfg.n_sublayers, stream, collect_alphas)
+        return self._site(cfg.n_sublayers, stream, collect_alphas, queries)
 
-    def _site(self, i: int, stream: _Stream, collect_alphas: bool) -> Tensor:
+    def _queries(self) -> list[Tensor] | None:
+        """The sites' queries formed in one launch, where no backward is to come and
+        each is the plain product of its factors; None where each site forms its own."""
+        sites = list(self.attn_res)
+        if (self.cfg.residual != "switchyard" or torch.is_grad_enabled()
+                or not all(type(s) is BlockAttnRes and "effective_query" not in s.__dict__ and s.g is not None
+                           and _lib.ordinary(s.w, s.g) for s in sites)):
+            return None
+        return torch._foreach_mul([s.w for s in sites], [s.g for s in sites])
+
+    def _site(self, i: int, stream: _Stream, collect_alphas: bool, queries: list[Tensor] | None) -> Tensor:
         cfg = self.cfg
+        q = self.attn_res[i].effective_query() if queries is None else queries[i]
         sources = stream.sources()
         n = len(sources)
         hip = cfg.residual == "switchyard"
         if hip and stream.buf is not None and not torch.is_grad_enabled() and not collect_alphas:
             with self._region("attnres_op"):
-                return _hip_module(stream.buf.slots[:n], self.attn_res[i], cfg.norm_eps)
-        q = self.attn_res[i].effective_query()
+                return _hip_stacked(stream.buf.slots[:n], q, cfg.norm_eps)
         if collect_alphas:
             self.last_alphas.append(_mean_alpha(sources, q, cfg.norm_eps))
         if cfg.sources == "stack":

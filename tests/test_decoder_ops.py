@@ -245,3 +245,27 @@ def test_a_backward_inside_a_transform_or_mode(op):
         tangent = torch.autograd.forward_ad.unpack_dual(got[0]).tangent
     want = torch.autograd.grad(ref, leaves, g[1])[0]  # the gradient is linear in g
     assert rel_l2(tangent.cpu(), want.cpu()) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [BF, F])
+def test_the_sites_agree_bit_for_bit_in_every_mode(dtype):
+    """Trained queries (no zeros, no unit gains): the three ways of presenting sources,
+    with and without a backward to come, see the same query and give the same bits."""
+    print(f"site bits {dtype}", flush=True)
+    outs = {}
+    for sources in ("stack", "arena", "table"):
+        torch.manual_seed(0)
+        cfg = ModelConfig(vocab_size=128, d_model=128, n_heads=2, d_ff=128, n_layers=3, n_blocks=3, max_seq_len=32,
+                          residual="switchyard", sources=sources)
+        model = Transformer(cfg)
+        for site in model.attn_res:
+            torch.nn.init.normal_(site.w, std=0.3)
+            torch.nn.init.normal_(site.g, mean=1.0, std=0.3)
+        model = model.to(DEV, dtype)
+        idx = torch.randint(0, 128, (2, 32), generator=torch.Generator().manual_seed(1)).to(DEV)
+        outs[sources, True] = model(idx).detach()
+        with torch.no_grad():
+            outs[sources, False] = model(idx)
+            assert torch.equal(model(idx, collect_alphas=True), outs[sources, False])
+    ref = outs["stack", True]
+    assert all(torch.equal(x, ref) for x in outs.values())
