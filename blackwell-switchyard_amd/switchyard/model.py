@@ -65,6 +65,7 @@ from torch import Tensor
 
 from . import _lib
 from .baselines import folded_form
+from .hip_op import block_attn_res_hip
 from .reference import DEFAULT_EPS, BlockAttnRes
 
 __all__ = [
@@ -197,13 +198,14 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(d))
 
     def forward(self, x: Tensor) -> Tensor:
+        w = self.weight
         if not torch.jit.is_scripting():
-            if _lib.ordinary(x, self.weight) and x.is_cuda:
-                out = _lib.native().rms_norm(x, self.weight, self.eps)
+            if _lib.ordinary(x, w) and x.is_cuda:
+                out = _lib.native().rms_norm(x, w, self.eps)
                 if out is not None:
                     return out
         inv = x.float().square().mean(dim=-1, keepdim=True).add(self.eps).rsqrt()
-        return x * inv.to(x.dtype) * self.weight
+        return x * inv.to(x.dtype) * w
 
 
 class Rotary(nn.Module):
@@ -240,8 +242,10 @@ class Attention(nn.Module):
         b, t, d = x.shape
         qkv = self.qkv(x).view(b, t, 3, self.heads, self.hd)
         split = None
-        if _lib.ordinary(qkv) and qkv.is_cuda and _only_forward(rotary, Rotary) and _lib.ordinary(rotary.cos, rotary.sin):
-            split = _lib.native().rope_qkv(qkv, rotary.cos, rotary.sin)
+        if _only_forward(rotary, Rotary):
+            cos, sin = rotary.cos, rotary.sin
+            if _lib.ordinary(qkv, cos, sin) and qkv.is_cuda:
+                split = _lib.native().rope_qkv(qkv, cos, sin)
         if split is None:
             q, k, v = qkv.unbind(2)
             q, k = rotary(q), rotary(k)
@@ -456,17 +460,11 @@ class _SlotSiteHIP(torch.autograd.Function):
         return (dq, None, None, None, *dv.unbind(0))
 
 
-def _hip_stacked(v: Tensor, q: Tensor, eps: float) -> Tensor:
-    from .hip_op import block_attn_res_hip
-
-    return block_attn_res_hip(v, q, eps)
-
-
 def _hip_table(sources: list[Tensor], q: Tensor, eps: float) -> Tensor:
     from .table_op import MAX_SOURCES, block_attn_res_sources
 
     if len(sources) > MAX_SOURCES:
-        return _hip_stacked(torch.stack(sources), q, eps)
+        return block_attn_res_hip(torch.stack(sources), q, eps)
     return block_attn_res_sources(sources, q, eps)
 
 
@@ -568,12 +566,16 @@ class Transformer(nn.Module):
     def _queries(self) -> list[Tensor] | None:
         """The sites' queries formed in one launch, where no backward is to come and
         each is the plain product of its factors; None where each site forms its own."""
-        sites = list(self.attn_res)
-        if (self.cfg.residual != "switchyard" or torch.is_grad_enabled()
-                or not all(type(s) is BlockAttnRes and "effective_query" not in s.__dict__ and s.g is not None
-                           and _lib.ordinary(s.w, s.g) for s in sites)):
+        if self.cfg.residual != "switchyard" or torch.is_grad_enabled():
             return None
-        return torch._foreach_mul([s.w for s in sites], [s.g for s in sites])
+        ws, gs = [], []
+        for s in self.attn_res:
+            w, g = s._parameters.get("w"), s._parameters.get("g")
+            if type(s) is not BlockAttnRes or "effective_query" in s.__dict__ or w is None or g is None:
+                return None
+            ws.append(w)
+            gs.append(g)
+        return torch._foreach_mul(ws, gs)
 
     def _site(self, i: int, stream: _Stream, collect_alphas: bool, queries: list[Tensor] | None) -> Tensor:
         cfg = self.cfg
@@ -583,14 +585,14 @@ class Transformer(nn.Module):
         hip = cfg.residual == "switchyard"
         if hip and stream.buf is not None and not torch.is_grad_enabled() and not collect_alphas:
             with self._region("attnres_op"):
-                return _hip_stacked(stream.buf.slots[:n], q, cfg.norm_eps)
+                return block_attn_res_hip(stream.buf.slots[:n], q, cfg.norm_eps)
         if collect_alphas:
             self.last_alphas.append(_mean_alpha(sources, q, cfg.norm_eps))
         if cfg.sources == "stack":
             with self._region("attnres_stage"):
                 v = torch.stack(sources)
             with self._region("attnres_op"):
-                return _hip_stacked(v, q, cfg.norm_eps) if hip else folded_form(v, q, cfg.norm_eps)
+                return block_attn_res_hip(v, q, cfg.norm_eps) if hip else folded_form(v, q, cfg.norm_eps)
         if cfg.sources == "table":
             with self._region("attnres_op"):
                 return _hip_table(sources, q, cfg.norm_eps)
