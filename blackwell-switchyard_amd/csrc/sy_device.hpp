@@ -307,10 +307,11 @@ __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, floa
   return acc;
 }
 
-// A lane's query chunks: packed in the sources' dtype, or (WIDE) as fp32 values
-// when the query has another dtype or a gain. fp32 sources hold any query as fp32
-// chunks.
-template <class T, bool WIDE, int VPL>
+// A lane's query chunks: packed in the sources' dtype, or as fp32 values when the query
+// has another dtype or a gain (kWideQuery), or for bf16 factors as two packed parts
+// (kSplitQuery). fp32 sources hold any query as fp32 chunks.
+enum QueryForm { kPacked = 0, kWideQuery = 1, kSplitQuery = 2 };
+template <class T, int FORM, int VPL>
 struct Query {
   i32x4_t q[VPL];
   __device__ __forceinline__ void load(const void* w, const void* gain, int wt, uint32_t d,
@@ -334,7 +335,7 @@ struct Query {
   }
 };
 template <class T, int VPL>
-struct Query<T, true, VPL> {
+struct Query<T, kWideQuery, VPL> {
   float f[VPL][T::ce];
   __device__ __forceinline__ void load(const void* w, const void* gain, int wt, uint32_t d,
                                        uint32_t lane_off, uint32_t step) {
@@ -345,6 +346,64 @@ struct Query<T, true, VPL> {
   }
   __device__ __forceinline__ float dot_short(const i32x4_t& x, int j, float acc) const {
     return dot_wide<T>(x, f[j], acc);
+  }
+};
+
+// The product of two bf16 factors has at most 16 significant bits: its rounding to bf16
+// and what that leaves are both exact, and two packed dots cost half the operations of
+// one on widened elements. The second part is in LDS, as the registers are full (each
+// thread reads only what it wrote; the opaque index keeps the compiler from holding it).
+template <class T, int VPL, int THREADS>
+struct QuerySplit {
+  static_assert(T::code == BF16::code, "fp16's exponents do not reach its remainders");
+  typedef i32x4_t Lds[VPL][THREADS];
+  i32x4_t hi[VPL];
+  __device__ __forceinline__ void load(Lds& lo, const void* w, const void* gain, int wt, uint32_t d,
+                                       uint32_t lane_off, uint32_t step) {
+    float f[VPL][T::ce];
+    ld_query_row(w, gain, wt, d, lane_off, step, f);
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      hi[j] = pack<T>(f[j]);
+#pragma unroll
+      for (int e = 0; e < T::ce; ++e) f[j][e] -= elem<T>(hi[j], e);
+      lo[j][threadIdx.x] = pack<T>(f[j]);
+    }
+  }
+  __device__ __forceinline__ float dot(const Lds& lo, const i32x4_t& x, int j, float acc) const {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return sy::dot<T>(x, lo[j][t], sy::dot<T>(x, hi[j], acc));
+  }
+};
+
+// A wide query in LDS, for 16-bit tiles whose registers are full: four elements a piece, a
+// lane's pieces `THREADS` apart (a wave's reads are contiguous). Each thread reads only
+// what it wrote, so no barrier is needed.
+template <class T, int VPL, int THREADS>
+struct QueryLds {
+  static constexpr int kPer = T::ce / 4;  // pieces of a chunk
+  i32x4_t s[VPL * kPer][THREADS];
+  __device__ __forceinline__ void load(const void* w, const void* gain, int wt, uint32_t d,
+                                       uint32_t lane_off, uint32_t step) {
+    float f[VPL][T::ce];
+    ld_query_row(w, gain, wt, d, lane_off, step, f);
+#pragma unroll
+    for (int i = 0; i < VPL * kPer; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[i][threadIdx.x][e] = __float_as_int(f[i / kPer][4 * (i % kPer) + e]);
+  }
+  // Chunk j. The opaque index keeps the compiler from reading a chunk once and holding
+  // it, which would take the registers again.
+  __device__ __forceinline__ void chunk(int j, float* f) const {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+#pragma unroll
+    for (int h = 0; h < kPer; ++h) {
+      const i32x4_t x = s[j * kPer + h][t];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * h + e] = __int_as_float(x[e]);
+    }
   }
 };
 

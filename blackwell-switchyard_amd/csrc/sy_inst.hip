@@ -292,8 +292,22 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
   if (tile_is(p, W_, V_, N_)) {                                                              \
     constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
     if (res) {                                                                               \
+      /* 9 rows on more than one wave: see k_fwd_res. */                                     \
+      if constexpr (T::code == BF16::code && W_ > 1 && V_ == 4 && N_ == 9) {                 \
+        if (a.gain != nullptr && a.w_dtype == a.v_dtype) {                                   \
+          static const KernelRes ks =                                                        \
+              resources_of(k_fwd_res<T, W_, V_, N_, false, false, kSplitQuery>, kB);         \
+          const int grid = launch_grid(ks, a.n_tok, kT);                                     \
+          const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * kT);                         \
+          hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, kSplitQuery>), dim3(grid), \
+                             dim3(kB), 0, s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, \
+                             a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, \
+                             n_iter, nullptr, nullptr);                                      \
+          return hipGetLastError();                                                          \
+        }                                                                                    \
+      }                                                                                      \
       static const KernelRes kr =                                                            \
-          resources_of(k_fwd_res<T, W_, V_, N_, false, false, true>, kB);                    \
+          resources_of(k_fwd_res<T, W_, V_, N_, false, false, kWideQuery>, kB);              \
       const int grid = launch_grid(kr, a.n_tok, kT);                                         \
       if (info) {                                                                            \
         *info = kr;                                                                          \
@@ -301,7 +315,7 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
         return hipSuccess;                                                                   \
       }                                                                                      \
       const int n_iter = (int)cdiv(a.n_tok, (int64_t)grid * kT);                             \
-      hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, true>), dim3(grid),         \
+      hipLaunchKernelGGL((k_fwd_res<T, W_, V_, N_, false, false, kWideQuery>), dim3(grid),   \
                          dim3(kB), 0, s, a.v, a.w, a.gain, a.w_dtype, (St*)a.out, a.stats, a.m_out, \
                          a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d, a.eps, inv_d, n_iter, \
                          nullptr, nullptr);                                                  \

@@ -166,7 +166,7 @@ k_fwd(const RowTable v, const void* __restrict__ w,
   const uint32_t row_bytes = (uint32_t)d * sizeof(S);
   const uint32_t lane_off = (uint32_t)(seg * 64 + lane) * 16u;
 
-  Query<T, WIDE, VPL> wq;
+  Query<T, WIDE ? kWideQuery : kPacked, VPL> wq;
   [[maybe_unused]] i32x4_t own = {-1, -1, -1, -1};
   if constexpr (UNAL) {
     static_assert(WIDE, "unaligned rows hold the query as fp32 values");
@@ -523,9 +523,16 @@ k_batched(const RowTable v, const typename T::storage* __restrict__ q,
 // weights carry a different rounding than the two-pass form's, so a token's
 // bits depend on whether it is its wave's last (both within one rounding).
 // WIDE as in k_fwd. Its 9-row four-chunk tiles would take 256-268 VGPRs; they are
-// held to 256, two waves a SIMD like the packed query's (239).
-template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false, bool WIDE = false>
-__global__ void __launch_bounds__(FwdGeom<W>::kBlock, WIDE && VPL == 4 && NR == 9 ? 2 : 1)
+// held to 256, two waves a SIMD like the packed query's (239). On one wave that fits; on
+// more, where the cross-wave sums take registers too, it spilled 8 VGPRs, and waiting for
+// a spilled value also waits for the rows prefetched before it. There the query is in LDS
+// (QueryLds), or for bf16 factors split in two packed parts (QuerySplit: the widened dots'
+// operations lie between a token's loads and the next one's). A no-grad module call with
+// 16-bit factors, us: with the product as a 16-bit tensor / spilled / now, bf16
+// N=9 T=8192 D=4096 115.7 / 124.1 / 117.2, T=4096 D=8192 117.4 / 129.0 / 119.7; fp16
+// 115.1 / 122.4 / 118.6 and 115.6 / 127.0 / 119.1.
+template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false, int QRY = kPacked>
+__global__ void __launch_bounds__(FwdGeom<W>::kBlock, QRY != kPacked && VPL == 4 && NR == 9 ? 2 : 1)
 k_fwd_res(const RowTable v, const void* __restrict__ w,
       const void* __restrict__ gain, int wt,
           typename T::storage* __restrict__ out, float* __restrict__ stats,
@@ -559,8 +566,21 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
   // sits at the use).
   const float* pstat_src = (lane & 1) ? pl : pm;
 
-  Query<T, WIDE, VPL> wq;
-  wq.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
+  constexpr bool kWide = QRY == kWideQuery;
+  constexpr bool kLdsQ = kWide && W > 1 && VPL == 4 && NR == 9;
+  using Lds = QueryLds<T, kLdsQ ? VPL : 1, kLdsQ ? FwdGeom<W>::kBlock : 1>;
+  [[maybe_unused]] __shared__ std::conditional_t<kLdsQ, Lds, char> wl;
+  constexpr bool kSplit = QRY == kSplitQuery;
+  using Split = QuerySplit<BF16, VPL, FwdGeom<W>::kBlock>;
+  [[maybe_unused]] __shared__ std::conditional_t<kSplit, typename Split::Lds, char> lo;
+  [[maybe_unused]] std::conditional_t<kSplit, Split, Query<T, kSplit ? kPacked : QRY, VPL>> wq;
+  if constexpr (kLdsQ) wl.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
+  else if constexpr (kSplit) wq.load(lo, w, gain, wt, (uint32_t)d, lane_off, kStep);
+  else wq.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
+  auto qdot = [&](const i32x4_t& c, int j, float acc) {
+    if constexpr (kSplit) return wq.dot(lo, c, j, acc);
+    else return wq.dot(c, j, acc);
+  };
   i32x4_t x[NR][VPL];
   float pstat = 0.0f;
   {
@@ -611,9 +631,9 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
               float ss = 0.0f, dt = 0.0f;
 #pragma unroll
               for (int j = 0; j < VPL; ++j) {
-                ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
-                dt = wq.dot(x[n][j], j, dt);
-                reconvert<WIDE>(x[n][j]);
+                ss = row_dot<T, kWide>(x[n][j], x[n][j], ss);
+                dt = qdot(x[n][j], j, dt);
+                reconvert<kWide>(x[n][j]);
               }
               const float pv[2] = {ss, dt};
               const float s2 = tsum<2>(pv, lane);  // lanes 0..31: ss, 32..63: dt
@@ -677,18 +697,34 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
       float tv[P];
 #pragma unroll
       for (int i = 0; i < P; ++i) tv[i] = 0.0f;
+      if constexpr (kLdsQ) {  // chunk by chunk: each of the query's is read once a token
 #pragma unroll
-      for (int n = 0; n < NR; ++n) {
-        if (n < opaque(rows)) {
-          float ss = 0.0f, dt = 0.0f;
+        for (int j = 0; j < VPL; ++j) {
+          float q[CE];
+          wl.chunk(j, q);
 #pragma unroll
-          for (int j = 0; j < VPL; ++j) {
-            ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
-            dt = wq.dot(x[n][j], j, dt);
-            reconvert<WIDE>(x[n][j]);
+          for (int n = 0; n < NR; ++n) {
+            if (n < opaque(rows)) {
+              tv[n] = row_dot<T, kWide>(x[n][j], x[n][j], tv[n]);
+              tv[NR + n] = dot_wide<T>(x[n][j], q, tv[NR + n]);
+              reconvert<kWide>(x[n][j]);
+            }
           }
-          tv[n] = ss;
-          tv[NR + n] = dt;
+        }
+      } else {
+#pragma unroll
+        for (int n = 0; n < NR; ++n) {
+          if (n < opaque(rows)) {
+            float ss = 0.0f, dt = 0.0f;
+#pragma unroll
+            for (int j = 0; j < VPL; ++j) {
+              ss = row_dot<T, kWide>(x[n][j], x[n][j], ss);
+              dt = qdot(x[n][j], j, dt);
+              reconvert<kWide>(x[n][j]);
+            }
+            tv[n] = ss;
+            tv[NR + n] = dt;
+          }
         }
       }
       row_sums_transposed<W, 2, NR, TPB, P>(tv, part, 2, rows, red[k & 1], slot, seg, lane);
@@ -699,9 +735,9 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
           float ss = 0.0f, dt = 0.0f;
 #pragma unroll
           for (int j = 0; j < VPL; ++j) {
-            ss = row_dot<T, WIDE>(x[n][j], x[n][j], ss);
-            dt = wq.dot(x[n][j], j, dt);
-            reconvert<WIDE>(x[n][j]);
+            ss = row_dot<T, kWide>(x[n][j], x[n][j], ss);
+            dt = qdot(x[n][j], j, dt);
+            reconvert<kWide>(x[n][j]);
           }
           part[n] = wave_sum(ss);
           part[NR + n] = wave_sum(dt);

@@ -13,6 +13,7 @@ if not torch.cuda.is_available():  # pragma: no cover
     pytest.skip("needs a HIP device", allow_module_level=True)
 
 from oracle.reference import block_attn_res_oracle, dtype_floor, oracle_grads, rel_l2  # noqa: E402
+from switchyard import _lib  # noqa: E402
 from switchyard.triton_op import BlockAttnResTriton  # noqa: E402
 
 DEV = "cuda"
@@ -75,3 +76,34 @@ def test_a_recorded_backward_can_be_differentiated_by_the_factors(wdt):
         dq = dg.double() / mod.w.double()
     for got, want in ((gg, dq), (ww, 2 * dq)):  # dg's rounding, and one of the result
         assert got.dtype == wdt and rel_l2(got, want.cpu()) <= (1e-5 if wdt == F else 1e-2)
+
+
+# Nine-row four-chunk tiles on two, four and eight waves (past the tile rule for few
+# tokens), at full rows and where the last chunks are partial, above and at one token.
+LDS_SHAPES = [(9, 600, 4096), (7, 530, 2312), (9, 520, 8192), (5, 515, 4104), (9, 3, 16384), (6, 1, 8200)]
+
+
+@pytest.mark.parametrize("shape", LDS_SHAPES)
+@pytest.mark.parametrize("dtypes", [(BF, BF), (HF, HF), (BF, F), (HF, BF)])
+def test_queries_held_in_lds(shape, dtypes):
+    """The forward's factors in LDS: fp32 values, or a bf16 product in two exact parts. The
+    logits themselves (the operator's stats) are within fp32 rounding of the exact
+    product's: sums of up to D terms, at most 64 to a lane."""
+    vdt, wdt = dtypes
+    n, t, d = shape
+    print(f"lds query {shape} {dtypes}", flush=True)
+    gen = torch.Generator().manual_seed(d + t)
+    v = torch.randn(n, 1, t, d, generator=gen).to(vdt)
+    w = (torch.randn(d, generator=gen) * d**-0.5).to(wdt)
+    gain = (1 + 0.3 * torch.randn(d, generator=gen)).to(wdt)
+    vd, wd, gd = v.to(DEV), w.to(DEV), gain.to(DEV)
+    out, stats = torch.empty(1, t, d, device=DEV, dtype=vdt), torch.empty(2, n, t, device=DEV)
+    _lib.check(_lib.lib().sy_fwd_gain(vd.data_ptr(), wd.data_ptr(), gd.data_ptr(), out.data_ptr(), stats.data_ptr(),
+                                      n, t, d, t * d, _lib.dtype_code(vdt), _lib.dtype_code(wdt), 1e-6,
+                                      _lib.stream_ptr(vd.device)), "sy_fwd_gain")
+    q = w.double() * gain.double()
+    ref = block_attn_res_oracle(v.double(), q)
+    assert rel_l2(out, ref) <= 1.10 * dtype_floor(ref, vdt)
+    r = torch.rsqrt(v.double().square().mean(-1) + 1e-6)[:, 0]
+    logits = (v.double() @ q)[:, 0] * r
+    assert rel_l2(stats[0], logits) <= 2e-6 and rel_l2(stats[1], r) <= 1e-6
