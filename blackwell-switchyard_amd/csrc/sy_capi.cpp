@@ -425,8 +425,8 @@ int bwd_main_impl(const RowTable& v, bool v_ok, const void* w, const void* g, co
   int grid = 0;
   rc = bwd_grid_for(p, unal, n_src, n_tok, d, v_dtype, w_dtype, stats != nullptr, variant, &grid);
   if (rc != SY_OK) return rc;
-  // A two-factor query may take the generic kernel where the workspace was sized for
-  // the packed one's tile: persistent over tokens, it runs on what there is.
+  // Without stats a two-factor query takes the generic kernel where the workspace was
+  // sized for the packed one's tile: persistent over tokens, it runs on what there is.
   if (gain != nullptr && p.family == SY_FAMILY_GENERIC && workspace != nullptr)
     grid = (int)std::min<int64_t>(grid, workspace_bytes / (d * (int64_t)sizeof(float)));
   if (grid < 1) return SY_ERR_WORKSPACE;
@@ -526,10 +526,12 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
                        int w_dtype, int aligned, sy_plan* out) {
   if (out == nullptr) return SY_ERR_NULL;
   if (n_tok < 0) return SY_ERR_SHAPE;
+  const bool gain = (w_dtype & SY_WITH_GAIN) != 0;
+  w_dtype &= ~SY_WITH_GAIN;
   int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
   bool unal = false;
   if (rc == SY_OK && (op == SY_OP_FWD || op == SY_OP_BWD))
-    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal);
+    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal, 1, 0, gain);
   if (rc != SY_OK || unal) return rc;
   if (op == SY_OP_FWD || op == SY_OP_BWD) apply_tile_rules(op, n_src, n_tok, d, out);
   return SY_OK;

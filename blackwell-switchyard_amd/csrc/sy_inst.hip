@@ -203,6 +203,7 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
   const float inv_d = 1.0f / (float)a.d;
   const int64_t slots = (int64_t)grid * p.tokens_per_block;
   const int n_iter = (int)cdiv(a.n_tok, slots);
+  const bool wide = a.w_dtype != a.v_dtype || a.gain != nullptr;
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
     if (a.stats == nullptr || a.listed || a.gm != nullptr) return hipErrorInvalidConfiguration; \
@@ -220,6 +221,19 @@ hipError_t SY_FN(launch_bwd_vec_)(const sy_plan& p, const BwdArgs& a, int grid, 
 #define X(W_, V_, N_)                                                                        \
   if (tile_is(p, W_, V_, N_)) {                                                              \
     const int var = a.listed ? kBwdListed : (a.gm != nullptr ? kBwdStatsGrad : kBwdStacked); \
+    /* Only with stats does a tile hold a query that is not packed like v; the lean   */     \
+    /* tile does so for the stacked operator gradient.                                */     \
+    constexpr bool lean = W_ == 8 && V_ == 4 && T::ce == 8;                                  \
+    if (wide && (a.stats == nullptr || (lean && var != kBwdStacked))) return hipErrorInvalidConfiguration; \
+    if constexpr (lean) {                                                                    \
+      if (wide) {                                                                            \
+        hipLaunchKernelGGL((k_bwd<T, W_, V_, N_, true, kBwdStacked, false, true>), dim3(grid), \
+                           dim3(BwdGeom<W_, V_>::kBlock), 0, s, a.v, a.w, a.gain, a.w_dtype, \
+                           (const St*)a.g, a.stats, a.gm, a.gl, a.dv, a.partial, a.n_src,    \
+                           a.n_tok, a.d, a.eps, inv_d, n_iter);                              \
+        return hipGetLastError();                                                            \
+      }                                                                                      \
+    }                                                                                        \
     if (a.stats != nullptr) {                                                                \
       if (var == kBwdListed) SY_BWD_LAUNCH(W_, V_, N_, true, kBwdListed);                    \
       else if (var == kBwdStatsGrad) SY_BWD_LAUNCH(W_, V_, N_, true, kBwdStatsGrad);         \

@@ -913,9 +913,14 @@ k_sol_res(const RowTable v, typename T::storage* __restrict__ out, int n_src, in
 // UNAL: rows of any start and length of at least 16 bytes, as in k_fwd (with stats,
 // rows through the table's pointers). With the dw reduction, N=5 T=1023 D=777 fp16:
 // 12.0 us against 46.2 element by element; N=9 T=4096 D=2047 bf16 68 against 430.
+// LDSQ: the lean tile (below) with a query that is not packed like v -- two factors,
+// whose product is never rounded -- kept as fp32 values in LDS, 64 KiB a workgroup.
+// A module's forward + backward, bf16, D=16384 T=1024, us, with the product as a 16-bit
+// tensor / element-wise / so: N=9 251 / 1087 / 226, N=4 105 / 1392 / 102 (43 spilled VGPRs
+// at nine rows, the packed query's tile 59: w's registers are free).
 enum BwdVariant { kBwdStacked = 0, kBwdListed = 1, kBwdStatsGrad = 2 };
 
-template <class T, int W, int VPL, int NR, bool STATS, int VAR, bool UNAL = false>
+template <class T, int W, int VPL, int NR, bool STATS, int VAR, bool UNAL = false, bool LDSQ = false>
 __global__ void __launch_bounds__((BwdGeom<W, VPL, NR>::kBlock))
 k_bwd(const RowTable v, const void* __restrict__ w,
       const void* __restrict__ gain, int wt,
@@ -977,7 +982,12 @@ k_bwd(const RowTable v, const void* __restrict__ w,
   float wf[VPL][CE];
   [[maybe_unused]] i32x4_t wq[VPL];
   [[maybe_unused]] i32x4_t own = {-1, -1, -1, -1};
-  if constexpr (UNAL) {
+  using Lds = QueryLds<T, LDSQ ? VPL : 1, LDSQ ? 64 * W : 1>;
+  [[maybe_unused]] __shared__ std::conditional_t<LDSQ, Lds, char> wl;
+  if constexpr (LDSQ) {
+    static_assert(STATS && kLean, "the other tiles hold any query as fp32 copies");
+    wl.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
+  } else if constexpr (UNAL) {
     static_assert(STATS && !kLean, "unaligned rows: with the forward's stats");
 #pragma unroll
     for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, gain, lane_off + j * kStep, row_bytes, wt, wf[j]);
@@ -1189,13 +1199,22 @@ k_bwd(const RowTable v, const void* __restrict__ w,
             // Lean tiles widen w and grad_out again for every row: opaque
             // copies of the packed words keep the compiler from hoisting the
             // conversions out of the loops, which would rebuild the fp32 copies.
-            i32x4_t wj = wq[j], gj = gk[j];
-            asm volatile("" : "+v"(wj), "+v"(gj));
+            i32x4_t gj = gk[j];
+            asm volatile("" : "+v"(gj));
+            float wj[CE];
+            if constexpr (LDSQ) {
+              wl.chunk(j, wj);
+            } else {
+              i32x4_t wp = wq[j];
+              asm volatile("" : "+v"(wp));
+#pragma unroll
+              for (int e = 0; e < CE; ++e) wj[e] = elem<T>(wp, e);
+            }
 #pragma unroll
             for (int e = 0; e < CE; ++e) {
               float xv = elem<T>(x[n][j], e);
               if constexpr (T::code == F16::code) asm volatile("" : "+v"(xv));
-              f[e] = fmaf(c, xv, fmaf(da, elem<T>(wj, e), al[n] * elem<T>(gj, e)));
+              f[e] = fmaf(c, xv, fmaf(da, wj[e], al[n] * elem<T>(gj, e)));
               dwa[j][e] = fmaf(da_w, xv, dwa[j][e]);
             }
           } else {

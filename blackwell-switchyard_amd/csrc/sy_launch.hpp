@@ -260,6 +260,9 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
 //    1024 chunks; the backward with stats, up to 16 sources and not for the (o, m, l)
 //    gradient. N=5 T=1023 D=777 fp16: forward 18.0 -> 6.4 us, backward 46.2 -> 12.0.
 // A query given as two factors (`gain`) is held as fp32 values too, whatever its dtype.
+// On that eight-wave tile it is held in LDS, for factors of the sources' dtype, whose
+// rounded product ran the tile before the kernels formed it: N=9 T=1024 D=16384 forward +
+// backward 251 us with the rounded product, 1087 on the generic kernel, 226 so.
 // `variant` as in bwd_plan (backward only).
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
                      sy_plan* out, bool* unal, int has_stats = 1, int variant = 0, bool gain = false);

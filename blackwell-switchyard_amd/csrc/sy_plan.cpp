@@ -255,6 +255,7 @@ int make_plan(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_
 int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype, int aligned,
                      sy_plan* out, bool* unal, int has_stats, int variant, bool gain) {
   *unal = false;
+  const bool same = v_dtype == w_dtype;
   if (gain) w_dtype = v_dtype == SY_F32 ? SY_BF16 : SY_F32;  // plans as another dtype does
   const int rc = make_plan(op, n_src, 0, d, v_dtype, w_dtype, aligned, out, has_stats);
   if (rc != SY_OK || out->family != SY_FAMILY_GENERIC) return rc;
@@ -266,7 +267,7 @@ int make_launch_plan(int op, int64_t n_src, int64_t d, int v_dtype, int w_dtype,
     if (make_plan(op, n_src, 0, d, v_dtype, v_dtype, aligned, &q, has_stats) != SY_OK) return rc;
     const bool packed = op == SY_OP_BWD && q.elems_per_chunk == 8 && q.waves_per_token == 8 &&
                         q.chunks_per_lane == 4;
-    if (!packed) *out = q;
+    if (!packed || (gain && same && variant == 0)) *out = q;
     return rc;
   }
   const int64_t e = (d + ce - 1) / ce;

@@ -120,10 +120,12 @@ int sy_plan_for(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int 
 /* sy_plan_for for a launch of n_tok tokens on the current device: for the
  * forward and the backward, the tile sy_fwd / sy_bwd run, with the token-count
  * rule and any sy_tuning_set tile override applied; other ops as
- * sy_plan_for. Without a device the token-count rule is skipped. No
+ * sy_plan_for. w_dtype | SY_WITH_GAIN asks for sy_fwd_gain / sy_bwd_gain.
+ * Without a device the token-count rule is skipped. No
  * counterpart in the reference, whose launch configuration ignores the token
  * count (src/switchyard/triton_op.py:130-150); it serves benchmarks and
  * callers that report the launched tile. */
+#define SY_WITH_GAIN 0x100
 int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int v_dtype,
                        int w_dtype, int aligned, sy_plan* out);
 

@@ -427,3 +427,16 @@ def test_tuning_rejects_out_of_range_values(field, val):
     assert _lib.lib().sy_tuning_get(ctypes.byref(got)) == OK
     assert getattr(got, field) == 0
     assert _lib.lib().sy_tuning_get(None) == NULL
+
+
+@pytest.mark.parametrize("n,rows", [(2, 4), (4, 4), (5, 9), (9, 9)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_gain_keeps_the_widest_rows_tile(n, rows, dtype):
+    """The rounded product of two 16-bit factors runs the eight-wave tile; so do the factors."""
+    for d in (8200, 16384):
+        p = _lib.plan(_lib.OP_BWD, n, d, dtype, n_tok=2048, gain=True)
+        assert (p["family_name"], p["waves_per_token"], p["chunks_per_lane"], p["rows_per_tile"]) == ("resident", 8, 4, rows)
+        assert p == _lib.plan(_lib.OP_BWD, n, d, dtype, n_tok=2048)
+    # a query of another dtype has no tile there, with or without a gain
+    for gain in (False, True):
+        assert _lib.plan(_lib.OP_BWD, n, 16384, dtype, w_dtype=torch.float32, n_tok=2048, gain=gain)["family_name"] == "generic"

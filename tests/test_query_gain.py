@@ -107,3 +107,26 @@ def test_queries_held_in_lds(shape, dtypes):
     r = torch.rsqrt(v.double().square().mean(-1) + 1e-6)[:, 0]
     logits = (v.double() @ q)[:, 0] * r
     assert rel_l2(stats[0], logits) <= 2e-6 and rel_l2(stats[1], r) <= 1e-6
+
+
+@pytest.mark.parametrize("shape", [(9, 300, 8200), (4, 270, 16384), (5, 2, 12288), (2, 300, 8200)])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_gradients_of_the_widest_rows(shape, dtype):
+    """The eight-wave tile with the factors in LDS: one and two tokens a workgroup, partial
+    last chunks. Held to the floor of one rounding, which a rounded product does not meet."""
+    n, t, d = shape
+    print(f"widest rows {shape} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(d + t)
+    v = torch.randn(n, 1, t, d, generator=gen).to(dtype)
+    w = (torch.randn(d, generator=gen) * d**-0.5).to(dtype)
+    gain = (1 + 0.3 * torch.randn(d, generator=gen)).to(dtype)
+    go = torch.randn(1, t, d, generator=gen).to(dtype)
+    mod = BlockAttnResTriton(d).to(DEV).to(dtype)
+    with torch.no_grad():
+        mod.w.copy_(w)
+        mod.g.copy_(gain)
+    vv = v.to(DEV).requires_grad_()
+    dv, dw, dg = torch.autograd.grad(mod(vv), [vv, mod.w, mod.g], go.to(DEV))
+    rdv, rdq = oracle_grads(v.double(), w.double() * gain.double(), go.double())
+    for got, want in ((dv, rdv), (dw, rdq * gain.double()), (dg, rdq * w.double())):
+        assert rel_l2(got, want) <= 1.10 * dtype_floor(want, dtype)
