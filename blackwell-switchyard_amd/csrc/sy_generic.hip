@@ -52,6 +52,9 @@ __device__ float block_max(float x, float* scr) {
 // Pass 1 for one token: per-row (sum of squares, query dot[, grad dot]) for
 // every row, written to ss[], qd[] and gd[] in LDS. Rows go in groups of 8 so
 // a thread carries 16-24 partial sums.
+// GAIN: the query is w * gain, elsewhere gain is not looked at (a branch and a product an
+// element cost the other callers 1-3%: N=40 T=1024 D=4096 forward + backward GENT).
+template <bool GAIN>
 __device__ void row_scalars(const RowTable& v, const void* w, const void* gain, const void* g,
                             int n_src, int64_t tok, int d, int vt, int wt, float* ss, float* qd, float* gd,
                             float* scr) {
@@ -64,7 +67,8 @@ __device__ void row_scalars(const RowTable& v, const void* w, const void* gain, 
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = b[r] = c[r] = 0.0f;
     for (int k = tid; k < d; k += kBlock) {
-      const float wk = load_elem(w, k, wt) * (gain ? load_elem(gain, k, wt) : 1.0f);
+      float wk = load_elem(w, k, wt);
+      if constexpr (GAIN) wk *= load_elem(gain, k, wt);
       const float gk = g ? load_elem(g, tok * d + k, vt) : 0.0f;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -107,6 +111,7 @@ __device__ void row_scalars(const RowTable& v, const void* w, const void* gain, 
 }
 
 // LDS layout (floats): [0, n) lg, [n, 2n) ss/r, [2n, 3n) gd, then 257 scratch.
+template <bool GAIN>
 __global__ void __launch_bounds__(kBlock)
 k_fwd_generic(const RowTable v, const void* __restrict__ w, const void* __restrict__ gain,
               void* __restrict__ out,
@@ -119,7 +124,7 @@ k_fwd_generic(const RowTable v, const void* __restrict__ w, const void* __restri
   float* scr = sh + 2 * n_src;
   const int tid = threadIdx.x;
   const int64_t tok = blockIdx.x;
-  row_scalars(v, w, gain, nullptr, n_src, tok, d, vt, wt, ss, lg, nullptr, scr);
+  row_scalars<GAIN>(v, w, gain, nullptr, n_src, tok, d, vt, wt, ss, lg, nullptr, scr);
 
   float m = -INFINITY;
   for (int n = tid; n < n_src; n += kBlock) {
@@ -167,6 +172,7 @@ k_sol_generic(const RowTable v, void* __restrict__ out, int n_src, int64_t n_tok
 // Persistent over tokens; workgroup b accumulates its dw contribution in its
 // own fp32 row partial[b][:] (no other workgroup touches it). gm != nullptr
 // selects the gradient of the unnormalised (o, m, l) triple, as in k_bwd.
+template <bool GAIN>
 __global__ void __launch_bounds__(kBlock)
 k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restrict__ gain,
               const void* __restrict__ g,
@@ -183,7 +189,7 @@ k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restri
   for (int k = tid; k < d; k += kBlock) prow[k] = 0.0f;
 
   for (int64_t tok = blockIdx.x; tok < n_tok; tok += gridDim.x) {
-    row_scalars(v, w, gain, g, n_src, tok, d, vt, wt, da, al, gc, scr);
+    row_scalars<GAIN>(v, w, gain, g, n_src, tok, d, vt, wt, da, al, gc, scr);
     float m = -INFINITY;
     for (int n = tid; n < n_src; n += kBlock) {
       const float r = rsqrtf(fmaf(da[n], inv_d, eps));
@@ -237,7 +243,8 @@ k_bwd_generic(const RowTable v, const void* __restrict__ w, const void* __restri
     __syncthreads();
     for (int k = tid; k < d; k += kBlock) {
       const float gk = load_elem(g, tok * d + k, vt);
-      const float wk = load_elem(w, k, wt) * (gain ? load_elem(gain, k, wt) : 1.0f);
+      float wk = load_elem(w, k, wt);
+      if constexpr (GAIN) wk *= load_elem(gain, k, wt);
       float dwk = 0.0f;
       for (int n = 0; n < n_src; ++n) {
         const float x = load_elem(row_of<const char>(v, n), tok * d + k, vt);
@@ -281,7 +288,7 @@ k_bwd_batched_generic(const RowTable v, const void* __restrict__ q, const void* 
     for (int s = 0; s < n_q; ++s) {
       const char* qs = static_cast<const char*>(q) + (int64_t)s * d * es;
       const char* gs = static_cast<const char*>(g) + (int64_t)s * n_tok * d * es;
-      row_scalars(v, qs, nullptr, gs, nn, tok, d, vt, vt, ss, qd, gd, scr);
+      row_scalars<false>(v, qs, nullptr, gs, nn, tok, d, vt, vt, ss, qd, gd, scr);
       float m = -INFINITY;
       for (int n = tid; n < nn; n += kBlock) {
         const float r = rsqrtf(fmaf(ss[n], inv_d, eps));
@@ -505,7 +512,7 @@ k_probe_mix(const char* __restrict__ src, char* __restrict__ dst, int64_t out_by
 
 hipError_t launch_fwd_generic(const FwdArgs& a, hipStream_t s) {
   const size_t lds = (size_t)(2 * a.n_src + 257) * sizeof(float);
-  hipLaunchKernelGGL(k_fwd_generic, dim3((unsigned)a.n_tok), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.out,
+  hipLaunchKernelGGL(a.gain != nullptr ? k_fwd_generic<true> : k_fwd_generic<false>, dim3((unsigned)a.n_tok), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.out,
                      a.stats, a.m_out, a.l_out, a.normalize, a.n_src, a.stat_rows(), a.n_tok, a.d,
                      a.v_dtype, a.w_dtype, a.eps, 1.0f / (float)a.d);
   return hipGetLastError();
@@ -519,7 +526,7 @@ hipError_t launch_sol_generic(const FwdArgs& a, hipStream_t s) {
 
 hipError_t launch_bwd_generic(const BwdArgs& a, int grid, hipStream_t s) {
   const size_t lds = (size_t)(3 * a.n_src + 257) * sizeof(float);
-  hipLaunchKernelGGL(k_bwd_generic, dim3(grid), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.g, a.gm, a.gl,
+  hipLaunchKernelGGL(a.gain != nullptr ? k_bwd_generic<true> : k_bwd_generic<false>, dim3(grid), dim3(kBlock), lds, s, a.v, a.w, a.gain, a.g, a.gm, a.gl,
                      a.dv, a.partial, a.n_src, a.n_tok, a.d, a.v_dtype, a.w_dtype, a.eps,
                      1.0f / (float)a.d);
   return hipGetLastError();
