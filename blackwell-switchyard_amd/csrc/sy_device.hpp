@@ -295,6 +295,41 @@ __device__ __forceinline__ void ld_query_row(const void* w, const void* gain, in
     ld_query_of(w, gain, false, false, d, lane_off, step, f);
 }
 
+// The same where the query mostly has the sources' dtype and no gain: that one is loaded
+// first, as packed words, and all others out of line. Behind their branches its loads were
+// waited for before the first rows were asked for, and the launch's code was longer to
+// fetch (fp32 N=6 T=1430 D=512 forward 6.0 -> 6.6 us, backward 8.9 -> 9.4; forward +
+// backward 22.5 so, 21.3 now and without any of them. Loads without branches, finished
+// after the first rows are asked for, took 22.8).
+// An fp32 query stays in the words it was loaded to (no copies, which would wait for it).
+template <class T, int VPL>
+__device__ __forceinline__ void ld_query(const void* w, const void* gain, int wt, uint32_t d,
+                                         uint32_t lane_off, uint32_t step, float (&f)[VPL][T::ce]) {
+  constexpr bool kF32 = T::code == F32::code;
+  i32x4_t q[VPL];
+  if (__builtin_expect(gain == nullptr && wt == T::code, 1)) {
+    const auto r = make_rsrc(w, d * (uint32_t)sizeof(typename T::storage));
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) q[j] = ld16(r, lane_off + j * step);
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+#pragma unroll
+      for (int e = 0; e < (kF32 ? 0 : T::ce); ++e) f[j][e] = elem<T>(q[j], e);
+  } else {
+    ld_query_row(w, gain, wt, d, lane_off, step, f);
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+#pragma unroll
+      for (int e = 0; e < (kF32 ? 4 : 0); ++e) q[j][e] = __float_as_int(f[j][e]);
+  }
+  if constexpr (kF32) {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[j][e] = __int_as_float(q[j][e]);
+  }
+}
+
 // acc + sum_e x[e] * f[e] with an fp32 query chunk.
 template <class T>
 __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, float acc) {
@@ -318,7 +353,7 @@ struct Query {
                                        uint32_t lane_off, uint32_t step) {
     if constexpr (T::code == F32::code) {
       float f[VPL][4];
-      ld_query_row(w, gain, wt, d, lane_off, step, f);
+      ld_query<T>(w, gain, wt, d, lane_off, step, f);
 #pragma unroll
       for (int j = 0; j < VPL; ++j) q[j] = pack<T>(f[j]);
     } else {

@@ -993,7 +993,7 @@ k_bwd(const RowTable v, const void* __restrict__ w,
     for (int j = 0; j < VPL; ++j) ld_query_any<CE>(w, gain, lane_off + j * kStep, row_bytes, wt, wf[j]);
     own = tail_mask(lane_off + (VPL - 1) * kStep, row_bytes);
   } else if constexpr (STATS && !kLean) {
-    ld_query_row(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
+    ld_query<T>(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
   } else {
     const auto wr = make_rsrc(w, row_bytes);
 #pragma unroll
@@ -1346,7 +1346,7 @@ k_bwd_tall(const RowTable v, const void* __restrict__ w,
   const int iters = n_iter;  // every slot meets the same barriers
 
   float wf[VPL][CE];
-  ld_query_row(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
+  ld_query<T>(w, gain, wt, (uint32_t)d, lane_off, kStep, wf);
   float dwa[VPL][CE];
 #pragma unroll
   for (int j = 0; j < VPL; ++j)
