@@ -295,6 +295,35 @@ class _TwoPhase(torch.autograd.Function):
         return dv, dw, None, None
 
 
+def _by_groups(v: torch.Tensor, w: torch.Tensor, split: int) -> bool:
+    """Whether a training call differentiates the two phases instead of running one
+    backward over all sources: where that one has no register tile but both groups'
+    have, or all sources are more than it takes. Both sides measured, bf16 forward +
+    backward on the device, groups / one, us: N=32 D=8192 T=64 201 / 913, T=2048
+    2352 / 3059; N=16 D=16384 T=512 764 / 1347; N=17 D=4160 T=512 268 / 373; N=24
+    D=512 T=8192 561 / 580, T=16384 1042 / 1139; N=17 D=128 T=8192 206 / 242, T=16384
+    337 / 460. Launched one by one, the groups' fifteen operations take the host
+    420-570 us, which one backward undercuts below the token counts here (N=17
+    D=4160 T=64 425 / 191, N=24 D=512 T=2048 552 / 155). fp32 rows gain nothing
+    (N=20 D=4096 T=1024 763 / 588)."""
+    n, b, t, d = v.shape
+    if not (torch.is_grad_enabled() and (v.requires_grad or w.requires_grad)) or n <= 9 or not v.is_cuda:
+        return False
+    if n > 4096:  # sources of one element-wise launch
+        return split <= 4096 and n - split <= 4096
+    if d > 4096:
+        few = b * t < 512 and n * d < 1 << 17
+    else:
+        few = d > 512 or b * t <= 8192
+    if few or n > 32 or max(split, n - split) > 16 or v.dtype == torch.float32 or w.dtype != v.dtype:
+        return False
+
+    def tiled(rows: int) -> bool:
+        return _lib.plan(_lib.OP_BWD, rows, d, v.dtype)["family_name"] != "generic"
+
+    return not tiled(n) and tiled(split) and tiled(n - split)
+
+
 def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: float = DEFAULT_EPS):
     """The two-phase schedule for one query: sources ``[0, split)`` reduced to
     their ``(o, m, l)``, then sources ``[split, N)`` reduced and merged with
@@ -305,6 +334,8 @@ def block_attn_res_two_phase(v: torch.Tensor, w: torch.Tensor, split: int, eps: 
     if not 0 < split < n:
         raise ValueError(f"split must be in (0, {n}), got {split}")
     split = operator.index(split)  # a fraction is no source index
+    if _by_groups(v, w, split):
+        return attn_with_stats_merge(v[split:], w, *attn_with_stats(v[:split], w, eps), eps=eps)[0]
     if _lib.ordinary(v, w):
         out = _lib.native().block_attn_res_two_phase(v, w, split, float(eps))
         if out is not None:
