@@ -796,7 +796,7 @@ def batched_sweep(args, results, failed):
             check[f"out[{k}]"] = _gate(tag, s0["out"][k], ref)
         worst = max(check.values(), key=lambda c: c["rel_l2"])
         check = {"queries": q, "ok": all(c["ok"] for c in check.values()), "worst": worst}
-        plan = _lib.plan(_lib.OP_BATCHED, n, d, dt, n_q=q)
+        plan = _lib.plan(_lib.OP_BATCHED, n, d, dt, n_q=q, n_tok=b * t)
         config3 = (n, b, t, d) == (9, 1, 4096, 2048)
         rec = {"sweep": ("batched" if q == 8 else "batched-q") if config3 else "batched-shape",
                "impl": "switchyard_hip", "N": n, "B": b, "T": t, "D": d, "Q": q, "dtype": tag,

@@ -456,6 +456,23 @@ int bwd_impl(const RowTable& v, bool v_ok, const void* w, const void* g, const f
   return status(launch_dw_reduce((const float*)workspace, rows, (int)d, dw, w_dtype, s, w, gain, dgain));
 }
 
+// The batched forward's plan for a launch.
+int batched_plan(int64_t n_src, int64_t n_q, int64_t n_tok, int64_t d, int dtype, int aligned,
+                 sy_plan* p) {
+  const int rc = make_plan(SY_OP_BATCHED, n_src, n_q, d, dtype, dtype, aligned, p);
+  if (rc != SY_OK) return rc;
+  apply_tile_override(SY_OP_BATCHED, n_src, d, p);
+  // The matrix kernel's store offsets are 32-bit; past that, per-query launches.
+  if (p->family == SY_FAMILY_MATRIX && !matrix_batched_offsets_fit(n_q, n_tok, d))
+    p->family = SY_FAMILY_PER_QUERY;
+  int cus = 0;
+  if (cu_count(&cus) != hipSuccess) cus = 1;
+  sy_tuning forced;  // a measurement override of the register tile is kept
+  const bool tile = tuning_snapshot(&forced) && forced.batched_tile[0] != 0;
+  if (!tile && batched_any_wanted(*p, n_src, n_q, n_tok, d, dtype, cus)) p->family = SY_FAMILY_STREAM;
+  return SY_OK;
+}
+
 // Batched forward: the resident kernel, else one forward launch per query
 // written straight into out[q] (and m_out[q], l_out[q]).
 int batched_impl(const RowTable& v, bool v_ok, const void* q, void* out, float* m_out, float* l_out,
@@ -463,18 +480,10 @@ int batched_impl(const RowTable& v, bool v_ok, const void* q, void* out, float* 
                  float eps, hipStream_t s) {
   const bool aligned = vec_rows(v_ok, d, dtype) && al16(q) && al16(out);
   sy_plan p;
-  int rc = make_plan(SY_OP_BATCHED, n_src, n_q, d, dtype, dtype, aligned, &p);
+  int rc = batched_plan(n_src, n_q, n_tok, d, dtype, aligned, &p);
   if (rc != SY_OK) return rc;
-  apply_tile_override(SY_OP_BATCHED, n_src, d, &p);
   if (n_tok == 0) return SY_OK;
-  // The matrix kernel's store offsets are 32-bit; past that, per-query launches.
-  if (p.family == SY_FAMILY_MATRIX && !matrix_batched_offsets_fit(n_q, n_tok, d))
-    p.family = SY_FAMILY_PER_QUERY;
-  int cus = 0;
-  if (cu_count(&cus) != hipSuccess) cus = 1;
-  sy_tuning forced;  // a measurement override of the register tile is kept
-  const bool tile = tuning_snapshot(&forced) && forced.batched_tile[0] != 0;
-  if (!tile && batched_any_wanted(p, n_src, n_q, n_tok, d, dtype, cus)) {
+  if (p.family == SY_FAMILY_STREAM) {
     const BatchedArgs a{v,          q,        out,   m_out,  l_out, normalize,
                         (int)n_src, (int)n_q, n_tok, (int)d, dtype, eps};
     return status(launch_batched_any(a, s));
@@ -528,6 +537,13 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
   if (n_tok < 0) return SY_ERR_SHAPE;
   const bool gain = (w_dtype & SY_WITH_GAIN) != 0;
   w_dtype &= ~SY_WITH_GAIN;
+  if (op == SY_OP_BATCHED) return batched_plan(n_src, n_q, n_tok, d, v_dtype, aligned, out);
+  if (op == SY_OP_BWD_BATCHED) {
+    const int rc = bwd_batched_plan(n_src, n_q, n_tok, d, v_dtype, aligned, n_tok * d * esize(v_dtype), out);
+    if (rc == SY_OK && aligned && two_pass_wanted(*out, n_src, n_q, n_tok, d, v_dtype))
+      out->family = SY_FAMILY_TWO_PASS;
+    return rc;
+  }
   int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
   bool unal = false;
   if (rc == SY_OK && (op == SY_OP_FWD || op == SY_OP_BWD))

@@ -21,7 +21,7 @@ LIB_PATH = pathlib.Path(__file__).resolve().parent / "libswitchyard_hip.so"
 SY_F32, SY_F16, SY_BF16 = 0, 1, 2
 OP_FWD, OP_BWD, OP_BATCHED, OP_SOL, OP_BWD_BATCHED = 0, 1, 2, 3, 4
 WITH_GAIN = 0x100  # SY_WITH_GAIN
-FAMILY_NAMES = {0: "resident", 1: "chunked", 2: "generic", 3: "per_query", 4: "matrix"}
+FAMILY_NAMES = {0: "resident", 1: "chunked", 2: "generic", 3: "per_query", 4: "matrix", 5: "stream", 6: "two_pass"}
 
 _DTYPE_CODES = {torch.float32: SY_F32, torch.float16: SY_F16, torch.bfloat16: SY_BF16}
 
@@ -199,7 +199,7 @@ def plan(op: int, n_src: int, d: int, dtype: torch.dtype, *, n_q: int = 0,
     """The execution plan the library picks for a shape (pure host arithmetic).
     With ``n_tok``, the tile a launch of that many tokens runs on the current
     device (``sy_plan_for_tokens``: the forward and backward also depend on
-    the token count); then ``gain`` asks for the launch of a query with a gain."""
+    the token count, the batched ops have two families more); then ``gain`` asks for the launch of a query with a gain."""
     p = Plan()
     if n_tok is None:
         rc = lib().sy_plan_for(op, n_src, n_q, d, dtype_code(dtype), dtype_code(w_dtype or dtype),

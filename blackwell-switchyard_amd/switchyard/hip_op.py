@@ -225,10 +225,13 @@ def block_attn_res_batched_train(
     The reference's batched API is output-only and raises under autograd
     (triton_op.py:463-467, kept as is in ``block_attn_res_batched``); this is
     its training contract. Forward: the same single read of ``v`` for all
-    queries. Backward: one persistent kernel reads ``v`` and the ``S``
-    output gradients once, writes ``dv = sum_s dv_s`` rounded once and fp32
-    per-workgroup ``dq`` partials, then the fixed-order reduction writes
-    ``dq`` -- two kernels, bit-reproducible.
+    queries. Backward: ``dv = sum_s dv_s`` rounded once and fp32 per-workgroup
+    ``dq`` partials, then the fixed-order reduction writes ``dq``;
+    bit-reproducible. On the matrix cores (16-bit D of 512 to 2048) and on the
+    register tile (few queries) one persistent kernel reads ``v`` and the ``S``
+    output gradients once; other shapes of whole 16-byte chunks, up to 16
+    sources and queries, read them twice, first for every token's coefficients
+    (``sy_plan_for_tokens``: ``two_pass``); the rest run element-wise.
     """
     if _lib.ordinary(v, queries):
         out = _lib.native().block_attn_res_batched_train(v, queries, float(eps))
@@ -244,9 +247,13 @@ def block_attn_res_batched(
 
     Same contract as the reference's ``block_attn_res_batched``
     (triton_op.py:438-501): ``out[s] == block_attn_res_triton(v, queries[s])``,
-    ``[S, B, T, D]``, no backward. For N, D, dtype the resident kernel holds
-    and S <= 16 one kernel reads ``v`` once; other shapes issue one forward
-    launch per query, written straight into ``out[s]`` (no stack).
+    ``[S, B, T, D]``, no backward. One kernel reads ``v`` once from memory: on
+    the matrix cores, on the register tile, or (up to 16 sources and queries,
+    rows of any start and width of at least 16 bytes) with matrix products
+    straight from the rows, which it reads again from cache
+    (``sy_plan_for_tokens``: ``stream``). Other shapes, and one or two queries
+    without a tile, issue one forward launch per query, written straight into
+    ``out[s]`` (no stack).
     """
     if _lib.ordinary(v, queries):
         out = _lib.native().block_attn_res_batched(v, queries, float(eps))

@@ -77,8 +77,12 @@ typedef enum sy_family {
   SY_FAMILY_CHUNKED = 1,   /* register tile of NR rows, online softmax over chunks */
   SY_FAMILY_GENERIC = 2,   /* element-wise loads, two passes per token             */
   SY_FAMILY_PER_QUERY = 3, /* batched op answered by one forward launch per query  */
-  SY_FAMILY_MATRIX = 4     /* batched op on the matrix cores: 4 waves per token,
+  SY_FAMILY_MATRIX = 4,    /* batched op on the matrix cores: 4 waves per token,
                               [N, D] staged in LDS, queries in registers         */
+  /* Reported by sy_plan_for_tokens only; the tile fields are then not meant:      */
+  SY_FAMILY_STREAM = 5,    /* batched forward, rows of any start straight from
+                              memory into matrix products                        */
+  SY_FAMILY_TWO_PASS = 6   /* batched backward: coefficients, then their products  */
 } sy_family;
 
 /* How a call will be executed: which kernel family and which compile-time tile.
@@ -110,8 +114,8 @@ typedef struct sy_plan {
  * some shapes reported as generic, per-query or resident launch a faster kernel
  * with the same results: a query of another dtype, rows that start at no
  * 16-byte boundary or have an odd D, and batched shapes outside the matrix
- * tiles; sy_kernel_info and sy_plan_for_tokens report
- * the launched tile, this function, having no token count, does not.
+ * tiles. sy_plan_for_tokens reports what is launched (sy_kernel_info too, for
+ * the forward and the backward); this function, having no token count, does not.
  * Replaces the dispatch helpers _launch_config, _bwd_launch and
  * _batched_launch (src/switchyard/triton_op.py:130-150, :267-276, :420-435). */
 int sy_plan_for(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int w_dtype,
@@ -119,7 +123,8 @@ int sy_plan_for(int op, int64_t n_src, int64_t n_q, int64_t d, int v_dtype, int 
 
 /* sy_plan_for for a launch of n_tok tokens on the current device: for the
  * forward and the backward, the tile sy_fwd / sy_bwd run, with the token-count
- * rule and any sy_tuning_set tile override applied; other ops as
+ * rule and any sy_tuning_set tile override applied; for the batched ops the
+ * family sy_fwd_batched / sy_bwd_batched run, sources n_tok * d apart; others as
  * sy_plan_for. w_dtype | SY_WITH_GAIN asks for sy_fwd_gain / sy_bwd_gain.
  * Without a device the token-count rule is skipped. No
  * counterpart in the reference, whose launch configuration ignores the token

@@ -14,6 +14,7 @@ if not torch.cuda.is_available():  # pragma: no cover
 
 from oracle import c_oracle  # noqa: E402
 from oracle.reference import dtype_floor, rel_l2  # noqa: E402
+from switchyard import _lib  # noqa: E402
 from switchyard.hip_op import block_attn_res_batched  # noqa: E402
 from switchyard.stats_op import block_attn_res_batched_with_stats  # noqa: E402
 
@@ -75,3 +76,13 @@ def test_misaligned_buffers_and_guards(dtype):
     ref = torch.from_numpy(c_oracle.batched(v[:, 0].double().numpy(), q.double().numpy()))
     assert rel_l2(out[: s * t * d].view(s, t, d).cpu(), ref) <= _bar(ref, dtype)
     assert bool((buf[:31] == 7).all()) and bool((buf[31 + s * t * d:] == 7).all())
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("dtype", [BF, HF, F])
+def test_what_is_launched(case, dtype):
+    n, s, t, d = case
+    few = {(1, 8, 12, 320), (16, 1, 21, 63)}  # too few pairs, too few queries
+    tiles = {(9, 8, 1500, 256), (9, 8, 70, 2560), (9, 16, 65, 8)}  # fp32 of up to nine rows
+    family = _lib.plan(_lib.OP_BATCHED, n, d, dtype, n_q=s, n_tok=t)["family_name"]
+    assert (family == "stream") == (case not in few and not (dtype == F and case in tiles))

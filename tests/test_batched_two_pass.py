@@ -15,6 +15,7 @@ if not torch.cuda.is_available():  # pragma: no cover
 
 from oracle import c_oracle  # noqa: E402
 from oracle.reference import dtype_floor, rel_l2  # noqa: E402
+from switchyard import _lib  # noqa: E402
 from switchyard.hip_op import block_attn_res_batched_train  # noqa: E402
 
 DEV = "cuda"
@@ -47,3 +48,47 @@ def test_two_pass_batched_backward(case, dtype):
         assert not dq.any()
     else:
         assert rel_l2(dq, rdq) <= bar(rdq)
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("dtype", [BF, HF, F])
+def test_what_is_launched(case, dtype):
+    n, s, t, d = case
+    few = {(1, 8, 12, 320), (2, 1, 700, 64), (9, 3, 65, 8)}  # few queries keep the register tile,
+    small = {(4, 4, 37, 4096), (5, 5, 1, 2056)}  # 16-bit ones also at few tokens
+    family = _lib.plan(_lib.OP_BWD_BATCHED, n, d, dtype, n_q=s, n_tok=t)["family_name"]
+    assert (family == "two_pass") == (case not in few and not (dtype != F and case in small))
+
+
+def test_a_workspace_too_small_for_two_passes():
+    """A source stride past the matrix kernel's offsets, with the workspace sized for that
+    kernel, runs the register tile (at this many tokens the coefficients do not fit); with
+    room for them two passes; with room for neither it is refused. Nothing is written past
+    the workspace."""
+    n, s, t, d = 9, 8, 7000, 512
+    stride = 400 << 20  # elements; the matrix kernel adds three to a 31-bit byte offset
+    gen = torch.Generator().manual_seed(1)
+    v, q = torch.randn(n, t, d, generator=gen).to(BF), (torch.randn(s, d, generator=gen) * 2.0 / d**0.5).to(BF)
+    g = torch.randn(s, t, d, generator=gen).to(BF)
+    buf = torch.empty((n - 1) * stride + t * d, device=DEV, dtype=BF)
+    for k in range(n):
+        buf[k * stride : k * stride + t * d].copy_(v[k].flatten())
+    qd, gd = q.to(DEV), g.to(DEV)
+    need = _lib.lib().sy_bwd_batched_workspace_bytes(n, s, t, d, _lib.dtype_code(BF))
+    rdv, rdq = (torch.from_numpy(x) for x in c_oracle.batched_backward(*[x.double().numpy() for x in (v, q, g)]))
+    got = []
+    for size in (64 << 20, need, s * d * 4 - 16):
+        print(f"two-pass workspace {size}", flush=True)
+        dv, dq = torch.empty(n, t, d, device=DEV, dtype=BF), torch.empty(s, d, device=DEV, dtype=BF)
+        ws = torch.full((size // 4 + 1024,), 7.0, device=DEV)
+        rc = _lib.lib().sy_bwd_batched(buf.data_ptr(), qd.data_ptr(), gd.data_ptr(), dv.data_ptr(), dq.data_ptr(),
+                                       ws.data_ptr(), size, n, s, t, d, stride, _lib.dtype_code(BF), 1e-6,
+                                       _lib.stream_ptr(buf.device))
+        assert (ws[size // 4 :] == 7.0).all()
+        if size < need:
+            assert rc < 0
+            continue
+        assert rc == 0
+        assert rel_l2(dv.cpu(), rdv) <= 1.10 * dtype_floor(rdv, BF) and rel_l2(dq.cpu(), rdq) <= 1.10 * dtype_floor(rdq, BF)
+        got.append(dv)
+    assert not torch.equal(*got)  # two kernels, two orders of sums
