@@ -987,7 +987,7 @@ int sy_merge_stats_bwd(const void* o1, const float* m1, const float* l1, const v
 int sy_rms_norm(const void* x, const void* w, void* out, float* rinv, int64_t n_tok, int64_t d,
                 int dtype, float eps, void* stream) {
   if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
-  if (n_tok < 0 || n_tok > 0x3fffffff || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
+  if (n_tok < 0 || n_tok > ((int64_t)1 << 40) || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
   if (n_tok == 0) return SY_OK;
   if (!x || !w || !out) return SY_ERR_NULL;
   if (!al16(x) || !al16(w) || !al16(out)) return SY_ERR_SHAPE;
@@ -1004,7 +1004,7 @@ int sy_rms_norm_bwd(const void* x, const void* w, const void* grad_out, const fl
                     void* dw, void* workspace, int64_t workspace_bytes, int64_t n_tok, int64_t d,
                     int dtype, void* stream) {
   if (!valid_dtype(dtype)) return SY_ERR_DTYPE;
-  if (n_tok < 0 || n_tok > 0x3fffffff || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
+  if (n_tok < 0 || n_tok > ((int64_t)1 << 40) || d < 1 || !norm_fits(d, dtype)) return SY_ERR_SHAPE;
   if (!dw || (n_tok != 0 && (!x || !w || !grad_out || !rinv || !dx))) return SY_ERR_NULL;
   if (!al16(x) || !al16(w) || !al16(grad_out) || !al16(dx) || !al16(workspace)) return SY_ERR_SHAPE;
   const hipStream_t s = (hipStream_t)stream;

@@ -31,28 +31,28 @@ k_rms_norm(const typename T::storage* __restrict__ x, const typename T::storage*
            float eps, float inv_d) {
   using S = typename T::storage;
   const int lane = threadIdx.x & 63;
-  const int64_t tok = (int64_t)blockIdx.x * kWaves + wave_id();
-  if (tok >= n_tok) return;
   const uint32_t row_bytes = (uint32_t)d * sizeof(S);
-  const auto xr = make_rsrc(x + tok * d, row_bytes);
   const auto wr = make_rsrc(w, row_bytes);
-  i32x4_t v[VPL], g[VPL];
+  for (int64_t tok = (int64_t)blockIdx.x * kWaves + wave_id(); tok < n_tok; tok += (int64_t)gridDim.x * kWaves) {
+    const auto xr = make_rsrc(x + tok * d, row_bytes);
+    i32x4_t v[VPL], g[VPL];
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) v[j] = ld16_stream(xr, (lane + 64 * j) * 16u);
+    for (int j = 0; j < VPL; ++j) v[j] = ld16_stream(xr, (lane + 64 * j) * 16u);
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) g[j] = ld16(wr, (lane + 64 * j) * 16u);
-  float ss = 0.0f;
+    for (int j = 0; j < VPL; ++j) g[j] = ld16(wr, (lane + 64 * j) * 16u);
+    float ss = 0.0f;
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) ss = dot<T>(v[j], v[j], ss);
-  const float r = rsqrtf(fmaf(wave_sum(ss), inv_d, eps));
-  if (rinv != nullptr && lane == 0) rinv[tok] = r;
-  const auto orr = make_rsrc(out + tok * d, row_bytes);
+    for (int j = 0; j < VPL; ++j) ss = dot<T>(v[j], v[j], ss);
+    const float r = rsqrtf(fmaf(wave_sum(ss), inv_d, eps));
+    if (rinv != nullptr && lane == 0) rinv[tok] = r;
+    const auto orr = make_rsrc(out + tok * d, row_bytes);
 #pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    float f[T::ce];
+    for (int j = 0; j < VPL; ++j) {
+      float f[T::ce];
 #pragma unroll
-    for (int e = 0; e < T::ce; ++e) f[e] = elem<T>(v[j], e) * r * elem<T>(g[j], e);
-    st16(orr, (lane + 64 * j) * 16u, pack<T>(f));
+      for (int e = 0; e < T::ce; ++e) f[e] = elem<T>(v[j], e) * r * elem<T>(g[j], e);
+      st16(orr, (lane + 64 * j) * 16u, pack<T>(f));
+    }
   }
 }
 
@@ -244,8 +244,11 @@ hipError_t norm_t(const NormArgs& a, hipStream_t s) {
   using St = typename T::storage;
   const float inv_d = 1.0f / (float)a.d;
   if (a.go == nullptr) {
-    hipLaunchKernelGGL((k_rms_norm<T, VPL>), dim3((unsigned)((a.n_tok + kWaves - 1) / kWaves)), dim3(kBlock),
-                       0, s, (const St*)a.x, (const St*)a.w, (St*)a.out, a.rinv, a.n_tok, a.d, a.eps, inv_d);
+    // A workgroup for every four tokens, up to a grid that is a launch at any token count
+    // (2^32 threads are none).
+    const unsigned grid = (unsigned)std::min<int64_t>((a.n_tok + kWaves - 1) / kWaves, 1 << 20);
+    hipLaunchKernelGGL((k_rms_norm<T, VPL>), dim3(grid), dim3(kBlock), 0, s, (const St*)a.x, (const St*)a.w,
+                       (St*)a.out, a.rinv, a.n_tok, a.d, a.eps, inv_d);
   } else {
     hipLaunchKernelGGL((k_rms_norm_bwd<T, VPL>), dim3((unsigned)a.rows), dim3(kBlock), 0, s, (const St*)a.x,
                        (const St*)a.w, (const St*)a.go, a.rinv, (St*)a.out, a.partial, a.n_tok, a.d, inv_d);

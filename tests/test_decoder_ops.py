@@ -269,3 +269,22 @@ def test_the_sites_agree_bit_for_bit_in_every_mode(dtype):
             assert torch.equal(model(idx, collect_alphas=True), outs[sources, False])
     ref = outs["stack", True]
     assert all(torch.equal(x, ref) for x in outs.values())
+
+
+def test_a_norm_over_more_tokens_than_one_launch_has_waves():
+    """2^26 tokens of a wave each would be 2^32 threads, which is no launch."""
+    t = (1 << 26) + 5
+    print("rms_norm at 2^26 tokens", flush=True)
+    x = torch.zeros(t, 8, device=DEV, dtype=BF)
+    rows = torch.tensor([0, 1, (1 << 22) + 3, (1 << 26) - 1, t - 1], device=DEV)
+    x[rows] = _rand(5, 8, dtype=BF, seed=1)
+    w, g = _rand(8, dtype=BF, seed=2), _rand(5, 8, dtype=BF, seed=3)
+    go = torch.zeros_like(x)
+    go[rows] = g
+    small = [y.clone().requires_grad_() for y in (x[rows], w)]
+    big = [x.requires_grad_(), w.clone().requires_grad_()]
+    want = torch.autograd.grad(_lib.native().rms_norm(*small, 1e-6), small, g)
+    out = _lib.native().rms_norm(*big, 1e-6)
+    dx, dw = torch.autograd.grad(out, big, go)
+    assert torch.equal(out[rows], _lib.native().rms_norm(*small, 1e-6))
+    assert torch.equal(dx[rows], want[0]) and rel_l2(dw.cpu(), want[1].double().cpu()) <= 4e-3  # one rounding
