@@ -99,6 +99,21 @@ int bwd_plan(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, 
   return rc;
 }
 
+// The forward's plan for a launch. The unaligned kernels launch all tokens at once, on up
+// to eight waves each, and fewer than 2^32 threads are a launch: the element-wise kernel's
+// four waves reach twice as far.
+int fwd_plan(int64_t n_src, int64_t n_tok, int64_t d, int v_dtype, int w_dtype, int aligned, bool gain,
+             sy_plan* p, bool* unal) {
+  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, p, unal, 1, 0, gain);
+  if (rc != SY_OK) return rc;
+  if (*unal && n_tok > 0xffffffffLL / p->block_threads * p->tokens_per_block) {
+    *unal = false;
+    return make_plan(SY_OP_FWD, n_src, 0, d, v_dtype, w_dtype, 0, p);
+  }
+  if (!*unal) apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, p);
+  return SY_OK;
+}
+
 // Partial rows the backward's workspace provides: the largest persistent
 // grid of the plans an aligned call takes (every variant, with and without
 // forward stats) -- vector tiles, and the generic kernel where an aligned
@@ -361,10 +376,8 @@ int fwd_impl(const RowTable& v, bool v_ok, const void* w, void* out, float* stat
   const bool aligned = vec_rows(v_ok, d, v_dtype) && al16(w) && al16(out) && al16(gain);
   sy_plan p;
   bool unal = false;
-  const int rc = make_launch_plan(SY_OP_FWD, n_src, d, v_dtype, w_dtype, aligned, &p, &unal, 1, 0,
-                                  gain != nullptr);
+  const int rc = fwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, gain != nullptr, &p, &unal);
   if (rc != SY_OK) return rc;
-  if (!unal) apply_tile_rules(SY_OP_FWD, n_src, n_tok, d, &p);
   if (n_tok == 0) return SY_OK;
   FwdArgs a{v,      w,       out,     stats,   m_out, l_out, normalize, (int)n_src,
             n_tok,  (int)d,  v_dtype, w_dtype, eps};
@@ -544,13 +557,12 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
       out->family = SY_FAMILY_TWO_PASS;
     return rc;
   }
-  int rc = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
   bool unal = false;
-  if (rc == SY_OK && (op == SY_OP_FWD || op == SY_OP_BWD))
-    rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal, 1, 0, gain);
-  if (rc != SY_OK || unal) return rc;
-  if (op == SY_OP_FWD || op == SY_OP_BWD) apply_tile_rules(op, n_src, n_tok, d, out);
-  return SY_OK;
+  if (op == SY_OP_FWD) return fwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, gain, out, &unal);
+  if (op != SY_OP_BWD) return make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  const int rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal, 1, 0, gain);
+  if (rc == SY_OK && !unal) apply_tile_rules(op, n_src, n_tok, d, out);
+  return rc;
 }
 
 int sy_fwd(const void* v, const void* w, void* out, float* stats, int64_t n_src, int64_t n_tok,

@@ -440,3 +440,13 @@ def test_a_gain_keeps_the_widest_rows_tile(n, rows, dtype):
     # a query of another dtype has no tile there, with or without a gain
     for gain in (False, True):
         assert _lib.plan(_lib.OP_BWD, n, 16384, dtype, w_dtype=torch.float32, n_tok=2048, gain=gain)["family_name"] == "generic"
+
+
+def test_odd_rows_of_more_tokens_than_one_launch_takes():
+    """2^32 threads are no launch: eight waves a token reach 2^23 tokens, the element-wise
+    kernel's four 2^24."""
+    def family(d, n_tok, **kw):
+        return _lib.plan(_lib.OP_FWD, 1, d, torch.bfloat16, n_tok=n_tok, **kw)["family_name"]
+
+    assert family(4097, (1 << 23) - 1) == "resident" and family(4097, 1 << 23) == "generic"
+    assert family(4104, 1 << 23, aligned=False) == "generic" and family(2049, 1 << 23) == "resident"
