@@ -157,7 +157,7 @@ k_bb_coef(const RowTable v, const typename T::storage* __restrict__ q,
   constexpr bool TWO = SG > 2;
   constexpr int CE = T::ce;
   constexpr int kCols = 4 * CE;  // columns of a step
-    constexpr int kU = TWO ? 4 : 8;  // steps of a batch
+  constexpr int kU = TWO ? 4 : 8;  // steps of a batch
   constexpr int kTpb = kCoefWaves / W;  // tokens a workgroup takes at once
   static_assert(W == 1 || W == kCoefWaves, "a token is a wave's or a workgroup's");
   __shared__ __align__(16) float xl[TWO ? 2 : 1][W > 1 ? W : 1][64][4];
