@@ -15,8 +15,8 @@
 // v and g are read twice (43 slabs of [tokens, D] where one pass needs 26 at N=9,
 // S=8), against the register tile's single pass with 18 wave reductions and a barrier
 // a query and three VALU operations for every (query, source, element). N=9 S=8
-// T=4096 D=4096 bf16: 574 us in one pass, 295 in two -- coefficients 130 (570 MB, 4.4
-// TB/s: 64-byte row pieces), apply 160 (873 MB, 5.5 TB/s), reduction 5.
+// T=4096 D=4096 bf16: 574 us in one pass, 295 in two -- coefficients 130-145 (570 MB,
+// 3.9-4.4 TB/s: 64-byte row pieces), apply 160-170 (885 MB, 5.2-5.5 TB/s), reduction 5.
 //
 // Reference: the batched forward is src/switchyard/triton_op.py:378-501; it has no
 // backward (the single-query derivation is at :205-214).
@@ -482,9 +482,10 @@ k_bb_apply(const RowTable v, const typename T::storage* __restrict__ q,
 // (W = 1). First the logits, straight from memory on MFMA as in k_bb_coef (queries as
 // B), summed over the waves through LDS; every wave then forms the softmax and keeps
 // the token's weights [n][s] as A operands, one value a lane, and in a second walk over
-// the token's rows -- now in L2 -- out_s = sum_n P_sn v_n on v_mfma_f32_4x4x1 as in
-// k_bb_apply: whole chunks in and out, exact fp32 weights. Memory-bound: v is read
-// from HBM once (the register tile computes S dots and S sums a row on the VALU).
+// the token's rows out_s = sum_n P_sn v_n on v_mfma_f32_4x4x1 as in k_bb_apply: whole
+// chunks in and out, exact fp32 weights. Memory-bound: the second walk finds part of the
+// rows in L2 and the rest in the last-level cache (N=12 S=8 T=4096 D=1280: 1.6 times the
+// rows' bytes pass the L2); the register tile computes S dots and S sums a row on the VALU.
 // bf16 T=4096: N=9 S=8 D=1280 74 -> 62 us, D=2560 144 -> 108; N=12 S=8 D=1280 159 (a
 // launch a query) -> 64; N=9 S=8 T=1023 D=777 195 -> 17.5. Its two walks do not
 // overlap within a wave, which leaves it at 1.5-1.8x the bytes' time.

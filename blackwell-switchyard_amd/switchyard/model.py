@@ -333,6 +333,9 @@ class _Stream:
     def sources(self) -> list[Tensor]:
         return self.blocks if self.running is None else [*self.blocks, self.running]
 
+    def count(self) -> int:
+        return len(self.blocks) + (self.running is not None)
+
     def accumulate(self, y: Tensor, region=contextlib.nullcontext) -> None:
         """Add a sublayer output to the running sum; in arena mode also copy
         the new sum into its slot (the staging cost, inside ``region``). With
@@ -555,11 +558,11 @@ class Transformer(nn.Module):
             if i > 0 and i % cfg.block_size == 0:
                 stream.close_block()
             h = self._site(i, stream, collect_alphas, queries)
-            counts.append(len(stream.sources()))
+            counts.append(stream.count())
             y = fn(norm(h), self.rotary)
             stream.accumulate(y, lambda: self._region("attnres_stage"))
         stream.close_block()
-        counts.append(len(stream.sources()))
+        counts.append(stream.count())
         self.last_source_counts = counts
         return self._site(cfg.n_sublayers, stream, collect_alphas, queries)
 
@@ -579,13 +582,13 @@ class Transformer(nn.Module):
 
     def _site(self, i: int, stream: _Stream, collect_alphas: bool, queries: list[Tensor] | None) -> Tensor:
         cfg = self.cfg
-        q = self.attn_res[i].effective_query() if queries is None else queries[i]
-        sources = stream.sources()
-        n = len(sources)
         hip = cfg.residual == "switchyard"
-        if hip and stream.buf is not None and not torch.is_grad_enabled() and not collect_alphas:
+        q = self.attn_res[i].effective_query() if queries is None else queries[i]
+        n = stream.count()
+        if hip and stream.buf is not None and not collect_alphas and not torch.is_grad_enabled():
             with self._region("attnres_op"):
                 return block_attn_res_hip(stream.buf.slots[:n], q, cfg.norm_eps)
+        sources = stream.sources()
         if collect_alphas:
             self.last_alphas.append(_mean_alpha(sources, q, cfg.norm_eps))
         if cfg.sources == "stack":
