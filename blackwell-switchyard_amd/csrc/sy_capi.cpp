@@ -548,8 +548,10 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
                        int w_dtype, int aligned, sy_plan* out) {
   if (out == nullptr) return SY_ERR_NULL;
   if (n_tok < 0) return SY_ERR_SHAPE;
-  const bool gain = (w_dtype & SY_WITH_GAIN) != 0;
-  w_dtype &= ~SY_WITH_GAIN;
+  const bool gain = (op == SY_OP_FWD || op == SY_OP_BWD) && (w_dtype & SY_WITH_GAIN) != 0;
+  if (gain) w_dtype &= ~SY_WITH_GAIN;
+  const int known = make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  if (known != SY_OK) return known;
   if (op == SY_OP_BATCHED) return batched_plan(n_src, n_q, n_tok, d, v_dtype, aligned, out);
   if (op == SY_OP_BWD_BATCHED) {
     const int rc = bwd_batched_plan(n_src, n_q, n_tok, d, v_dtype, aligned, n_tok * d * esize(v_dtype), out);
@@ -559,7 +561,7 @@ int sy_plan_for_tokens(int op, int64_t n_src, int64_t n_q, int64_t n_tok, int64_
   }
   bool unal = false;
   if (op == SY_OP_FWD) return fwd_plan(n_src, n_tok, d, v_dtype, w_dtype, aligned, gain, out, &unal);
-  if (op != SY_OP_BWD) return make_plan(op, n_src, n_q, d, v_dtype, w_dtype, aligned, out);
+  if (op != SY_OP_BWD) return SY_OK;
   const int rc = make_launch_plan(op, n_src, d, v_dtype, w_dtype, aligned, out, &unal, 1, 0, gain);
   if (rc == SY_OK && !unal) apply_tile_rules(op, n_src, n_tok, d, out);
   return rc;

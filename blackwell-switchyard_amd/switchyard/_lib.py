@@ -204,7 +204,8 @@ def plan(op: int, n_src: int, d: int, dtype: torch.dtype, *, n_q: int = 0,
     """The execution plan the library picks for a shape (pure host arithmetic).
     With ``n_tok``, the tile a launch of that many tokens runs on the current
     device (``sy_plan_for_tokens``: the forward and backward also depend on
-    the token count, the batched ops have two families more); then ``gain`` asks for the launch of a query with a gain."""
+    the token count, the batched ops have two families more); then ``gain``
+    asks for the launch of a query with a gain."""
     p = Plan()
     if n_tok is None:
         rc = lib().sy_plan_for(op, n_src, n_q, d, dtype_code(dtype), dtype_code(w_dtype or dtype),

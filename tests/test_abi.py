@@ -450,3 +450,18 @@ def test_odd_rows_of_more_tokens_than_one_launch_takes():
 
     assert family(4097, (1 << 23) - 1) == "resident" and family(4097, 1 << 23) == "generic"
     assert family(4104, 1 << 23, aligned=False) == "generic" and family(2049, 1 << 23) == "resident"
+
+
+def test_the_launch_plan_refuses_what_the_plan_refuses():
+    p = _lib.Plan()
+
+    def rc(op, n, n_q, d, vt, wt):
+        a = _lib.lib().sy_plan_for(op, n, n_q, d, vt, wt, 1, ctypes.byref(p))
+        assert a == _lib.lib().sy_plan_for_tokens(op, n, n_q, 64, d, vt, wt, 1, ctypes.byref(p))
+        return a
+
+    for op in (_lib.OP_FWD, _lib.OP_BWD, _lib.OP_BATCHED, _lib.OP_SOL, _lib.OP_BWD_BATCHED):
+        assert rc(op, 9, 8, 512, 2, 2) == OK
+        assert rc(op, 9, 8, 512, 2, 7) < 0 and rc(op, 9, 8, 512, 7, 2) < 0 and rc(op, 0, 8, 512, 2, 2) < 0
+    assert rc(_lib.OP_BATCHED, 9, 0, 512, 2, 2) < 0 and rc(99, 9, 8, 512, 2, 2) < 0
+    assert _lib.lib().sy_plan_for_tokens(_lib.OP_BATCHED, 9, 8, 64, 512, 2, 2 | _lib.WITH_GAIN, 1, ctypes.byref(p)) < 0
