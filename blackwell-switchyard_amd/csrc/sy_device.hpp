@@ -384,32 +384,57 @@ struct Query<T, kWideQuery, VPL> {
   }
 };
 
-// The product of two bf16 factors has at most 16 significant bits: its rounding to bf16
-// and what that leaves are both exact, and two packed dots cost half the operations of
-// one on widened elements. The second part is in LDS, as the registers are full (each
-// thread reads only what it wrote; the opaque index keeps the compiler from holding it).
+// The product of two bf16 (fp16) factors has at most 16 (22) significant bits: its
+// rounding to that type and what that leaves are both exact, and two packed dots cost half
+// the operations of one on widened elements. fp16 has not the exponents for that, so a
+// lane scales its products by the power of two that brings the largest below 2^15, and
+// their remainders by 2^11: what then lies below fp16's range is under 2^-29 of the
+// largest. The second part is in LDS, as the registers are full (each thread reads only
+// what it wrote; the opaque index keeps the compiler from holding it).
 template <class T, int VPL, int THREADS>
 struct QuerySplit {
-  static_assert(T::code == BF16::code, "fp16's exponents do not reach its remainders");
+  static constexpr bool kF16 = T::code == F16::code;
   typedef i32x4_t Lds[VPL][THREADS];
   i32x4_t hi[VPL];
+  float scale;
   __device__ __forceinline__ void load(Lds& lo, const void* w, const void* gain, int wt, uint32_t d,
                                        uint32_t lane_off, uint32_t step) {
     float f[VPL][T::ce];
     ld_query_row(w, gain, wt, d, lane_off, step, f);
+    int shift = 0;
+    if constexpr (kF16) {
+      float top = 0.0f;
+#pragma unroll
+      for (int j = 0; j < VPL; ++j)
+#pragma unroll
+        for (int e = 0; e < T::ce; ++e) top = fmaxf(top, fabsf(f[j][e]));
+      shift = 15 - __builtin_amdgcn_frexp_expf(top);
+      scale = ldexpf(1.0f, -shift);
+    }
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
+      if constexpr (kF16) {
+#pragma unroll
+        for (int e = 0; e < T::ce; ++e) f[j][e] = ldexpf(f[j][e], shift);
+      }
       hi[j] = pack<T>(f[j]);
 #pragma unroll
-      for (int e = 0; e < T::ce; ++e) f[j][e] -= elem<T>(hi[j], e);
+      for (int e = 0; e < T::ce; ++e) f[j][e] = (f[j][e] - elem<T>(hi[j], e)) * (kF16 ? 2048.0f : 1.0f);
       lo[j][threadIdx.x] = pack<T>(f[j]);
     }
   }
+  // A row's chunks are added from zero; done() is then its dot.
   __device__ __forceinline__ float dot(const Lds& lo, const i32x4_t& x, int j, float acc) const {
     int t = threadIdx.x;
     asm volatile("" : "+v"(t));
-    return sy::dot<T>(x, lo[j][t], sy::dot<T>(x, hi[j], acc));
+    if constexpr (kF16) {
+      const float rest = sy::dot<T>(x, lo[j][t], 0.0f);
+      return sy::dot<T>(x, hi[j], fmaf(rest, 1.0f / 2048.0f, acc));
+    } else {
+      return sy::dot<T>(x, lo[j][t], sy::dot<T>(x, hi[j], acc));
+    }
   }
+  __device__ __forceinline__ float done(float acc) const { return kF16 ? acc * scale : acc; }
 };
 
 // A wide query in LDS, for 16-bit tiles whose registers are full: four elements a piece, a

@@ -307,7 +307,7 @@ hipError_t SY_FN(launch_fwd_wide_)(const sy_plan& p, const FwdArgs& a, hipStream
     constexpr int kB = FwdGeom<W_>::kBlock, kT = FwdGeom<W_>::kTpb;                          \
     if (res) {                                                                               \
       /* 9 rows on more than one wave: see k_fwd_res. */                                     \
-      if constexpr (T::code == BF16::code && W_ > 1 && V_ == 4 && N_ == 9) {                 \
+      if constexpr (T::ce == 8 && W_ > 1 && V_ == 4 && N_ == 9) {                 \
         if (a.gain != nullptr && a.w_dtype == a.v_dtype) {                                   \
           static const KernelRes ks =                                                        \
               resources_of(k_fwd_res<T, W_, V_, N_, false, false, kSplitQuery>, kB);         \

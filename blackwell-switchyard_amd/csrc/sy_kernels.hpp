@@ -526,11 +526,11 @@ k_batched(const RowTable v, const typename T::storage* __restrict__ q,
 // held to 256, two waves a SIMD like the packed query's (239). On one wave that fits; on
 // more, where the cross-wave sums take registers too, it spilled 8 VGPRs, and waiting for
 // a spilled value also waits for the rows prefetched before it. There the query is in LDS
-// (QueryLds), or for bf16 factors split in two packed parts (QuerySplit: the widened dots'
+// (QueryLds), or for two factors of the sources' dtype split in two packed parts (QuerySplit: the widened dots'
 // operations lie between a token's loads and the next one's). A no-grad module call with
 // 16-bit factors, us: with the product as a 16-bit tensor / spilled / now, bf16
 // N=9 T=8192 D=4096 115.7 / 124.1 / 117.2, T=4096 D=8192 117.4 / 129.0 / 119.7; fp16
-// 115.1 / 122.4 / 118.6 and 115.6 / 127.0 / 119.1.
+// 115.1 / 122.4 / 117.5 (fp32 values in LDS 118.6) and 115.6 / 127.0 / 118.8.
 template <class T, int W, int VPL, int NR, bool MERGE = false, bool FIN = false, int QRY = kPacked>
 __global__ void __launch_bounds__(FwdGeom<W>::kBlock, QRY != kPacked && VPL == 4 && NR == 9 ? 2 : 1)
 k_fwd_res(const RowTable v, const void* __restrict__ w,
@@ -571,7 +571,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
   using Lds = QueryLds<T, kLdsQ ? VPL : 1, kLdsQ ? FwdGeom<W>::kBlock : 1>;
   [[maybe_unused]] __shared__ std::conditional_t<kLdsQ, Lds, char> wl;
   constexpr bool kSplit = QRY == kSplitQuery;
-  using Split = QuerySplit<BF16, VPL, FwdGeom<W>::kBlock>;
+  using Split = QuerySplit<std::conditional_t<kSplit, T, BF16>, VPL, FwdGeom<W>::kBlock>;
   [[maybe_unused]] __shared__ std::conditional_t<kSplit, typename Split::Lds, char> lo;
   [[maybe_unused]] std::conditional_t<kSplit, Split, Query<T, kSplit ? kPacked : QRY, VPL>> wq;
   if constexpr (kLdsQ) wl.load(w, gain, wt, (uint32_t)d, lane_off, kStep);
@@ -580,6 +580,10 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
   auto qdot = [&](const i32x4_t& c, int j, float acc) {
     if constexpr (kSplit) return wq.dot(lo, c, j, acc);
     else return wq.dot(c, j, acc);
+  };
+  auto qdone = [&](float acc) {
+    if constexpr (kSplit) return wq.done(acc);
+    else return acc;
   };
   i32x4_t x[NR][VPL];
   float pstat = 0.0f;
@@ -723,7 +727,7 @@ k_fwd_res(const RowTable v, const void* __restrict__ w,
               reconvert<kWide>(x[n][j]);
             }
             tv[n] = ss;
-            tv[NR + n] = dt;
+            tv[NR + n] = qdone(dt);
           }
         }
       }

@@ -130,3 +130,23 @@ def test_gradients_of_the_widest_rows(shape, dtype):
     rdv, rdq = oracle_grads(v.double(), w.double() * gain.double(), go.double())
     for got, want in ((dv, rdv), (dw, rdq * gain.double()), (dg, rdq * w.double())):
         assert rel_l2(got, want) <= 1.10 * dtype_floor(want, dtype)
+
+
+@pytest.mark.parametrize("size", [1e-7, 1e-4, 1.0, 250.0])
+@pytest.mark.parametrize("dtype", [BF, HF])
+def test_split_products_of_any_size(size, dtype):
+    """A lane's products from below fp16's normal range to beyond its largest number, of
+    very different sizes within a lane: the logits keep fp32 accuracy."""
+    n, t, d = 6, 515, 2312
+    print(f"split products {size} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(7)
+    v = torch.randn(n, 1, t, d, generator=gen).to(dtype)
+    spread = torch.exp2(-torch.randint(0, 12, (d,), generator=gen).float())
+    w, gain = (torch.randn(d, generator=gen) * size).to(dtype), (torch.randn(d, generator=gen) * size * spread).to(dtype)
+    vd, wd, gd = v.to(DEV), w.to(DEV), gain.to(DEV)
+    out, stats = torch.empty(1, t, d, device=DEV, dtype=dtype), torch.empty(2, n, t, device=DEV)
+    _lib.check(_lib.lib().sy_fwd_gain(vd.data_ptr(), wd.data_ptr(), gd.data_ptr(), out.data_ptr(), stats.data_ptr(),
+                                      n, t, d, t * d, _lib.dtype_code(dtype), _lib.dtype_code(dtype), 1e-6,
+                                      _lib.stream_ptr(vd.device)), "sy_fwd_gain")
+    r = torch.rsqrt(v.double().square().mean(-1) + 1e-6)[:, 0]
+    assert rel_l2(stats[0], (v.double() @ (w.double() * gain.double()))[:, 0] * r) <= 2e-6 and out.isfinite().all()
