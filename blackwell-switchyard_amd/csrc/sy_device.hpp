@@ -343,7 +343,8 @@ __device__ __forceinline__ float dot_wide(const i32x4_t& x, const float* f, floa
 }
 
 // A lane's query chunks: packed in the sources' dtype, or as fp32 values when the query
-// has another dtype or a gain (kWideQuery), or for bf16 factors as two packed parts
+// has another dtype or a gain (kWideQuery), or for two 16-bit factors of the sources' dtype
+// as the two packed parts of their product
 // (kSplitQuery). fp32 sources hold any query as fp32 chunks.
 enum QueryForm { kPacked = 0, kWideQuery = 1, kSplitQuery = 2 };
 template <class T, int FORM, int VPL>
